@@ -365,10 +365,10 @@ def kernel_class_of(short: str) -> str | None:
     """Map a rocprof kernel name to the profiling class bench.py reports
     (igemm_kernel<MB, NB, WM, WN, ...> -> conv3d_igemm_m{16*MB*WM}n{16*NB*WN}, the
     split-fp16 kernels igemm_x3s_kernel / igemm_x3_kernel -> conv3d_x3s_* / conv3d_x3_*, and
-    both Winograd kernels, one box a workgroup and persistent, -> conv3d_wino)."""
+    the Winograd kernels -> conv3d_wino)."""
     import re
 
-    if short.startswith(("wino_x3_kernel", "wino_x3p_kernel")):
+    if short.startswith(("wino_yx_kernel", "wino_x3_kernel", "wino_x3p_kernel")):
         return "conv3d_wino"
     m = re.match(r"igemm(_x3s|_x3)?_kernel<(\d+), (\d+), (\d+), (\d+)([^>]*)>", short)
     if not m:
@@ -639,12 +639,19 @@ def measured_traffic(kernel_class: str) -> float | None:
     return None
 
 
-def kernel_table(classes: dict, steps: int, traffic: bool = True) -> tuple[dict, dict]:
+# MFMA products the Winograd kernel issues per product of the direct convolution: F(2x2) in
+# (y, x), 16 positions per 4 outputs and 9 taps, the z taps direct
+WINO_ISSUED = 16 / 36
+
+
+def kernel_table(classes: dict, steps: int, traffic: bool = True,
+                 wino_issued: float = 64 / 216) -> tuple[dict, dict]:
     """Per-kernel-class rates of a KernelProfile (launches and ms per step) and the roofline
     object of the dominant class (largest share of the timed region): algorithmic FLOPs or
     bytes over its launch time, against the published peak of the unit that bounds it.
     `traffic`: take the HBM bytes per launch from the liver-case counter summary (only the
-    liver workload's launches are the ones it measured)."""
+    liver workload's launches are the ones it measured).  `wino_issued`: issued products per
+    direct product of the Winograd class (the default is F(2x2x2)'s)."""
     kernels = {}
     for name, c in sorted(classes.items(), key=lambda kv: -kv[1]["ms"]):
         entry = {"launches": c["launches"] // steps, "ms": round(c["ms"] / steps, 3)}
@@ -659,10 +666,9 @@ def kernel_table(classes: dict, steps: int, traffic: bool = True) -> tuple[dict,
                 entry["frac_fp16_mfma_issued"] = round(
                     entry["tflops"] * SPLIT_PRODUCTS * 28 / 27 / PEAK_FP16_MFMA_TFLOPS, 4)
             elif name == "conv3d_wino":
-                # issued fp16 MFMA work: 3 products per term, 64 transform positions per 8
-                # outputs in place of 8 x 27 taps
+                # issued fp16 MFMA work: 3 products per term of the transformed convolution
                 entry["frac_fp16_mfma_issued"] = round(
-                    entry["tflops"] * SPLIT_PRODUCTS * 64 / 216 / PEAK_FP16_MFMA_TFLOPS, 4)
+                    entry["tflops"] * SPLIT_PRODUCTS * wino_issued / PEAK_FP16_MFMA_TFLOPS, 4)
             elif name.startswith("tconv3d_x3"):
                 # issued MFMA work of the pointwise GEMM: 3 fp16 products per term (1 bf16
                 # product in the bf16 variant; bf16 and fp16 share the dense peak); the
@@ -859,7 +865,8 @@ def ensemble_workload(args) -> int:
         torch.cuda.synchronize()
         step_s = (time.perf_counter() - t0) / args.steps
     device_peak_gb = peak.gb()
-    kernels, roofline = kernel_table(prof.classes, steps=args.steps, traffic=False)
+    kernels, roofline = kernel_table(prof.classes, steps=args.steps, traffic=False,
+                                     wino_issued=WINO_ISSUED)
     steps = [len(s) for s in sw.compute_steps([max(a, b) for a, b in zip(volume.shape[1:], patch)],
                                               patch, step_fraction=0.5)]
     tiles = int(np.prod(steps))
@@ -1078,7 +1085,7 @@ def main() -> int:
 
     device_peak_gb = peak.gb()
     classes = prof.classes
-    kernels, roofline = kernel_table(classes, steps=args.steps)
+    kernels, roofline = kernel_table(classes, steps=args.steps, wino_issued=WINO_ISSUED)
     # 3x3x3 convolution rate against the float32-class MFMA peak of the arithmetic used
     conv_frac = conv_mfma_frac(classes, args.precision)
 

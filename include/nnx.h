@@ -52,7 +52,7 @@ const char* nnx_version(void);
  * too, with a per-tile power-of-two scale of the raw input (nnx_conv3d_direct_small_cin_split);
  * other first convolutions keep float32 products.  Meets the float32 logits tolerance;
  * hidden activations must stay below 65504 in magnitude at layers on the direct split kernels
- * and below 8188 at the Winograd layers (the input transform sums up to 8 of them before the
+ * and below 16376 at the Winograd layers (the input transform sums up to 4 of them before the
  * split).  They are InstanceNorm outputs, so with ordinary affine parameters they do; a
  * checkpoint whose activations exceed the range makes the forward fail with a ContractError
  * that names the layer (nnx_set_layer_checks), never a silent result. */
@@ -191,7 +191,7 @@ void nnx_sw_release(void);
  * forward has produced non-finite logits; they serialise the forward.
  * Replaces nothing in the reference, whose float32 path has no operand range: it names the
  * layer where the split-fp16 precisions meet theirs (its inputs beyond 65504, or beyond
- * 8188 at a Winograd layer, whose input transform adds up to 8 of them). */
+ * 16376 at a Winograd layer, whose input transform adds up to 4 of them). */
 int nnx_set_layer_checks(int enable);
 
 /* Count non-finite float32 values; *d_count (device uint32) is overwritten.
@@ -250,17 +250,17 @@ int nnx_conv3d_split(const float* d_x1, int c1, const float* d_x2, int c2, const
                      float scale, const float* d_bias, float* d_y, int batch, const int* in_size,
                      int cout, const int* ksize, const int* stride, void* stream);
 
-/* The same convolution in Winograd form F(2x2x2, 3x3x3) for stride-1 3x3x3 layers with
- * C_out % 32 == 0 and c1, c2 multiples of 16: per 2x2x2 output tile the 4x4x4 input patch
- * and each 3x3x3 filter are transformed (additions, and halves for the filter: exact in
- * float32 / float64), the 64 transform positions are multiplied as split-fp16 products
- * (hi*hi + hi*lo + lo*hi, float32 accumulation) on fp16 MFMA, and the output transform
- * returns the tile; 64 products per 8 outputs instead of 216.  Filters are transformed in
- * float64, multiplied by `scale` (nnx_winograd_weight_scale(max |w|)) and split when
- * packed; outputs are multiplied by 1/scale (exact), + bias.  Replaces the same reference
- * calls as nnx_conv3d_igemm (mx.conv3d via _unbiased_convolution,
- * src/nnunet_mlx/model/network.py:240-269, and the split concat convolution,
- * src/nnunet_mlx/model/network.py:305-322). */
+/* The same convolution in Winograd form F(2x2, 3x3) over (y, x) for stride-1 3x3x3 layers
+ * with C_out % 32 == 0 and c1, c2 multiples of 16: per z plane and 2x2 output tile the 4x4
+ * input patch and each 3x3 filter slice are transformed (additions, and halves for the filter:
+ * exact in float32 / float64), the 16 transform positions are multiplied as split-fp16
+ * products (hi*hi + hi*lo + lo*hi, float32 accumulation) on fp16 MFMA and summed over the
+ * three z taps, and the output transform returns the tile; 48 products per 4 outputs instead
+ * of 108.  Filters are transformed in float64, multiplied by `scale`
+ * (nnx_winograd_weight_scale(max |w|)) and split when packed; outputs are multiplied by
+ * 1/scale (exact), + bias.  Replaces the same reference calls as nnx_conv3d_igemm (mx.conv3d
+ * via _unbiased_convolution, src/nnunet_mlx/model/network.py:240-269, and the split concat
+ * convolution, src/nnunet_mlx/model/network.py:305-322). */
 float nnx_winograd_weight_scale(float max_abs); /* 0 for a negative or non-finite argument */
 size_t nnx_conv3d_winograd_packed_bytes(int cout, int c1, int c2);
 int nnx_conv3d_winograd_pack_weight(const float* d_weight /* (Cout,3,3,3,c1+c2) */, int cout,

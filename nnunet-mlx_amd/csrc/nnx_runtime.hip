@@ -530,7 +530,7 @@ struct Runner {
     // Implicit GEMM: the epilogue writes per-tile statistics, so the norm never re-reads the
     // tensor for them.
     const ConvGeom g = make_conv_geom(n, in.d, c.k, c.s);
-    const int tiles = c.wino    ? conv_wino_stats_tiles(g)
+    const int tiles = c.wino    ? conv_wino_stats_tiles(g, c.cout)
                       : c.split ? conv_x3_stats_tiles(g, c.cout)
                                 : conv_stats_tiles(g, c.cout, c.cin1, c.cin2);
     if (plan->planning) {

@@ -1,39 +1,58 @@
-// Winograd F(2x2x2, 3x3x3) convolution for the stride-1, padding-1 3x3x3 layers, with
-// split-fp16 products (hi*hi + hi*lo + lo*hi, float32 accumulation) on
-// v_mfma_f32_32x32x16_f16.
+// Convolution of the stride-1, padding-1 3x3x3 layers: Winograd F(2x2, 3x3) in the (y, x)
+// plane, the three z taps summed directly, with split-fp16 products (hi*hi + hi*lo + lo*hi,
+// float32 accumulation) on v_mfma_f32_32x32x16_f16.
 //
-// A 2x2x2 output tile is Y = A^T [ U (.) V ] A along each axis, with V = B^T d B the
-// transform of the tile's 4x4x4 input patch and U = G w G^T the transform of the 3x3x3
-// filter (F(2,3): B^T = [1 0 -1 0; 0 1 1 0; 0 -1 1 0; 0 1 0 -1], G = [1 0 0; .5 .5 .5;
-// .5 -.5 .5; 0 0 1], A^T = [1 1 1 0; 0 1 -1 -1]).  Summed over input channels, each of the
-// 64 transform positions xi = (xz, xy, xx) is an independent GEMM M[xi] = V[xi] U[xi]
-// (tiles x C_in times C_in x C_out): 64 products per 8 outputs instead of 216, so the
-// three split products cost fewer MFMA operations than one product of the direct
-// convolution.  The transforms are exact additions/subtractions of float32 values (and
-// the 1/2 of G, exact), so the arithmetic stays float32-class; U is formed in float64 and
-// rounded once, V in float32, each then split into fp16 halves.
+// For each z plane a 2x2 output tile is Y = A^T [ sum_kz U[kz] (.) V[z + kz - 1] ] A, with
+// V = B^T d B the transform of the tile's 4x4 input patch and U[kz] = G w[kz] G^T the
+// transform of the filter's kz slice (F(2,3): B^T = [1 0 -1 0; 0 1 1 0; 0 -1 1 0; 0 1 0 -1],
+// G = [1 0 0; .5 .5 .5; .5 -.5 .5; 0 0 1], A^T = [1 1 1 0; 0 1 -1 -1]).  Summed over input
+// channels and z taps, each of the 16 transform positions xi = (xy, xx) is an independent
+// GEMM.  Against F(2x2x2) in all three axes this issues 12 products an output instead of 8,
+// but transforms and splits 4 values an output instead of 8, keeps 4 accumulators an output
+// instead of 8 (so the register file holds a box of twice the voxels) and reads each
+// transformed plane for three output planes; the three-axis form was bound by the VALU work
+// of the transform and split and by the fixed cost of its small boxes, with the matrix cores
+// 15 % busy.  The transforms are exact additions of float32 values (and the 1/2 of G, exact),
+// so the arithmetic stays float32-class; U is formed in float64 and rounded once, V in
+// float32, each then split into fp16 halves.  V adds up to 4 inputs.
 //
-// Workgroup: 8 waves (two a SIMD), an output box of 4 x 8 x 8 voxels (2 x 4 x 4 tiles, the 32
-// MFMA rows) of one batch item, and 32 output channels (the 32 MFMA columns).  Wave
-// w = 2 xz + p owns the 8 transform positions (xz, xy = 2p or 2p + 1, xx = 0..3): its
-// accumulators are 8 blocks of 32 x 32 floats (128 registers a lane), which leaves room for
-// a second wave on the SIMD to issue while one waits.  Per chunk of 16 input channels:
-//   1. the raw 6 x 10 x 10 input halo was fetched by global_load_lds_dwordx4 into one of two
-//      LDS buffers during the previous chunk;
-//   2. 400 threads apply the pending InstanceNorm (+ LeakyReLU) of the input to in-volume
-//      voxels (inputs without one, such as the transposed convolution's output in a decoder
-//      convolution, skip it) and write the z-transform (4 xz x 2 tile rows of z) as 8 padded planes, laid
-//      out so that the 32 tiles of a half-wave read 32 different 16-byte bank groups; then
-//      the next chunk's halo DMA is issued;
-//   3. per y-row of its positions, each wave reads two z-transformed rows of its tile patch,
-//      forms V (y- then x-transform), splits it into fp16 halves in registers and issues
-//      three MFMAs per position against the packed U of this chunk, read from L2 four
-//      positions ahead.
-// Epilogue: each wave applies the x- and y-output transforms to its accumulators, the eight
-// partials are combined through LDS (z-output transform), scaled back, + bias, written to
-// an LDS tile for the InstanceNorm partials of the box and stored as 16-byte channel runs.
+// Workgroup: 8 waves (two a SIMD), an output box of ZB z planes x 32 tiles (4 x 8 tiles =
+// 8 x 16 voxels, or 8 x 4 tiles where that wastes less) and 32 output channels.  Wave
+// w = 2 xy + h owns the positions (xy, xx = 0, 1) for h = 0 and (xy, xx = 3, 2) for h = 1: its
+// accumulators are 2 x ZB blocks of 32 x 32 floats (128 registers a lane at ZB = 4), which
+// leaves room for a second wave on the SIMD to issue while one waits.  Per chunk of 16 input
+// channels:
+//   1. the raw halo, (ZB + 2) planes, was fetched by global_load_lds_dwordx4 into one of two
+//      LDS buffers during the previous chunk, its slots laid out so that the 32 tiles of a
+//      half-wave read 32 different 16-byte bank groups;
+//   2. each thread applies the input's pending InstanceNorm (+ LeakyReLU) in place to the
+//      lines that it fetched itself (so it waits for its own loads only); one barrier;
+//   3. the next chunk's halo DMA is issued, into the other buffer;
+//   4. per input plane each wave reads the two rows and three columns of its positions'
+//      patches, forms V, splits it in registers and issues the products with the packed U of
+//      every z tap that reaches an output plane of the box (up to 18 MFMAs).  U (2 positions x
+//      3 taps, 48 registers) is reloaded from L2 tap by tap as the chunk's last product with it
+//      is issued, so its latency is covered by the planes that follow.
+// Epilogue, a z plane at a time: each wave applies its share of the x-output transform and
+// writes its two partials to LDS, and a thread sums the eight waves' partials of one tile
+// column for four output channels (y-output transform), scales back, adds the bias and stores
+// 16 bytes; the InstanceNorm partials of the box are reduced from the same registers.
+//
+// The kernel is persistent: one workgroup a CU loops over boxes.  The eight XCDs take contiguous
+// ranges of the (column block, box) pairs, column block slowest, so an XCD's L2 holds one
+// column block's packed weights and neighbouring boxes' halos.  The last chunk of a box
+// issues the next box's first halo DMA and U loads; the epilogue exchanges through the raw
+// buffer that this DMA does not target.
+//
+// Bound by power and issue together: a 128 -> 128 layer on 32^3 x 8 keeps the matrix cores 38 %
+// busy at 1.9 GHz (2.4 GHz with the products left out, 2.0 GHz with the products alone), and
+// leaving out any one part (products 38 %, halo DMA 21 %, transform and split 18 %, epilogue
+// 11 %, patch reads 9 %, U loads 7 %) takes its share off the time.  Measured against the
+// three-axis form it replaces, ms: 32 + 32 -> 32 on 128^3 x 8 4.57 -> 3.94 (472 TFLOP/s of the
+// direct convolution's work), 128 -> 128 on 32^3 x 8 0.489 -> 0.438 (529), 64 -> 64 on
+// 37 x 61 x 43 x 4 0.256 -> 0.216 (398); error against float64 2.6e-7 to 3.6e-7 relative
+// (the three-axis form 2.5e-7 to 3.2e-7, the direct split kernel 3.4e-7).
 #include <cmath>
-#include <cstdlib>
 #include <string>
 #include <type_traits>
 
@@ -48,23 +67,34 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 
-constexpr int kWThreads = 512;                    // 8 waves, two a SIMD
-constexpr int kSteps = 8;                         // transform positions (steps) per wave
-constexpr int kRing = 4;                          // B operands of four steps in flight
-constexpr int kWChunk = 16;                       // input channels per chunk (one MFMA K)
-constexpr int kHaloVox = 6 * 10 * 10;             // input halo of a 4 x 8 x 8 output box
-constexpr int kRawLines = kHaloVox * 4;           // 16-byte lines (4 channels each)
-constexpr int kRawRounds = (kRawLines + kWThreads - 1) / kWThreads;
-constexpr int kRawSlots = kRawRounds * kWThreads;  // 16-byte slots per raw buffer
-constexpr int kZRow = 41;                          // slots per z-plane row: 10 voxels x 4 + 1
-constexpr int kZPlane = 411;                       // slots per plane: 10 rows + 1 slot
-constexpr int kZSlots = 8 * kZPlane;
-constexpr int kMaxChannels = 1024;                 // c1 + c2 (pending-norm parameters in LDS)
-constexpr int kTileStride = 36;                    // floats per voxel row of the output tile
-// epilogue: 8 waves x 32 tiles x 32 columns of partials over the raw and z arrays, then the
-// output tile + reduction in the raw array
-static_assert(8 * 32 * 32 <= 2 * kRawSlots + kZSlots, "epilogue partials fit the main LDS");
-static_assert(256 * kTileStride / 4 + kWThreads / 4 <= 2 * kRawSlots, "output tile fits");
+constexpr int kWThreads = 512;    // 8 waves, two a SIMD
+constexpr int kWChunk = 16;       // input channels per chunk (one MFMA K)
+constexpr int kMaxChannels = 1024;  // c1 + c2 (pending-norm parameters in LDS)
+constexpr int kPlane = 768;       // 16-byte slots of a raw halo plane: 1.5 rounds of the workgroup
+constexpr int kPositions = 16;    // transform positions (xy, xx)
+constexpr int kTapWords = 128;    // packed words of one (position, z tap): hi, lo x 64 lanes
+constexpr int kPartSlots = 8 * 2 * 32 * 8;  // epilogue partials: wave, ox, tile, 4 columns
+constexpr int kRedSlots = 2 * 8 * 8;        // InstanceNorm partials: pass, wave, 4 columns
+
+// Box geometry.  A raw halo plane is stored as [y / 2][y % 2][x / 2][x % 2 ...] (tile rows and
+// columns are every second row and column) with q = channel quad fastest: slot = yi * py +
+// jump * (yi / 4) + yp * pyp + xp * pxp + xi * 4 + q.  For a fixed (row, column, quad) of the
+// patch the 32 tiles then fall on 32 different slots modulo 32 (ds_read_b128 serves 32 lanes
+// a pass from 32 16-byte groups).
+template <int ZB, bool TALL>
+struct WinoBoxGeom {
+  static constexpr int ty = TALL ? 8 : 4, tx = TALL ? 4 : 8;  // tiles
+  static constexpr int by = 2 * ty, bx = 2 * tx;              // output voxels
+  static constexpr int hz = ZB + 2, hy = by + 2, hx = bx + 2;  // halo
+  static constexpr int pxp = (tx + 1) * 4, pyp = 2 * pxp, py = 2 * pyp + 1;
+  static constexpr int jump = TALL ? 12 : 0;
+  static constexpr int slots = hz * kPlane;
+  // the epilogue's partials and reductions use one raw buffer
+  static constexpr int buf = slots > kPartSlots + kRedSlots ? slots : kPartSlots + kRedSlots;
+  static_assert(py * ty + jump * (ty / 4) + 2 * pyp <= kPlane, "a halo plane fits its slots");
+  static_assert(hz % 2 == 0, "plane pairs are three rounds of the workgroup");
+  static_assert(2 * buf * 16 + 3 * kMaxChannels * 4 + 128 <= 160 * 1024, "LDS");
+};
 
 struct WinoArgs {
   const float* x0;
@@ -74,11 +104,10 @@ struct WinoArgs {
   const float* bias;
   float* y;
   int D, H, W;
-  int cout, ntn;
+  int cout;
   int nbz, nby, nbx;
-  int nwg;
   int nbox;   // batch * nbz * nby * nbx (boxes of one column block)
-  int nvirt;  // nbox * ntn: (column block, box) pairs, column block slowest
+  int nvirt;  // nbox * cout / 32: (column block, box) pairs, column block slowest
   float out_scale;
   float4* stats;
   const float4* nrm0;
@@ -113,468 +142,52 @@ __device__ __forceinline__ void split8(const float (&v)[8], h8& hi, h8& lo) {
   }
 }
 
-// Two z-plane rows of a tile patch (4 columns x 2 channel halves each, 16 B per read) at LDS
-// byte offsets a and b, with the wait for them.  Written as one asm block so that the
-// compiler's wait-count pass does not see LDS reads here: it would otherwise order them
-// behind the halo DMA issued just before into another buffer (it cannot tell the two apart)
-// and wait for that DMA first.
-__device__ __forceinline__ void zrow_pair(unsigned a, unsigned b, f4 (&va)[8], f4 (&vb)[8]) {
+// Six patch points (two rows x columns P, Q, R; 8 channels each, two 16-byte reads) of halo
+// plane Z at LDS byte addresses ad[row * 3 + column], with the wait for them.  Written as
+// one asm block so that the compiler's wait-count pass does not see LDS reads here: it
+// would otherwise order them behind the halo DMA in flight to the other buffer (it cannot
+// tell the two apart) and wait for that DMA first.
+template <int Z>
+__device__ __forceinline__ void read_patch(const unsigned (&ad)[6], f4 (&v)[12]) {
   asm volatile(
-      "ds_read_b128 %0, %16\n\tds_read_b128 %1, %16 offset:16\n\t"
-      "ds_read_b128 %2, %16 offset:64\n\tds_read_b128 %3, %16 offset:80\n\t"
-      "ds_read_b128 %4, %16 offset:128\n\tds_read_b128 %5, %16 offset:144\n\t"
-      "ds_read_b128 %6, %16 offset:192\n\tds_read_b128 %7, %16 offset:208\n\t"
-      "ds_read_b128 %8, %17\n\tds_read_b128 %9, %17 offset:16\n\t"
-      "ds_read_b128 %10, %17 offset:64\n\tds_read_b128 %11, %17 offset:80\n\t"
-      "ds_read_b128 %12, %17 offset:128\n\tds_read_b128 %13, %17 offset:144\n\t"
-      "ds_read_b128 %14, %17 offset:192\n\tds_read_b128 %15, %17 offset:208\n\t"
+      "ds_read_b128 %0, %12 offset:%18\n\tds_read_b128 %1, %12 offset:%19\n\t"
+      "ds_read_b128 %6, %15 offset:%18\n\tds_read_b128 %7, %15 offset:%19\n\t"
+      "ds_read_b128 %2, %13 offset:%18\n\tds_read_b128 %3, %13 offset:%19\n\t"
+      "ds_read_b128 %8, %16 offset:%18\n\tds_read_b128 %9, %16 offset:%19\n\t"
+      "ds_read_b128 %4, %14 offset:%18\n\tds_read_b128 %5, %14 offset:%19\n\t"
+      "ds_read_b128 %10, %17 offset:%18\n\tds_read_b128 %11, %17 offset:%19\n\t"
       "s_waitcnt lgkmcnt(0)"
-      : "=&v"(va[0]), "=&v"(va[1]), "=&v"(va[2]), "=&v"(va[3]), "=&v"(va[4]), "=&v"(va[5]),
-        "=&v"(va[6]), "=&v"(va[7]), "=&v"(vb[0]), "=&v"(vb[1]), "=&v"(vb[2]), "=&v"(vb[3]),
-        "=&v"(vb[4]), "=&v"(vb[5]), "=&v"(vb[6]), "=&v"(vb[7])
-      : "v"(a), "v"(b)
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]),
+        "=&v"(v[6]), "=&v"(v[7]), "=&v"(v[8]), "=&v"(v[9]), "=&v"(v[10]), "=&v"(v[11])
+      : "v"(ad[0]), "v"(ad[1]), "v"(ad[2]), "v"(ad[3]), "v"(ad[4]), "v"(ad[5]),
+        "n"(Z * kPlane * 16), "n"(Z * kPlane * 16 + 16)
       : "memory");
 }
 
-// For lanes 0-31: x + (lane + 32's x), by v_permlane32_swap (lanes 32-63 of the first
-// operand trade places with lanes 0-31 of the second) instead of an LDS permute.  Lanes
-// 32-63 get x + x (unused).
-__device__ __forceinline__ float add_upper_half(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
-                                                  false);
-  return x + __uint_as_float(r[1]);
+// x summed over the eight lanes of a wave that share lane % 8, in every lane: a rotation by
+// 8 within rows of 16, then v_permlane16_swap and v_permlane32_swap (each leaves a pair's two
+// values in every lane of the pair).
+__device__ __forceinline__ float sum_stride8(float x) {
+  x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x128, 0xf, 0xf, false));
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// The InstanceNorm apply pass's operations: r = fma(x - mean, scale, beta), then
-// max(s * r, r) with s = the LeakyReLU slope under the activation and s = 1 (the identity,
-// exactly) without it.
-__device__ __forceinline__ f4 wino_norm(f4 v, const float4 (&p)[4], float s) {
+__device__ __forceinline__ f4 sum_stride8(f4 v) {
   f4 r;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const float t = fmaf(v[q] - p[q].x, p[q].y, p[q].z);
-    r[q] = fmaxf(s * t, t);
-  }
+  for (int e = 0; e < 4; ++e) r[e] = sum_stride8(v[e]);
   return r;
 }
 
+// Barrier that waits for this wave's LDS accesses only (not __syncthreads(), whose release
+// fence would also wait for the halo DMA and the stores in flight).
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// The end of a box's epilogue, shared by both kernels.  yo[k][oz] holds, for column
-// c = tid % 32 and tile (tid / 32) + 16 k of the box, the four (oy, ox) outputs of z output
-// oz.  The values go to the output tile in LDS (row per box voxel, stride kTileStride) and
-// leave as 16-byte channel runs; the box's InstanceNorm partials per column (mean over the
-// valid voxels, then the centred sum of squares) are reduced from the registers: a thread's
-// 16 voxels, the two lanes of a wave holding the column, then the eight waves through the
-// two 256-float arrays after the tile.  Barriers wait for LDS only.  kFull: the box lies
-// wholly inside the volume (no per-voxel checks).
-template <bool kFull>
-__device__ __forceinline__ void wino_epilogue_tail_t(const WinoArgs& a, const f4 (&yo)[2][2],
-                                                     float* otile, int tid, int lane, int wave,
-                                                     int b, int nt, int bzi, int byi, int bxi) {
-  const int oz0 = bzi * 4, oy0 = byi * 8, ox0 = bxi * 8;
-  const int c = tid & 31;
-  auto voxel = [&](int k, int oz, int e) {
-    const int tile = (tid >> 5) + 16 * k;
-    const int tz = tile >> 4, ty = (tile >> 2) & 3, tx = tile & 3;
-    return ((2 * tz + oz) * 8 + 2 * ty + (e >> 1)) * 8 + 2 * tx + (e & 1);
-  };
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-#pragma unroll
-    for (int oz = 0; oz < 2; ++oz)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) otile[voxel(k, oz, e) * kTileStride + c] = yo[k][oz][e];
-  auto valid = [&](int v) {
-    return oz0 + (v >> 6) < a.D && oy0 + ((v >> 3) & 7) < a.H && ox0 + (v & 7) < a.W;
-  };
-  float* red = otile + 256 * kTileStride;  // [wave][column] sums, then centred squares
-  const int nz = min(4, a.D - oz0), ny = min(8, a.H - oy0), nx = min(8, a.W - ox0);
-  const float cnt = (float)(nz * ny * nx);
-  if (a.stats) {
-    float sm = 0.f;
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-#pragma unroll
-      for (int oz = 0; oz < 2; ++oz)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (kFull || valid(voxel(k, oz, e))) sm += yo[k][oz][e];
-    sm = add_upper_half(sm);
-    if (lane < 32) red[wave * 32 + c] = sm;
-  }
-  lds_barrier();  // the tile and the sums
-  if (a.stats) {
-    // the eight waves' sums read together, then added in wave order
-    float rv[kWThreads / 64];
-#pragma unroll
-    for (int w = 0; w < kWThreads / 64; ++w) rv[w] = red[w * 32 + c];
-    float tot = 0.f;
-#pragma unroll
-    for (int w = 0; w < kWThreads / 64; ++w) tot += rv[w];
-    const float mean = tot / cnt;
-    float m2 = 0.f;
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-#pragma unroll
-      for (int oz = 0; oz < 2; ++oz)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (kFull || valid(voxel(k, oz, e))) {
-            const float d = yo[k][oz][e] - mean;
-            m2 = fmaf(d, d, m2);
-          }
-    m2 = add_upper_half(m2);
-    if (lane < 32) red[256 + wave * 32 + c] = m2;
-    lds_barrier();
-    if (tid < 32) {
-#pragma unroll
-      for (int w = 0; w < kWThreads / 64; ++w) rv[w] = red[256 + w * 32 + c];
-      float tm = 0.f;
-#pragma unroll
-      for (int w = 0; w < kWThreads / 64; ++w) tm += rv[w];
-      const int tiles = a.nbz * a.nby * a.nbx;
-      const int tile_s = (bzi * a.nby + byi) * a.nbx + bxi;
-      a.stats[((int64_t)b * tiles + tile_s) * a.cout + nt * 32 + c] = make_float4(mean, tm, cnt, 0.f);
-    }
-  }
-  // stores: 256 voxels x 8 runs of 4 channels; thread tid stores run tid % 8 of voxel
-  // (z, y, x) = (k, (tid / 64) % 8, (tid / 8) % 8) of the box in round k, so only z moves
-  // between its rounds (one 64-bit address, then a plane stride)
-  const int qd = tid & 7, vyx = (tid >> 3) & 63;
-  const int yy = oy0 + (vyx >> 3), xx = ox0 + (vyx & 7);
-  const int64_t base =
-      (((int64_t)b * a.D + oz0) * a.H * a.W + (int64_t)yy * a.W + xx) * a.cout + nt * 32 + 4 * qd;
-  const int64_t zstride = (int64_t)a.H * a.W * a.cout;
-  static_assert(256 * 8 / kWThreads == 4 && kWThreads == 512, "one box z-plane a round");
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int v = k * 64 + vyx;
-    if (kFull || valid(v)) {
-      const float* src = otile + v * kTileStride + 4 * qd;
-      *reinterpret_cast<f4*>(a.y + base + k * zstride) = f4{src[0], src[1], src[2], src[3]};
-    }
-  }
-}
-
-__device__ __forceinline__ void wino_epilogue_tail(const WinoArgs& a, const f4 (&yo)[2][2],
-                                                   float* otile, int tid, int lane, int wave,
-                                                   int b, int nt, int bzi, int byi, int bxi) {
-  // uniform over the workgroup
-  if (bzi * 4 + 4 <= a.D && byi * 8 + 8 <= a.H && bxi * 8 + 8 <= a.W)
-    wino_epilogue_tail_t<true>(a, yo, otile, tid, lane, wave, b, nt, bzi, byi, bxi);
-  else
-    wino_epilogue_tail_t<false>(a, yo, otile, tid, lane, wave, b, nt, bzi, byi, bxi);
-}
-
-__global__ __launch_bounds__(kWThreads, 1) void wino_x3_kernel(WinoArgs a) {
-  // three LDS objects: the compiler then knows that the halo DMA into s_raw does not write
-  // what the later reads of s_prm read
-  __shared__ __align__(16) f4 s_raw[2 * kRawSlots];  // two raw halo buffers
-  __shared__ __align__(16) f4 s_z[kZSlots];          // z-transformed planes
-  __shared__ __align__(16) f4 s_prm[kMaxChannels];   // pending-norm parameters
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int logical = xcd_remap(blockIdx.x, a.nwg);
-  const int nt = logical % a.ntn;
-  int box = logical / a.ntn;
-  const int bxi = box % a.nbx;
-  box /= a.nbx;
-  const int byi = box % a.nby;
-  box /= a.nby;
-  const int bzi = box % a.nbz;
-  const int b = box / a.nbz;
-  const int oz0 = bzi * 4, oy0 = byi * 8, ox0 = bxi * 8;
-  const int iz0 = oz0 - 1, iy0 = oy0 - 1, ix0 = ox0 - 1;
-  const int64_t bvox = (int64_t)b * a.D * a.H * a.W;
-
-  // ---- raw halo fetch of one chunk into buffer `buf` (LDS slot = line = voxel * 4 + quad);
-  // this thread's lines r * kWThreads + tid have fixed voxels: their offsets inside the batch
-  // item (-1 outside the volume or past the halo) are computed once
-  const int cq_line = tid & 3;
-  int vofs[kRawRounds];
-#pragma unroll
-  for (int r = 0; r < kRawRounds; ++r) {
-    const int line = r * kWThreads + tid;
-    int o = -1;
-    if (line < kRawLines) {
-      const int v = line >> 2;
-      const int hz = v / 100, rem = v - hz * 100;
-      const int hy = rem / 10, hx = rem - hy * 10;
-      const int z = iz0 + hz, yy = iy0 + hy, xx = ix0 + hx;
-      if ((unsigned)z < (unsigned)a.D && (unsigned)yy < (unsigned)a.H &&
-          (unsigned)xx < (unsigned)a.W)
-        o = (z * a.H + yy) * a.W + xx;
-    }
-    vofs[r] = o;
-  }
-  // past the last chunk (live = false) every line reads the zero line: the DMA is issued
-  // unconditionally, so no branch joins paths with different counts of loads in flight
-  auto fetch = [&](int chunk, int buf, bool live) __attribute__((always_inline)) {
-    const bool first = chunk < a.chunks0;
-    const float* src = first ? a.x0 : a.x1;
-    const int C = first ? a.c0 : a.c1;
-    const float* base = src + bvox * C + (first ? chunk : chunk - a.chunks0) * kWChunk + cq_line * 4;
-    f4* dst = s_raw + buf * kRawSlots + wave * 64;
-#pragma unroll
-    for (int r = 0; r < kRawRounds; ++r) {
-      // both addresses formed and one selected: no branch around the load, so the
-      // compiler's wait counts stay exact
-      const float* in = base + (int64_t)(vofs[r] < 0 ? 0 : vofs[r]) * C;
-      const float* g = live && vofs[r] >= 0 ? in : g_wino_zero;
-      __builtin_amdgcn_global_load_lds(
-          g, (__attribute__((address_space(3))) void*)(dst + r * kWThreads), 16, 0, 0);
-    }
-  };
-
-  // ---- pending InstanceNorm parameters of every input channel (both inputs, in chunk
-  // order) for this batch item
-  for (int c = tid; c < a.c0 + a.c1; c += kWThreads) {
-    const float4* pp = c < a.c0 ? a.nrm0 : a.nrm1;
-    const int C = c < a.c0 ? a.c0 : a.c1;
-    const int cc = c < a.c0 ? c : c - a.c0;
-    float4 v = make_float4(0.f, 1.f, 0.f, 0.f);
-    if (pp) v = pp[(int64_t)b * C + cc];
-    s_prm[c] = f4{v.x, v.y, v.z, 0.f};
-  }
-
-  // ---- pending norm + z-transform: thread (hy, hx, quad) of the 10 x 10 x 4 columns.  A
-  // halo wholly inside the volume (uniform over the workgroup) needs no padding selects.
-  const bool interior = iz0 >= 0 && iz0 + 6 <= a.D && iy0 >= 0 && iy0 + 10 <= a.H &&
-                        ix0 >= 0 && ix0 + 10 <= a.W;
-  auto transform_column = [&](auto inner, int chunk, int buf, int col) __attribute__((always_inline)) {
-    const int hy = col / 40, rem = col - hy * 40;
-    const int hx = rem >> 2, cq = rem & 3;
-    const bool first = chunk < a.chunks0;
-    const float s = (first ? a.act0 : a.act1) != 0 ? a.slope : 1.f;
-    // parameters of inputs without a pending norm are (0, 1, 0): the identity
-    float4 pm[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const f4 v = s_prm[chunk * kWChunk + cq * 4 + q];
-      pm[q] = make_float4(v[0], v[1], v[2], 0.f);
-    }
-    const f4* raw = s_raw + buf * kRawSlots + (hy * 10 + hx) * 4 + cq;
-    f4 d[6];
-#pragma unroll
-    for (int hz = 0; hz < 6; ++hz) d[hz] = raw[hz * 400];
-    if constexpr (decltype(inner)::value == 2) {
-      // no pending norm: the raw values (the padding lines read the zero line)
-    } else if constexpr (decltype(inner)::value == 1) {
-#pragma unroll
-      for (int hz = 0; hz < 6; ++hz) d[hz] = wino_norm(d[hz], pm, s);
-    } else {
-      const bool inyx =
-          (unsigned)(iy0 + hy) < (unsigned)a.H && (unsigned)(ix0 + hx) < (unsigned)a.W;
-#pragma unroll
-      for (int hz = 0; hz < 6; ++hz) {
-        // the padding stays zero; in-volume voxels take the pending norm
-        const f4 t = wino_norm(d[hz], pm, s);
-        const bool inside = inyx && (unsigned)(iz0 + hz) < (unsigned)a.D;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) d[hz][e] = inside ? t[e] : 0.f;
-      }
-    }
-    f4* dst = s_z + hy * kZRow + hx * 4 + cq;
-#pragma unroll
-    for (int tz = 0; tz < 2; ++tz) {
-      const f4 d0 = d[2 * tz], d1 = d[2 * tz + 1], d2 = d[2 * tz + 2], d3 = d[2 * tz + 3];
-      dst[(0 * 2 + tz) * kZPlane] = d0 - d2;
-      dst[(1 * 2 + tz) * kZPlane] = d1 + d2;
-      dst[(2 * 2 + tz) * kZPlane] = d2 - d1;
-      dst[(3 * 2 + tz) * kZPlane] = d1 - d3;
-    }
-  };
-  auto transform = [&](int chunk, int buf) __attribute__((always_inline)) {
-    if (tid < 400) {
-      if ((chunk < a.chunks0 ? a.nrm0 : a.nrm1) == nullptr)
-        transform_column(std::integral_constant<int, 2>{}, chunk, buf, tid);
-      else if (interior)
-        transform_column(std::integral_constant<int, 1>{}, chunk, buf, tid);
-      else
-        transform_column(std::integral_constant<int, 0>{}, chunk, buf, tid);
-    }
-  };
-
-  // ---- this lane's tile, channel half and transform positions: wave = (xz, half p), the
-  // half owning xy = 2p and 2p + 1
-  const int xz = wave >> 1, p = wave & 1;
-  const int t = lane & 31, tzl = t >> 4, tyl = (t >> 2) & 3, txl = t & 3, g8 = lane >> 5;
-  // LDS byte offset of this lane's first z-row read (tile patch corner, channel half g8)
-  const unsigned zb_lds = (unsigned)(uintptr_t)(
-      (__attribute__((address_space(3))) f4*)s_z + ((xz * 2 + tzl) * kZPlane + (2 * tyl) * kZRow +
-                                                    (2 * txl) * 4 + 2 * g8));
-
-  // packed U: [nt][chunk][xi = (xz * 4 + xy) * 4 + xx][hi | lo][64 lanes] x 16 bytes; step
-  // s (local xy = s / 4, xx = s % 4) of a chunk uses position xi = xz * 16 + p * 8 + s
-  const uint4* ub = a.u + ((int64_t)nt * a.chunks * 64 + xz * 16 + p * kSteps) * 128 + lane;
-  auto uaddr = [&](int chunk, int step) { return ub + ((int64_t)chunk * 64 + step) * 128; };
-
-  f16v acc[2][4];
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int x = 0; x < 4; ++x)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[j][x][r] = 0.f;
-
-  uint4 uh[kRing], ul[kRing];
-  fetch(0, 0, true);
-#pragma unroll
-  for (int s = 0; s < kRing; ++s) {
-    const uint4* up = uaddr(0, s);
-    uh[s] = up[0];
-    ul[s] = up[64];
-  }
-
-  // the three products of step s (local xy = s / 4, xx = s % 4) for two steps at a time,
-  // then the refill of their ring slots kRing steps ahead
-  auto products = [&](int s0, const float (&q)[4][8], int chunk) __attribute__((always_inline)) {
-    h8 ah[2], al[2];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int xx = (s0 + k) & 3;
-      float v[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        if (xx == 0) v[e] = q[0][e] - q[2][e];
-        else if (xx == 1) v[e] = q[1][e] + q[2][e];
-        else if (xx == 2) v[e] = q[2][e] - q[1][e];
-        else v[e] = q[1][e] - q[3][e];
-      }
-      split8(v, ah[k], al[k]);
-    }
-    const int xy = s0 >> 2, x0 = s0 & 3;
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-      acc[xy][x0 + k] = mfma32(ah[k], *reinterpret_cast<const h8*>(&uh[(s0 + k) % kRing]),
-                               acc[xy][x0 + k]);
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-      acc[xy][x0 + k] = mfma32(ah[k], *reinterpret_cast<const h8*>(&ul[(s0 + k) % kRing]),
-                               acc[xy][x0 + k]);
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int s = s0 + k, slot = s % kRing;
-      acc[xy][x0 + k] = mfma32(al[k], *reinterpret_cast<const h8*>(&uh[slot]), acc[xy][x0 + k]);
-      // unconditional (past the last chunk the last chunk's words are read again)
-      const int ns = s + kRing;
-      int nchunk = ns < kSteps ? chunk : chunk + 1;
-      nchunk = nchunk < a.chunks ? nchunk : a.chunks - 1;
-      const uint4* up = uaddr(nchunk, ns & (kSteps - 1));
-      uh[slot] = up[0];
-      ul[slot] = up[64];
-    }
-  };
-
-  // one y-row of Q at a time: half 0 forms xy 0, 1 (r0 - r2, r1 + r2), half 1 xy 2, 3
-  // (r2 - r1, r1 - r3), i.e. Q0 = R[2p] - R[2 - p] and Q1 = R[1] + sg R[2 + p] with sg = +-1
-  // (fma: one rounding, as the add or subtract)
-  const float sg = p ? -1.f : 1.f;
-  // the host launches only layers with input channels (chunks >= 1): without this the
-  // compiler keeps a zeroed copy of the accumulators for the loop-skipping path as well
-  __builtin_assume(a.chunks > 0);
-  for (int chunk = 0; chunk < a.chunks; ++chunk) {
-    const int buf = chunk & 1;
-    __builtin_amdgcn_s_waitcnt(0);  // this thread's halo lines and B operands have landed
-    __syncthreads();                 // every thread's; the z-planes are free
-    transform(chunk, buf);
-    // the next chunk's halo into the other buffer (free since this chunk began), after this
-    // thread's reads of `buf`: a whole chunk of products covers its latency
-    const bool more = chunk + 1 < a.chunks;
-    fetch(more ? chunk + 1 : chunk, buf ^ 1, more);
-    // z-planes written: this thread's LDS writes complete, then the barrier.  Not
-    // __syncthreads(), whose release fence would also wait for the DMA just issued (nothing
-    // reads that buffer before the next chunk's full wait and barrier).
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      f4 va[8], vb[8];  // [column * 2 + half]
-      zrow_pair(zb_lds + (j == 0 ? 2 * p : 1) * kZRow * 16,
-                zb_lds + (j == 0 ? 2 - p : 2 + p) * kZRow * 16, va, vb);
-      float q[4][8];
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            q[c][4 * h + e] = j == 0 ? va[2 * c + h][e] - vb[2 * c + h][e]
-                                     : fmaf(sg, vb[2 * c + h][e], va[2 * c + h][e]);
-      products(4 * j, q, chunk);
-      products(4 * j + 2, q, chunk);
-    }
-  }
-
-  // ---- epilogue
-  // x- and y-output transforms of this wave's positions: per accumulator element, this
-  // half's share of the (oy, ox) outputs of its tile row for this xz (oy0 = xy0 + xy1 +
-  // xy2, oy1 = xy1 - xy2 - xy3)
-  __builtin_amdgcn_s_waitcnt(0);  // the last (zero-line) DMA has landed in s_raw
-  __syncthreads();                 // every wave is past its last z-plane read and DMA
-  // partials [wave][tile][column] x (oy0ox0, oy0ox1, oy1ox0, oy1ox1): waves 0-4 in s_raw,
-  // waves 5-7 in s_z
-  auto part = [&](int w, int tile, int c) -> f4& {
-    const int i = (w * 32 + tile) * 32 + c;
-    return i < 2 * kRawSlots ? s_raw[i] : s_z[i - 2 * kRawSlots];
-  };
-  const int col = lane & 31;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    float xo[2][2];  // [local xy][ox]
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const float m0 = acc[j][0][r], m1 = acc[j][1][r], m2 = acc[j][2][r], m3 = acc[j][3][r];
-      xo[j][0] = (m0 + m1) + m2;
-      xo[j][1] = (m1 - m2) - m3;
-    }
-    const f4 pv = p == 0 ? f4{xo[0][0] + xo[1][0], xo[0][1] + xo[1][1], xo[1][0], xo[1][1]}
-                         : f4{xo[0][0], xo[0][1], -(xo[0][0] + xo[1][0]), -(xo[0][1] + xo[1][1])};
-    const int tile = 8 * (r >> 2) + 4 * g8 + (r & 3);
-    part(wave, tile, col) = pv;
-  }
-  __syncthreads();
-  // z-output transform over the four xz partials: oz0 = P0 + P1 + P2, oz1 = P1 - P2 - P3;
-  // then the weight scale and the bias
-  constexpr int kPairs = 32 * 32 / kWThreads;
-  f4 yo[kPairs][2];  // [pair][oz]
-  const float bias_c = a.bias ? a.bias[nt * 32 + (tid & 31)] : 0.f;
-#pragma unroll
-  for (int k = 0; k < kPairs; ++k) {
-    const int idx = tid + k * kWThreads;
-    const int tile = idx >> 5, c = idx & 31;
-    f4 pz[4];
-#pragma unroll
-    for (int z = 0; z < 4; ++z) pz[z] = part(2 * z, tile, c) + part(2 * z + 1, tile, c);
-    const f4 y0 = (pz[0] + pz[1]) + pz[2];
-    const f4 y1 = (pz[1] - pz[2]) - pz[3];
-    yo[k][0] = y0 * a.out_scale;
-    yo[k][1] = y1 * a.out_scale;
-    if (a.bias) {
-      yo[k][0] = yo[k][0] + bias_c;
-      yo[k][1] = yo[k][1] + bias_c;
-    }
-  }
-  __syncthreads();  // every thread's partial reads are done: the tile may overwrite them
-  wino_epilogue_tail(a, yo, reinterpret_cast<float*>(s_raw), tid, lane, wave, b, nt, bzi, byi,
-                     bxi);
-}
-
-// ---- persistent variant ------------------------------------------------------------
-// One workgroup a CU loops over boxes.  The eight XCDs take contiguous ranges of the
-// (column block, box) pairs, column block slowest, and the G workgroups of an XCD interleave
-// over its range, so an XCD's L2 holds one column block's packed weights and neighbouring
-// boxes' halos.  The box arithmetic is the kernel above's, in the same order (the results
-// are bit-identical); what changes is the overlap between boxes: the last chunk of a box
-// issues the next box's first halo DMA and its B-operand refills load the next box's first
-// four steps, so the next box starts with its halo and weights landed instead of waiting for
-// them (~8k cycles a box).  The epilogue therefore keeps out of the raw halo buffers (its
-// partials, two rounds of 16 tiles, and its output tile live in the z-planes and the
-// parameter table, whose next box's values are loaded after it), its barriers wait for LDS
-// only, and the bias is read at box start.
 struct WinoBox {
   int nt, b, bzi, byi, bxi;
 };
@@ -592,97 +205,168 @@ __device__ __forceinline__ WinoBox wino_box(const WinoArgs& a, int v) {
   return r;
 }
 
-
-__global__ __launch_bounds__(kWThreads, 1) void wino_x3p_kernel(WinoArgs a) {
-  __shared__ __align__(16) f4 s_raw[2 * kRawSlots];  // two raw halo buffers
-  __shared__ __align__(16) f4 s_z[kZSlots];          // z-planes; epilogue partials and tile
-  __shared__ __align__(16) f4 s_prm[kMaxChannels];   // parameters; epilogue partials
-  // the bias of the current box's column block (read in the epilogue from LDS: a global
-  // read there would wait for the next box's halo DMA)
-  __shared__ float s_bias[32];
+template <int ZB, bool TALL>
+__global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
+  using G = WinoBoxGeom<ZB, TALL>;
+  __shared__ __align__(16) f4 s_raw[2 * G::buf];             // two raw halo buffers
+  __shared__ __align__(16) float s_prm[3 * kMaxChannels];    // mean, scale, beta by channel
+  __shared__ __align__(16) float s_bias[32];                 // of the current column block
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   // this workgroup's (column block, box) pairs: XCD blockIdx % 8 takes a contiguous range,
-  // its G workgroups interleave over it (the grid is a multiple of 8)
-  const int xcd = blockIdx.x & 7, G = gridDim.x >> 3;
+  // its workgroups interleave over it (the grid is a multiple of 8)
+  const int xcd = blockIdx.x & 7, stride = gridDim.x >> 3;
   const int vq = a.nvirt >> 3, vr = a.nvirt & 7;
   const int vbeg = xcd < vr ? xcd * (vq + 1) : vr * (vq + 1) + (xcd - vr) * vq;
   const int vend = vbeg + vq + (xcd < vr ? 1 : 0);
   int v = vbeg + (int)(blockIdx.x >> 3);
   if (v >= vend) return;  // uniform over the workgroup, before any barrier
-  const int xz = wave >> 1, p = wave & 1;
-  const float sg = p ? -1.f : 1.f;
   __builtin_assume(a.chunks > 0);
-  constexpr int kPairs = 32 * 32 / kWThreads;
+  const int64_t plane_vox = (int64_t)a.H * a.W;
+  constexpr int kRounds = G::hz / 2 * 3;
+  uint64_t zero = (uint64_t)g_wino_zero;
+  asm volatile("" : "+s"(zero));  // held, not loaded from the GOT at every use
 
-  // halo line offsets of a box inside its batch item (-1 outside the volume or the halo)
-  auto box_vofs = [&](int tid, const WinoBox& bx, int (&vofs)[kRawRounds])
+  // ---- raw halo lines.  Round 3 k + j of this thread is slot j * 512 + tid of the plane pair
+  // 2 k, 2 k + 1: three in-plane patterns j, the plane uniform over a wave.
+  auto round_plane = [&](int k, int j) { return 2 * k + ((j == 2 || (j == 1 && wave >= 4)) ? 1 : 0); };
+  // in-plane voxel offset (-1 outside the volume or on a padding slot) and channel quad of
+  // the three patterns for a box corner
+  auto box_lines = [&](int tid, const WinoBox& bx, int (&yx)[3], int& quads)
       __attribute__((always_inline)) {
-    const int iz0 = bx.bzi * 4 - 1, iy0 = bx.byi * 8 - 1, ix0 = bx.bxi * 8 - 1;
+    quads = 0;
 #pragma unroll
-    for (int r = 0; r < kRawRounds; ++r) {
-      const int line = r * kWThreads + tid;
-      int o = -1;
-      if (line < kRawLines) {
-        const int hv = line >> 2;
-        const int hz = hv / 100, rem = hv - hz * 100;
-        const int hy = rem / 10, hx = rem - hy * 10;
-        const int z = iz0 + hz, yy = iy0 + hy, xx = ix0 + hx;
-        if ((unsigned)z < (unsigned)a.D && (unsigned)yy < (unsigned)a.H &&
-            (unsigned)xx < (unsigned)a.W)
-          o = (z * a.H + yy) * a.W + xx;
-      }
-      vofs[r] = o;
+    for (int j = 0; j < 3; ++j) {
+      const int s = j == 0 ? tid : j == 1 ? (tid < 256 ? 512 + tid : tid - 256) : 256 + tid;
+      int t = s;
+      if constexpr (TALL) t = s < G::py * 4 + G::jump ? s : s < G::py * 8 + 2 * G::jump ? s - G::jump
+                                                                                       : s - 2 * G::jump;
+      const int yi = t / G::py, rem = t - yi * G::py;
+      const int yp = rem / G::pyp, rx = rem - yp * G::pyp;
+      const int xp = rx / G::pxp, rq = rx - xp * G::pxp;
+      const int hy = 2 * yi + yp, hx = 2 * (rq >> 2) + xp;
+      const int yy = bx.byi * G::by - 1 + hy, xx = bx.bxi * G::bx - 1 + hx;
+      const bool line = s - t == G::jump * (yi >> 2) && rem < 2 * G::pyp && hy < G::hy &&
+                        (unsigned)yy < (unsigned)a.H && (unsigned)xx < (unsigned)a.W;
+      yx[j] = line ? yy * a.W + xx : -1;
+      quads |= (rq & 3) << (8 * j);
     }
   };
-  // chunk `chunk` of item b's halo lines into buffer `buf` (live = false: the zero line)
-  auto fetch = [&](int tid, int b, const int (&vofs)[kRawRounds], int chunk, int buf, bool live)
-      __attribute__((always_inline)) {
+  // Rounds [r0, r1) of a chunk of a box's halo into buffer `buf` (live = false: the zero line),
+  // spread over the previous chunk's products.
+  struct Source {
+    uint64_t base;         // channel chunk of the halo's first plane (may lie outside the volume)
+    int64_t plane_bytes;
+    int C, z0;
+  };
+  auto source = [&](const WinoBox& bx, int chunk, bool live) __attribute__((always_inline)) {
     const bool first = chunk < a.chunks0;
-    const float* src = first ? a.x0 : a.x1;
-    const int C = first ? a.c0 : a.c1;
-    const int64_t bv = (int64_t)b * a.D * a.H * a.W;
-    const float* base = src + bv * C + (first ? chunk : chunk - a.chunks0) * kWChunk + (tid & 3) * 4;
-    f4* dst = s_raw + buf * kRawSlots + wave * 64;
+    Source r;
+    r.C = first ? a.c0 : a.c1;
+    r.plane_bytes = plane_vox * r.C * 4;
+    const int z = bx.bzi * ZB - 1;
+    r.base = (uint64_t)(first ? a.x0 : a.x1) + ((int64_t)bx.b * a.D + z) * r.plane_bytes +
+             (first ? chunk : chunk - a.chunks0) * kWChunk * 4;
+    r.z0 = live ? z : INT32_MIN / 2;
+    return r;
+  };
+  auto fetch = [&](const Source& src, const int (&yx)[3], int quads, int buf, auto r0c, auto r1c)
+      __attribute__((always_inline)) {
+    f4* dst = s_raw + buf * G::buf + wave * 64;
 #pragma unroll
-    for (int r = 0; r < kRawRounds; ++r) {
-      const float* in = base + (int64_t)(vofs[r] < 0 ? 0 : vofs[r]) * C;
-      const float* g = live && vofs[r] >= 0 ? in : g_wino_zero;
+    for (int r = decltype(r0c)::value; r < decltype(r1c)::value; ++r) {
+      const int k = r / 3, j = r % 3, p = round_plane(k, j);
+      // a per-lane plane index keeps the check a select of two addresses instead of a branch
+      const int z = yx[j] >= 0 ? src.z0 + p : -1;
+      const uint64_t in = src.base + p * src.plane_bytes +
+                          ((int64_t)yx[j] * src.C + ((quads >> (8 * j)) & 3) * 4) * 4;
+      const uint64_t g = (unsigned)z < (unsigned)a.D ? in : zero;
       __builtin_amdgcn_global_load_lds(
-          g, (__attribute__((address_space(3))) void*)(dst + r * kWThreads), 16, 0, 0);
+          (const void*)g, (__attribute__((address_space(3))) void*)(dst + r * kWThreads), 16, 0, 0);
     }
   };
+  // pending-norm parameters of every input channel (both inputs, in chunk order) of item b
   auto load_prm = [&](int tid, int b) __attribute__((always_inline)) {
+    if (!a.nrm0 && !a.nrm1) return;
     for (int c = tid; c < a.c0 + a.c1; c += kWThreads) {
       const float4* pp = c < a.c0 ? a.nrm0 : a.nrm1;
       const int C = c < a.c0 ? a.c0 : a.c1;
       const int cc = c < a.c0 ? c : c - a.c0;
       float4 pv = make_float4(0.f, 1.f, 0.f, 0.f);
       if (pp) pv = pp[(int64_t)b * C + cc];
-      s_prm[c] = f4{pv.x, pv.y, pv.z, 0.f};
+      s_prm[c] = pv.x;
+      s_prm[kMaxChannels + c] = pv.y;
+      s_prm[2 * kMaxChannels + c] = pv.z;
     }
   };
-  // packed U words of column block ntb, chunk, step (local position) for this lane
-  auto uaddr = [&](int lane, int ntb, int chunk, int step) {
-    return a.u + (((int64_t)ntb * a.chunks + chunk) * 64 + xz * 16 + p * kSteps + step) * 128 + lane;
+  // The input's pending InstanceNorm on this thread's lines of the chunk, in place (the apply
+  // pass's operations: t = fma(x - mean, scale, beta), then max(s * t, t) with s = the
+  // LeakyReLU slope under the activation and s = 1, the identity, without it).  Lines outside
+  // the volume stay zero.
+  auto normalise = [&](const WinoBox& bx, const int (&yx)[3], int quads, int chunk, int buf)
+      __attribute__((always_inline)) {
+    const bool first = chunk < a.chunks0;
+    if ((first ? a.nrm0 : a.nrm1) == nullptr) return;
+    const float s = (first ? a.act0 : a.act1) != 0 ? a.slope : 1.f;
+    f4* lines = s_raw + buf * G::buf + threadIdx.x;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      if (yx[j] < 0) continue;
+      const float* prm = s_prm + chunk * kWChunk + ((quads >> (8 * j)) & 3) * 4;
+      const f4 mean = *reinterpret_cast<const f4*>(prm);
+      const f4 scale = *reinterpret_cast<const f4*>(prm + kMaxChannels);
+      const f4 beta = *reinterpret_cast<const f4*>(prm + 2 * kMaxChannels);
+      f4 d[G::hz / 2];
+#pragma unroll
+      for (int k = 0; k < G::hz / 2; ++k) d[k] = lines[(3 * k + j) * kWThreads];
+#pragma unroll
+      for (int k = 0; k < G::hz / 2; ++k) {
+        const int z = bx.bzi * ZB - 1 + round_plane(k, j);
+        if ((unsigned)z >= (unsigned)a.D) continue;  // uniform over the wave
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float t = fmaf(d[k][e] - mean[e], scale[e], beta[e]);
+          d[k][e] = fmaxf(s * t, t);
+        }
+        lines[(3 * k + j) * kWThreads] = d[k];
+      }
+    }
   };
 
-  // loop-carried state: the halo offsets of the box whose first chunk is in flight, the
-  // B-operand ring, the bias of the current column block
-  int vofs[kRawRounds];
-  uint4 uh[kRing], ul[kRing];
+  // ---- this wave's positions: row pair (a, b) and sign of xy, columns P, Q, R and sign of xx.
+  // Q0 = d[a] + sy d[b]; the first position is P - Q (xx = 0, or minus xx = 3, a sign that
+  // the output transform undoes), the second R + sx Q (xx = 1 or 2).
+  const int xy = wave >> 1, h = wave & 1;
+  const int ra = xy == 0 ? 0 : xy == 2 ? 2 : 1, rb = xy == 2 ? 1 : xy == 3 ? 3 : 2;
+  const float sy = xy == 1 ? 1.f : -1.f;
+  const int cp = h ? 3 : 0, cq = h ? 1 : 2, cr = h ? 2 : 1;
+  const float sx = h ? -1.f : 1.f;
+  // packed U: [nt][chunk][position in wave order][z tap][hi | lo][64 lanes] x 16 bytes
+  auto uaddr = [&](int lane, int nt, int chunk) {
+    return a.u + (((int64_t)nt * a.chunks + chunk) * kPositions + 2 * wave) * 3 * kTapWords + lane;
+  };
+  uint4 ub[2][3][2];  // [position][z tap][hi | lo]
+  auto load_u = [&](const uint4* base, int kz) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int part = 0; part < 2; ++part)
+        ub[p][kz][part] = base[(p * 3 + kz) * kTapWords + part * 64];
+  };
+
+  // loop-carried: the lines of the box whose first chunk is in flight, its U, the raw buffer
+  int yx[3], quads, buf = 0;
   {
     const int tid = threadIdx.x;
     const WinoBox first = wino_box(a, v);
-    box_vofs(tid, first, vofs);
+    box_lines(tid, first, yx, quads);
     load_prm(tid, first.b);
-    fetch(tid, first.b, vofs, 0, 0, true);
-#pragma unroll
-    for (int s0 = 0; s0 < kRing; ++s0) {
-      const uint4* up = uaddr(tid & 63, first.nt, 0, s0);
-      uh[s0] = up[0];
-      ul[s0] = up[64];
-    }
     if (tid < 32) s_bias[tid] = a.bias ? a.bias[first.nt * 32 + tid] : 0.f;
+    fetch(source(first, 0, true), yx, quads, 0, std::integral_constant<int, 0>{},
+          std::integral_constant<int, kRounds>{});
+    const uint4* up = uaddr(tid & 63, first.nt, 0);
+#pragma unroll
+    for (int kz = 0; kz < 3; ++kz) load_u(up, kz);
+    lds_barrier();  // the parameters and the bias
   }
 
   for (;;) {
@@ -692,237 +376,252 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_x3p_kernel(WinoArgs a) {
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63;
     const WinoBox cur = wino_box(a, v);
-    const int vnext = v + G;
+    const int vnext = v + stride;
     const bool more = vnext < vend;
     const int vn = more ? vnext : v;  // the next box (this one again after the last)
-    const int nnt = vn / a.nbox;
-    const int iz0 = cur.bzi * 4 - 1, iy0 = cur.byi * 8 - 1, ix0 = cur.bxi * 8 - 1;
-    const bool interior = iz0 >= 0 && iz0 + 6 <= a.D && iy0 >= 0 && iy0 + 10 <= a.H &&
-                          ix0 >= 0 && ix0 + 10 <= a.W;
-    const int t = lane & 31, tzl = t >> 4, tyl = (t >> 2) & 3, txl = t & 3, g8 = lane >> 5;
-    const unsigned zb_lds = (unsigned)(uintptr_t)(
-        (__attribute__((address_space(3))) f4*)s_z + ((xz * 2 + tzl) * kZPlane + (2 * tyl) * kZRow +
-                                                      (2 * txl) * 4 + 2 * g8));
-    auto transform_column = [&](auto inner, int chunk, int buf, int col)
-        __attribute__((always_inline)) {
-      const int hy = col / 40, rem = col - hy * 40;
-      const int hx = rem >> 2, cq = rem & 3;
-      const bool first = chunk < a.chunks0;
-      const float sl = (first ? a.act0 : a.act1) != 0 ? a.slope : 1.f;
-      float4 pm[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const f4 pq = s_prm[chunk * kWChunk + cq * 4 + q];
-        pm[q] = make_float4(pq[0], pq[1], pq[2], 0.f);
-      }
-      const f4* raw = s_raw + buf * kRawSlots + (hy * 10 + hx) * 4 + cq;
-      f4 d[6];
-#pragma unroll
-      for (int hz = 0; hz < 6; ++hz) d[hz] = raw[hz * 400];
-      if constexpr (decltype(inner)::value == 2) {
-        // no pending norm: the raw values (the padding lines read the zero line)
-      } else if constexpr (decltype(inner)::value == 1) {
-#pragma unroll
-        for (int hz = 0; hz < 6; ++hz) d[hz] = wino_norm(d[hz], pm, sl);
-      } else {
-        const bool inyx =
-            (unsigned)(iy0 + hy) < (unsigned)a.H && (unsigned)(ix0 + hx) < (unsigned)a.W;
-#pragma unroll
-        for (int hz = 0; hz < 6; ++hz) {
-          const f4 tq = wino_norm(d[hz], pm, sl);
-          const bool inside = inyx && (unsigned)(iz0 + hz) < (unsigned)a.D;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) d[hz][e] = inside ? tq[e] : 0.f;
-        }
-      }
-      f4* dst = s_z + hy * kZRow + hx * 4 + cq;
-#pragma unroll
-      for (int tz = 0; tz < 2; ++tz) {
-        const f4 d0 = d[2 * tz], d1 = d[2 * tz + 1], d2 = d[2 * tz + 2], d3 = d[2 * tz + 3];
-        dst[(0 * 2 + tz) * kZPlane] = d0 - d2;
-        dst[(1 * 2 + tz) * kZPlane] = d1 + d2;
-        dst[(2 * 2 + tz) * kZPlane] = d2 - d1;
-        dst[(3 * 2 + tz) * kZPlane] = d1 - d3;
-      }
-    };
+    const WinoBox nxt = wino_box(a, vn);
 
-    f16v acc[2][4];
+    // LDS byte addresses of this lane's six patch points in plane 0 of buffer 0
+    unsigned ad[6];
+    {
+      const int t = lane & 31, g8 = lane >> 5;
+      const int tyl = TALL ? t >> 2 : t >> 3, txl = TALL ? t & 3 : t & 7;
+      const unsigned raw0 = (unsigned)(uintptr_t)((__attribute__((address_space(3))) f4*)s_raw);
+      auto point = [&](int r, int c) {
+        const int yi = tyl + (r >> 1);
+        return raw0 + 16u * (unsigned)(yi * G::py + G::jump * (yi >> 2) + (r & 1) * G::pyp +
+                                       (c & 1) * G::pxp + (txl + (c >> 1)) * 4 + 2 * g8);
+      };
+      ad[0] = point(ra, cp);
+      ad[1] = point(ra, cq);
+      ad[2] = point(ra, cr);
+      ad[3] = point(rb, cp);
+      ad[4] = point(rb, cq);
+      ad[5] = point(rb, cr);
+    }
+    {
+      const unsigned o = buf ? (unsigned)(G::buf * 16) : 0u;
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-      for (int x = 0; x < 4; ++x)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[jj][x][r] = 0.f;
+      for (int i = 0; i < 6; ++i) ad[i] += o;
+    }
 
-    // the three products of steps s0, s0 + 1, then their ring refills kRing steps ahead:
-    // past the chunk's last step the next chunk's, past the box's last chunk the next box's
-    // first chunk's (column block nnt)
-    auto products = [&](int s0, const float (&q)[4][8], int chunk) __attribute__((always_inline)) {
-      h8 ah[2], al[2];
+    f16v acc[2][ZB];
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const int xx = (s0 + k) & 3;
-        float vv[8];
+    for (int p = 0; p < 2; ++p)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          if (xx == 0) vv[e] = q[0][e] - q[2][e];
-          else if (xx == 1) vv[e] = q[1][e] + q[2][e];
-          else if (xx == 2) vv[e] = q[2][e] - q[1][e];
-          else vv[e] = q[1][e] - q[3][e];
+      for (int z = 0; z < ZB; ++z)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[p][z][r] = 0.f;
+
+    // input plane Z of the halo: V of both positions, then its products with every z tap kz
+    // whose output plane Z - kz lies in the box
+    auto plane = [&](auto zc) __attribute__((always_inline)) {
+      constexpr int Z = decltype(zc)::value;
+      f4 d[12];
+      read_patch<Z>(ad, d);
+      float vp[8], vq8[8], vr8[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        vp[e] = fmaf(sy, d[6 + (e >> 2)][e & 3], d[e >> 2][e & 3]);
+        vq8[e] = fmaf(sy, d[8 + (e >> 2)][e & 3], d[2 + (e >> 2)][e & 3]);
+        vr8[e] = fmaf(sy, d[10 + (e >> 2)][e & 3], d[4 + (e >> 2)][e & 3]);
+      }
+      float va[8], vb[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        va[e] = vp[e] - vq8[e];
+        vb[e] = fmaf(sx, vq8[e], vr8[e]);
+      }
+      h8 hi[2], lo[2];
+      split8(va, hi[0], lo[0]);
+      split8(vb, hi[1], lo[1]);
+#pragma unroll
+      for (int product = 0; product < 3; ++product)
+#pragma unroll
+        for (int kz = 0; kz < 3; ++kz) {
+          constexpr int none = -1;
+          const int o = Z - kz >= 0 && Z - kz < ZB ? Z - kz : none;
+          if (o == none) continue;
+#pragma unroll
+          for (int p = 0; p < 2; ++p)
+            acc[p][o] = mfma32(product == 2 ? lo[p] : hi[p],
+                               *reinterpret_cast<const h8*>(&ub[p][kz][product == 1 ? 1 : 0]),
+                               acc[p][o]);
         }
-        split8(vv, ah[k], al[k]);
-      }
-      const int xy = s0 >> 2, x0 = s0 & 3;
-#pragma unroll
-      for (int k = 0; k < 2; ++k)
-        acc[xy][x0 + k] = mfma32(ah[k], *reinterpret_cast<const h8*>(&uh[(s0 + k) % kRing]),
-                                 acc[xy][x0 + k]);
-#pragma unroll
-      for (int k = 0; k < 2; ++k)
-        acc[xy][x0 + k] = mfma32(ah[k], *reinterpret_cast<const h8*>(&ul[(s0 + k) % kRing]),
-                                 acc[xy][x0 + k]);
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const int st = s0 + k, slot_r = st % kRing;
-        acc[xy][x0 + k] = mfma32(al[k], *reinterpret_cast<const h8*>(&uh[slot_r]), acc[xy][x0 + k]);
-        const int ns = st + kRing;
-        const bool wrap = ns >= kSteps && chunk + 1 >= a.chunks;
-        const uint4* up = uaddr(lane, wrap ? nnt : cur.nt,
-                                ns < kSteps ? chunk : (wrap ? 0 : chunk + 1), ns & (kSteps - 1));
-        uh[slot_r] = up[0];
-        ul[slot_r] = up[64];
-      }
     };
 
     for (int chunk = 0; chunk < a.chunks; ++chunk) {
-      const int buf = chunk & 1;
-      __builtin_amdgcn_s_waitcnt(0);  // this thread's halo lines and B operands have landed
-      __syncthreads();                 // every thread's; the z-planes are free
-      if (tid < 400) {
-        if ((chunk < a.chunks0 ? a.nrm0 : a.nrm1) == nullptr)
-          transform_column(std::integral_constant<int, 2>{}, chunk, buf, tid);
-        else if (interior)
-          transform_column(std::integral_constant<int, 1>{}, chunk, buf, tid);
-        else
-          transform_column(std::integral_constant<int, 0>{}, chunk, buf, tid);
-      }
-      // the next chunk's halo into the other buffer; after the box's last chunk the next
-      // box's first chunk (the zero line after the last box)
-      if (chunk + 1 < a.chunks) {
-        fetch(tid, cur.b, vofs, chunk + 1, buf ^ 1, true);
-      } else {
-        // (from an opaque copy of the thread index: computed here, not hoisted to the box
-        // start and held through the chunk loop)
+      __builtin_amdgcn_s_waitcnt(0);  // this thread's halo lines and U have landed
+      normalise(cur, yx, quads, chunk, buf);
+      lds_barrier();  // every thread's lines; the other buffer is free
+      const bool last = chunk + 1 == a.chunks;
+      // the next chunk's halo; after the box's last chunk the next box's first (the zero line
+      // after the last box)
+      if (last) {
         int tid_n = tid;
-        asm volatile("" : "+v"(tid_n));
-        const WinoBox nb = wino_box(a, vn);
-        box_vofs(tid_n, nb, vofs);
-        fetch(tid_n, nb.b, vofs, 0, buf ^ 1, more);
+        asm volatile("" : "+v"(tid_n));  // computed here, not hoisted and held
+        box_lines(tid_n, nxt, yx, quads);
       }
-      lds_barrier();
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        f4 va[8], vb[8];
-        zrow_pair(zb_lds + (j == 0 ? 2 * p : 1) * kZRow * 16,
-                  zb_lds + (j == 0 ? 2 - p : 2 + p) * kZRow * 16, va, vb);
-        float q[4][8];
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              q[c][4 * h + e] = j == 0 ? va[2 * c + h][e] - vb[2 * c + h][e]
-                                       : fmaf(sg, vb[2 * c + h][e], va[2 * c + h][e]);
-        products(4 * j, q, chunk);
-        products(4 * j + 2, q, chunk);
+      const Source src = source(last ? nxt : cur, last ? 0 : chunk + 1, !last || more);
+      auto rounds = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int I = decltype(ic)::value;
+        fetch(src, yx, quads, buf ^ 1, std::integral_constant<int, I * kRounds / ZB>{},
+              std::integral_constant<int, (I + 1) * kRounds / ZB>{});
+      };
+      const uint4* un = uaddr(lane, last ? nxt.nt : cur.nt, last ? 0 : chunk + 1);
+      rounds(std::integral_constant<int, 0>{});
+      plane(std::integral_constant<int, 0>{});
+      rounds(std::integral_constant<int, 1>{});
+      plane(std::integral_constant<int, 1>{});
+      if constexpr (ZB == 4) {
+        rounds(std::integral_constant<int, 2>{});
+        plane(std::integral_constant<int, 2>{});
+        rounds(std::integral_constant<int, 3>{});
+        plane(std::integral_constant<int, 3>{});
       }
+      load_u(un, 0);
+      plane(std::integral_constant<int, ZB>{});
+      load_u(un, 1);
+      plane(std::integral_constant<int, ZB + 1>{});
+      load_u(un, 2);
+      const unsigned flip = buf ? 0u - (unsigned)(G::buf * 16) : (unsigned)(G::buf * 16);
+#pragma unroll
+      for (int i = 0; i < 6; ++i) ad[i] += flip;
+      buf ^= 1;
     }
 
-    // ---- epilogue in the z-planes and the parameter table only
-    lds_barrier();  // every wave is past its last z-plane read and parameter read
-    auto part = [&](int w, int tile, int c) -> f4& {
-      const int i = (w * 16 + tile) * 32 + c;  // 16 tiles a round
-      return i < kZSlots ? s_z[i] : s_prm[i - kZSlots];
-    };
-    const int col = lane & 31;
-    f4 yo[kPairs][2];
-    // this wave's partials of round h (p is uniform over the wave: one branch, no selects)
-    auto write_parts = [&](int h, auto P) __attribute__((always_inline)) {
+    // ---- epilogue, in the raw buffer of the box's last chunk
+    lds_barrier();  // every wave is past its last read of it
+    float* part = reinterpret_cast<float*>(s_raw + (buf ^ 1) * G::buf);
+    f4* red = s_raw + (buf ^ 1) * G::buf + kPartSlots;
+    if (nxt.b != cur.b) load_prm(tid, nxt.b);  // visible after the barriers below
+    const int quad = tid & 7, rho = (tid >> 3) & 31, ox = tid >> 8;
+    const f4 bias = *reinterpret_cast<const f4*>(s_bias + 4 * quad);
+    f4 yo[ZB][2];  // [z][oy]
 #pragma unroll
-      for (int r = 8 * h; r < 8 * h + 8; ++r) {
-        float xo[2][2];
+    for (int z = 0; z < ZB; ++z) {
+      // partials [wave][ox][tile][column]; tile row r sits at rho(r) = (r / 8) * 8 + (r % 4) * 2 +
+      // (r / 4) % 2, so that a wave's two row groups (r and r + 4) write different banks
+      float* pw = part + wave * 2048 + (lane >> 5) * 32 + (lane & 31);
+      auto write_parts = [&](auto hc) __attribute__((always_inline)) {
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-          const float m0 = acc[jj][0][r], m1 = acc[jj][1][r], m2 = acc[jj][2][r], m3 = acc[jj][3][r];
-          xo[jj][0] = (m0 + m1) + m2;
-          xo[jj][1] = (m1 - m2) - m3;
+        for (int r = 0; r < 16; ++r) {
+          const float ma = acc[0][z][r], mb = acc[1][z][r];
+          float x0, x1;
+          if constexpr (decltype(hc)::value == 0) {
+            x0 = ma + mb;  // xx 0, 1
+            x1 = mb;
+          } else {
+            x0 = mb;       // xx 2 and minus xx 3
+            x1 = ma - mb;
+          }
+          const int at = ((r >> 2) * 8 + (r & 3) * 2) * 32;
+          pw[at] = x0;
+          pw[1024 + at] = x1;
         }
-        f4 pv;
-        if constexpr (decltype(P)::value == 0)
-          pv = f4{xo[0][0] + xo[1][0], xo[0][1] + xo[1][1], xo[1][0], xo[1][1]};
-        else
-          pv = f4{xo[0][0], xo[0][1], -(xo[0][0] + xo[1][0]), -(xo[0][1] + xo[1][1])};
-        part(wave, 8 * (r >> 2) + 4 * g8 + (r & 3) - 16 * h, col) = pv;
-      }
-    };
-#pragma unroll
-    for (int h = 0; h < kPairs; ++h) {
-      if (p == 0)
-        write_parts(h, std::integral_constant<int, 0>{});
+      };
+      if (h == 0)
+        write_parts(std::integral_constant<int, 0>{});
       else
-        write_parts(h, std::integral_constant<int, 1>{});
+        write_parts(std::integral_constant<int, 1>{});
       lds_barrier();
-      {
-        const int tile = tid >> 5, c = tid & 31;
-        f4 pz[4];
+      if (z == 0 && nxt.nt != cur.nt && tid < 32)
+        s_bias[tid] = a.bias ? a.bias[nxt.nt * 32 + tid] : 0.f;  // every thread has read its own
+      const float* pr = part + ox * 1024 + rho * 32 + 4 * quad;
+      f4 m[4];
 #pragma unroll
-        for (int z = 0; z < 4; ++z) pz[z] = part(2 * z, tile, c) + part(2 * z + 1, tile, c);
-        const f4 y0 = (pz[0] + pz[1]) + pz[2];
-        const f4 y1 = (pz[1] - pz[2]) - pz[3];
-        yo[h][0] = y0 * a.out_scale;
-        yo[h][1] = y1 * a.out_scale;
-        if (a.bias) {
-          const float bc = s_bias[c];
-          yo[h][0] = yo[h][0] + bc;
-          yo[h][1] = yo[h][1] + bc;
-        }
-      }
+      for (int i = 0; i < 4; ++i)
+        m[i] = *reinterpret_cast<const f4*>(pr + (2 * i) * 2048) +
+               *reinterpret_cast<const f4*>(pr + (2 * i + 1) * 2048);
+      yo[z][0] = ((m[0] + m[1]) + m[2]) * a.out_scale + bias;
+      yo[z][1] = ((m[1] - m[2]) - m[3]) * a.out_scale + bias;
       lds_barrier();
     }
-    wino_epilogue_tail(a, yo, reinterpret_cast<float*>(s_z), tid, lane, wave, cur.b, cur.nt,
-                       cur.bzi, cur.byi, cur.bxi);
+    const int row = 8 * (rho >> 3) + 4 * (rho & 1) + ((rho >> 1) & 3);
+    const int yy = cur.byi * G::by + 2 * (TALL ? row >> 2 : row >> 3);
+    const int xx = cur.bxi * G::bx + 2 * (TALL ? row & 3 : row & 7) + ox;
+    const int z0 = cur.bzi * ZB;
+    const bool xin = xx < a.W;
+    auto valid = [&](int z, int oy) { return xin && yy + oy < a.H && z0 + z < a.D; };
+    if (a.stats) {
+      const int nz = min(ZB, a.D - z0), ny = min(G::by, a.H - cur.byi * G::by);
+      const int nx = min(G::bx, a.W - cur.bxi * G::bx);
+      const float cnt = (float)(nz * ny * nx);
+      f4 sm = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int z = 0; z < ZB; ++z)
+#pragma unroll
+        for (int oy = 0; oy < 2; ++oy)
+          if (valid(z, oy)) sm += yo[z][oy];
+      sm = sum_stride8(sm);
+      if (lane < 8) red[wave * 8 + quad] = sm;
+      lds_barrier();
+      f4 mean = red[quad];
+#pragma unroll
+      for (int w = 1; w < 8; ++w) mean += red[w * 8 + quad];
+      mean = mean / cnt;
+      f4 m2 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int z = 0; z < ZB; ++z)
+#pragma unroll
+        for (int oy = 0; oy < 2; ++oy)
+          if (valid(z, oy)) {
+            const f4 d = yo[z][oy] - mean;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m2[e] = fmaf(d[e], d[e], m2[e]);
+          }
+      m2 = sum_stride8(m2);
+      if (lane < 8) red[64 + wave * 8 + quad] = m2;
+      lds_barrier();
+      if (tid < 8) {
+        f4 t = red[64 + quad];
+#pragma unroll
+        for (int w = 1; w < 8; ++w) t += red[64 + w * 8 + quad];
+        const int tiles = a.nbz * a.nby * a.nbx;
+        const int tile = (cur.bzi * a.nby + cur.byi) * a.nbx + cur.bxi;
+        float4* out = a.stats + ((int64_t)cur.b * tiles + tile) * a.cout + cur.nt * 32 + 4 * quad;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] = make_float4(mean[e], t[e], cnt, 0.f);
+      }
+    }
+    float* out = a.y + (((int64_t)cur.b * a.D + z0) * plane_vox + (int64_t)yy * a.W + xx) * a.cout +
+                 cur.nt * 32 + 4 * quad;
+#pragma unroll
+    for (int z = 0; z < ZB; ++z)
+#pragma unroll
+      for (int oy = 0; oy < 2; ++oy)
+        if (valid(z, oy))
+          *reinterpret_cast<f4*>(out + (z * plane_vox + (int64_t)oy * a.W) * a.cout) = yo[z][oy];
     if (!more) break;
-    // the next box: its bias, and its item's parameters once every thread has read the tile
-    // and the partials out of the parameter table
-    if (nnt != cur.nt && tid < 32) s_bias[tid] = a.bias ? a.bias[nnt * 32 + tid] : 0.f;
     v = vnext;
-    lds_barrier();
-    load_prm(tid, wino_box(a, v).b);
   }
   // the last (zero-line) DMA lands before the workgroup's LDS is released
   __builtin_amdgcn_s_waitcnt(0);
 }
 
-// U[cout][cin][xi] = sum_{a,b,e} G[xz][a] G[xy][b] G[xx][e] w[cout][a][b][e][cin] in float64,
-// times `scale`, rounded to float32, split into fp16 halves.  Word layout:
-// packed[(((nt * chunks + chunk) * 64 + xi) * 2 + part) * 64 + lane], lane = column
-// (cout = nt * 32 + lane % 32) and k slot (cin = chunk channel 8 * (lane / 32) + q).
+// U[cout][cin][kz][xi] = sum_{b,e} G[xy][b] G[xx][e] w[cout][kz][b][e][cin] in float64, times
+// `scale`, rounded to float32, split into fp16 halves.  Word layout:
+// packed[((((nt * chunks + chunk) * 16 + pos) * 3 + kz) * 2 + part) * 64 + lane], pos = 2 * wave + i
+// in the kernel's order (xy = wave / 2; xx = 0, 1 for an even wave, 3, 2 for an odd one), lane =
+// column (cout = nt * 32 + lane % 32) and k slot (cin = chunk channel 8 * (lane / 32) + q).
 __global__ void pack_wino_weight_kernel(const float* __restrict__ w, uint4* __restrict__ out,
                                         int cout, int c1, int c2, int chunks0, int chunks,
                                         int ntn, float scale) {
   const double G[4][3] = {{1.0, 0.0, 0.0}, {0.5, 0.5, 0.5}, {0.5, -0.5, 0.5}, {0.0, 0.0, 1.0}};
   const int cin_total = c1 + c2;
-  const int64_t total = (int64_t)ntn * chunks * 64 * 64;
+  const int64_t total = (int64_t)ntn * chunks * kPositions * 3 * 64;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
        i += (int64_t)gridDim.x * blockDim.x) {
     const int lane = (int)(i & 63);
     int64_t rest = i >> 6;
-    const int xi = (int)(rest % 64);
-    rest /= 64;
+    const int kz = (int)(rest % 3);
+    rest /= 3;
+    const int pos = (int)(rest % kPositions);
+    rest /= kPositions;
     const int chunk = (int)(rest % chunks);
     const int nt = (int)(rest / chunks);
-    const int xz = xi >> 4, xy = (xi >> 2) & 3, xx = xi & 3;
+    const int xy = pos >> 2, odd = (pos >> 1) & 1, second = pos & 1;
+    const int xx = odd ? 3 - second : second;
     const int n = nt * 32 + (lane & 31);
     h8 hv, lv;
 #pragma unroll
@@ -939,31 +638,27 @@ __global__ void pack_wino_weight_kernel(const float* __restrict__ w, uint4* __re
       float v = 0.f;
       if (n < cout && wc >= 0) {
         double u = 0.0;
-        for (int az = 0; az < 3; ++az)
-          for (int ay = 0; ay < 3; ++ay)
-            for (int ax = 0; ax < 3; ++ax) {
-              const double gw = G[xz][az] * G[xy][ay] * G[xx][ax];
-              if (gw != 0.0)
-                u += gw * (double)w[(((int64_t)n * 3 + az) * 3 + ay) * 3 * cin_total +
-                                    (int64_t)ax * cin_total + wc];
-            }
+        for (int ay = 0; ay < 3; ++ay)
+          for (int ax = 0; ax < 3; ++ax) {
+            const double gw = G[xy][ay] * G[xx][ax];
+            if (gw != 0.0)
+              u += gw * (double)w[((((int64_t)n * 3 + kz) * 3 + ay) * 3 + ax) * cin_total + wc];
+          }
         v = (float)(u * (double)scale);
       }
-      const _Float16 h = (_Float16)v;
-      hv[q] = h;
-      lv[q] = (_Float16)(v - (float)h);
+      const _Float16 hh = (_Float16)v;
+      hv[q] = hh;
+      lv[q] = (_Float16)(v - (float)hh);
     }
-    const int64_t word = ((((int64_t)nt * chunks + chunk) * 64 + xi) * 2) * 64 + lane;
+    const int64_t word = (i >> 6) * kTapWords + lane;
     out[word] = *reinterpret_cast<const uint4*>(&hv);
     out[word + 64] = *reinterpret_cast<const uint4*>(&lv);
   }
 }
 
-}  // namespace
-
 // Compute units of the current device, rounded down to a multiple of the 8 XCDs (the
 // persistent kernel's grid: one workgroup a CU).
-static int device_cus() {
+int device_cus() {
   static int cached[64] = {0};
   int dev = 0;
   hip_check(hipGetDevice(&dev), "hipGetDevice");
@@ -977,12 +672,30 @@ static int device_cus() {
   return cached[dev];
 }
 
-// NNX_WINO_PERSISTENT=0 keeps every Winograd layer on the one-box-a-workgroup kernel (read
-// at each launch, for comparisons).
-static bool wino_persistent_enabled() {
-  const char* e = std::getenv("NNX_WINO_PERSISTENT");
-  return !(e && e[0] == '0');
+// The box of a layer: its z planes and tile grid, and the boxes per axis of an item.
+struct WinoPlan {
+  int zb;
+  bool tall;
+  int nbz, nby, nbx;
+};
+
+WinoPlan wino_plan(const ConvGeom& g, int cout) {
+  WinoPlan p{};
+  const int64_t wide = ceil_div(g.out[1], 8) * ceil_div(g.out[2], 16);
+  const int64_t tall = ceil_div(g.out[1], 16) * ceil_div(g.out[2], 8);
+  p.tall = tall < wide;
+  p.nby = (int)ceil_div(g.out[1], p.tall ? 16 : 8);
+  p.nbx = (int)ceil_div(g.out[2], p.tall ? 8 : 16);
+  const int64_t columns = (int64_t)g.batch * p.nby * p.nbx * ceil_div(cout, 32);
+  const int64_t cus = device_cus();
+  const int64_t rounds4 = ceil_div(columns * ceil_div(g.out[0], 4), cus);
+  const int64_t rounds2 = ceil_div(columns * ceil_div(g.out[0], 2), cus);
+  p.zb = 10 * rounds4 <= 6 * rounds2 ? 4 : 2;
+  p.nbz = (int)ceil_div(g.out[0], p.zb);
+  return p;
 }
+
+}  // namespace
 
 // Layers outside this set take the direct split kernel (the route is chosen with it).
 bool conv_wino_supported(const ConvGeom& g, int c1, int c2, int cout) {
@@ -992,13 +705,15 @@ bool conv_wino_supported(const ConvGeom& g, int c1, int c2, int cout) {
          c1 + c2 <= kMaxChannels;
 }
 
-int conv_wino_stats_tiles(const ConvGeom& g) {
-  return (int)(ceil_div(g.out[0], 4) * ceil_div(g.out[1], 8) * ceil_div(g.out[2], 8));
+int conv_wino_stats_tiles(const ConvGeom& g, int cout) {
+  const WinoPlan p = wino_plan(g, cout);
+  return p.nbz * p.nby * p.nbx;
 }
 
 float wino_weight_scale(float max_abs) {
-  // |U| <= (1.5)^3 max |w|: the scale keeps every split high half below 2^15 (the bound in
-  // float32, or in float64 where the float32 product would overflow)
+  // |U| <= (1.5)^2 max |w|: the scale keeps every split high half below 2^15, with the room of
+  // a third factor 1.5 (the bound in float32, or in float64 where the float32 product would
+  // overflow)
   require(std::isfinite(max_abs) && max_abs >= 0.f, "weight magnitude must be finite");
   const float bound = 3.375f * max_abs;
   return split_weight_scale(std::isfinite(bound) ? (double)bound : 3.375 * (double)max_abs);
@@ -1006,7 +721,7 @@ float wino_weight_scale(float max_abs) {
 
 int64_t conv_wino_packed_bytes(int cout, int c1, int c2) {
   const int64_t chunks = ceil_div(c1, kWChunk) + ceil_div(c2, kWChunk);
-  return ceil_div(cout, 32) * chunks * 64 * 2 * 64 * 16;
+  return ceil_div(cout, 32) * chunks * kPositions * 3 * kTapWords * 16;
 }
 
 void conv_wino_pack_weight(const float* d_w, int cout, int c1, int c2, float scale,
@@ -1017,7 +732,7 @@ void conv_wino_pack_weight(const float* d_w, int cout, int c1, int c2, float sca
   const int chunks0 = (int)ceil_div(c1, kWChunk);
   const int chunks = chunks0 + (int)ceil_div(c2, kWChunk);
   const int ntn = (int)ceil_div(cout, 32);
-  const int64_t total = (int64_t)ntn * chunks * 64 * 64;
+  const int64_t total = (int64_t)ntn * chunks * kPositions * 3 * 64;
   const int blocks = (int)std::min<int64_t>(ceil_div(total, 256), 65536);
   hipLaunchKernelGGL(pack_wino_weight_kernel, dim3(blocks), dim3(256), 0, st, d_w,
                      reinterpret_cast<uint4*>(d_packed), cout, c1, c2, chunks0, chunks, ntn,
@@ -1053,13 +768,14 @@ void conv3d_wino(const float* x1, int c1, const float* x2, int c2, const void* p
   a.H = g.in[1];
   a.W = g.in[2];
   a.cout = cout;
-  a.ntn = cout / 32;
-  a.nbz = (int)ceil_div(g.out[0], 4);
-  a.nby = (int)ceil_div(g.out[1], 8);
-  a.nbx = (int)ceil_div(g.out[2], 8);
-  const int64_t nwg = (int64_t)g.batch * a.nbz * a.nby * a.nbx * a.ntn;
+  const WinoPlan p = wino_plan(g, cout);
+  a.nbz = p.nbz;
+  a.nby = p.nby;
+  a.nbx = p.nbx;
+  const int64_t nwg = (int64_t)g.batch * a.nbz * a.nby * a.nbx * (cout / 32);
   require(nwg < (1LL << 31), "convolution grid too large");
-  a.nwg = (int)nwg;
+  a.nvirt = (int)nwg;
+  a.nbox = a.nvirt / (cout / 32);
   a.out_scale = 1.0f / scale;
   a.stats = stats;
   a.nrm0 = n1.params;
@@ -1072,14 +788,15 @@ void conv3d_wino(const float* x1, int c1, const float* x2, int c2, const void* p
   const double bytes = 4.0 * ((double)g.batch * g.in[0] * g.in[1] * g.in[2] * (c1 + c2) +
                               out_vox * cout);
   ProfScope prof("conv3d_wino", flops, bytes, st);
-  const int cus = device_cus();
-  if (a.chunks % 2 == 0 && wino_persistent_enabled() && a.nwg >= 4 * cus) {
-    a.nbox = a.nwg / a.ntn;
-    a.nvirt = a.nwg;
-    hipLaunchKernelGGL(wino_x3p_kernel, dim3(cus), dim3(kWThreads), 0, st, a);
-  } else {
-    hipLaunchKernelGGL(wino_x3_kernel, dim3(a.nwg), dim3(kWThreads), 0, st, a);
-  }
+  const dim3 grid((unsigned)std::min<int64_t>(device_cus(), ceil_div(nwg, 8) * 8)), block(kWThreads);
+  if (p.zb == 4 && !p.tall)
+    hipLaunchKernelGGL((wino_yx_kernel<4, false>), grid, block, 0, st, a);
+  else if (p.zb == 4)
+    hipLaunchKernelGGL((wino_yx_kernel<4, true>), grid, block, 0, st, a);
+  else if (!p.tall)
+    hipLaunchKernelGGL((wino_yx_kernel<2, false>), grid, block, 0, st, a);
+  else
+    hipLaunchKernelGGL((wino_yx_kernel<2, true>), grid, block, 0, st, a);
   launch_check("conv3d_winograd");
 }
 

@@ -356,7 +356,7 @@ def name_nonfinite_layer(error: ContractError, rerun) -> None:
             raise
         raise ContractError(
             f"non-finite logits: {located}.  The split-fp16 precisions take layer inputs below "
-            "65504 in magnitude (8188 at Winograd layers, whose input transform sums 8 of "
+            "65504 in magnitude (16376 at Winograd layers, whose input transform sums 4 of "
             "them); build this network with precision='fp32'") from error
     finally:
         lib.nnx_set_layer_checks(0)

@@ -187,6 +187,18 @@ def test_conv3d_winograd_random_shapes_match_float64(lib, case):
     _check_winograd_conv(lib, case)
 
 
+@pytest.mark.parametrize("case", [
+    (8, (18, 23, 31), 16, 16, 32),   # 4 x 8 x 16 boxes, every axis with a remainder
+    (8, (18, 33, 24), 32, 0, 64),    # 4 x 16 x 8 boxes
+    (1, (3, 8, 17), 32, 0, 32),      # 2 x 8 x 16 boxes
+    (1, (3, 17, 7), 16, 32, 32),     # 2 x 16 x 8 boxes, an odd chunk count
+], ids=lambda c: f"b{c[0]}-{c[1]}-c{c[2]}+{c[3]}-o{c[4]}")
+def test_conv3d_winograd_box_shapes_match_float64(lib, case):
+    """Each box shape of the Winograd kernel (the choice follows the volume and the number of
+    boxes) with remainders, at the same bar."""
+    _check_winograd_conv(lib, case)
+
+
 def _check_winograd_conv(lib, case):
     batch, size, c1, c2, cout = case
     print(f"winograd conv case {case}", flush=True)
