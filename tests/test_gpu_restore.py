@@ -153,3 +153,39 @@ def test_restore_class_labels_device_policy(device):
     order_z1 = ResamplingContract("resample_data_or_seg_to_shape", 1, 1, None)
     assert restore_class_labels_device(dev, (25, 20, 20), (2.5, 0.8, 0.8), (1.0, 0.64, 0.64),
                                        order_z1) is None
+
+
+@pytest.mark.parametrize("source,target,axis", [
+    ((9, 13, 70), (14, 9, 65), 0), ((9, 13, 70), (14, 9, 65), 1), ((9, 13, 70), (14, 9, 65), 2),
+    ((9, 13, 70), (14, 9, 65), -1), ((1, 1, 1), (3, 2, 5), 0), ((7, 5, 64), (2, 5, 129), 1),
+], ids=str)
+@pytest.mark.parametrize("special", [False, True], ids=["finite", "special"])
+def test_linear_restore_equals_the_resampler_by_class(device, source, target, axis, special):
+    """The one-pass order-1 restoration gives the labels of the spline resampler run class by
+    class and an argmax, bit for bit: every separate axis and none, up and down, rows around
+    the 64-voxel blocks; with infinities and NaN (which the resampler's clip replaces by the
+    plane's minimum) planted in two classes."""
+    from nnunet_mlx import _native
+    from nnunet_mlx.prediction.restore import resample_class_logits_argmax_spline_device
+    from tests.test_gpu_preprocess import spline_device
+
+    print(f"linear restore {source} -> {target} axis {axis} special {special}", flush=True)
+    rng = np.random.default_rng(5 + axis + sum(source))
+    logits = (rng.standard_normal((*source, 4)) * 3).astype(np.float32)
+    if special:
+        flat = logits.reshape(-1, 4)
+        for value in (np.nan, np.inf, -np.inf):
+            at = rng.integers(0, flat.shape[0], 3)
+            flat[at, 1] = value
+            flat[at[:1], 3] = value
+    values = spline_device(_native.load(), np.ascontiguousarray(np.moveaxis(logits, -1, 0)), target,
+                           1, axis)
+    got = resample_class_logits_argmax_spline_device(
+        torch.from_numpy(logits).to(device), target, order=1,
+        separate_axis=None if axis < 0 else axis)
+    # strict ">" from class 0 on, as the running argmax compares
+    best, want = values[0], np.zeros(target, np.uint16)
+    for c in range(1, 4):
+        higher = values[c] > best
+        best, want = np.where(higher, values[c], best), np.where(higher, c, want).astype(np.uint16)
+    np.testing.assert_array_equal(got.cpu().numpy().view(np.uint16), want)
