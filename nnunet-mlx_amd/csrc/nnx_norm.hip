@@ -466,9 +466,22 @@ __global__ __launch_bounds__(256) void nonfinite_kernel(const float* __restrict_
   if (threadIdx.x == 0) total = 0;
   __syncthreads();
   unsigned int local = 0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    local += isfinite(x[i]) ? 0u : 1u;
+  const int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  const int64_t threads = (int64_t)gridDim.x * blockDim.x;
+  // four 16-byte loads in flight where the tensor is aligned
+  const int64_t nvec = (reinterpret_cast<uintptr_t>(x) & 15) == 0 ? n / 4 : 0;
+  const float4* xv = reinterpret_cast<const float4*>(x);
+  auto bad = [](float4 v) {
+    return (isfinite(v.x) ? 0u : 1u) + (isfinite(v.y) ? 0u : 1u) + (isfinite(v.z) ? 0u : 1u) +
+           (isfinite(v.w) ? 0u : 1u);
+  };
+  int64_t i = tid;
+  for (; i + 3 * threads < nvec; i += 4 * threads) {
+    const float4 a = xv[i], b = xv[i + threads], c = xv[i + 2 * threads], d = xv[i + 3 * threads];
+    local += bad(a) + bad(b) + bad(c) + bad(d);
+  }
+  for (; i < nvec; i += threads) local += bad(xv[i]);
+  for (i = nvec * 4 + tid; i < n; i += threads) local += isfinite(x[i]) ? 0u : 1u;
   if (local) atomicAdd(&total, local);
   __syncthreads();
   if (threadIdx.x == 0 && total) atomicAdd(count, total);

@@ -112,7 +112,7 @@ __global__ __launch_bounds__(256) void restore_argmax_kernel(const void* __restr
 //
 // Roofline: HBM — the logits of the source planes that the nearest indices pick, once, and 2 B a
 // voxel.  300 x 534 x 534 x 3 float16 -> 120 x 512 x 512: 4.90 ms as 30 launches
-// through float64 volumes, 0.30 ms in one pass (0.27 GB of it needed: 0.9 TB/s).
+// through float64 volumes, 0.25 ms in one pass (0.27 GB of it needed: 1.1 TB/s).
 constexpr int kSplinePad = 12;
 
 struct LinTap {
@@ -309,7 +309,10 @@ void launch_linear(LinArgs a, int planes, float* minima, int64_t minima_room, hi
     a.minima = minima;
     hipLaunchKernelGGL(restore_minima_kernel<HALF>, dim3((unsigned)planes), dim3(1024), 0, st, a,
                        SEP, minima);
-    hipLaunchKernelGGL((restore_linear_kernel<HALF, SEP, true>), grid, dim3(256), 0, st, a);
+    // a small grid (it loops): nearly always every workgroup returns at once, and the full
+    // grid took 52 us to do so
+    hipLaunchKernelGGL((restore_linear_kernel<HALF, SEP, true>),
+                       dim3(grid.x, std::min(grid.y, 16u), std::min(grid.z, 16u)), dim3(256), 0, st, a);
   }
 }
 

@@ -152,6 +152,38 @@ def test_resample_spline_separate_axis(lib, axis):
     assert_one_rounding(got, want)
 
 
+@pytest.mark.parametrize("shape,new_shape,axis", [
+    ((1, 32, 63, 6), (40, 400, 7), -1),      # segments of 32 and 64 outputs and their remainders
+    ((1, 2, 31, 555), (3, 30, 600), -1),     # the last value of a row tile
+    ((1, 2, 4, 557), (2, 4, 1300), 0),       # one past a row tile, many outputs a sample
+    ((1, 3, 5, 1240), (7, 4, 300), 0),       # three row tiles, downsampled
+    ((1, 1, 1, 1), (3, 1, 5), -1),           # one sample a line
+    ((1, 130, 5, 4), (31, 9, 3), 1),         # separate middle axis
+], ids=str)
+def test_resample_spline_pieces(lib, shape, new_shape, axis):
+    """Order 3 at the edges of the pieces that a line is cut into."""
+    print(f"spline pieces {shape} -> {new_shape} axis {axis}", flush=True)
+    data = (np.random.default_rng(shape[3]).standard_normal(shape) * 3).astype(np.float32)
+    got = spline_device(lib, data, new_shape, 3, axis)
+    want = op.resample_data(data, new_shape, order=3, separate_axis=None if axis < 0 else axis)
+    assert_one_rounding(got, want)
+
+
+def test_crop_normalize_long_rows(lib):
+    """Rows past one round of eight loads a lane, in each order of the axes."""
+    raw = (np.random.default_rng(2).standard_normal((1, 3, 2, 1030)) * 9).astype(np.float32)
+    for transpose in itertools.permutations(range(3)):
+        out_size = tuple(raw.shape[1 + a] for a in transpose)
+        out = torch.full((1, *out_size), float("nan"), device="cuda")
+        norm = np.zeros((1, 4), dtype=np.float32)
+        _native.check(lib.nnx_crop_normalize(
+            dev(raw).data_ptr(), 1, _native.i64s(raw.shape[1:]), _native.ints(transpose),
+            _native.i64s((0, 0, 0)), _native.i64s(out_size), _native.ints([_native.NNX_NORM_NONE]),
+            norm.ctypes.data_as(ctypes.POINTER(ctypes.c_float)), out.data_ptr(), stream()))
+        np.testing.assert_array_equal(out.cpu().numpy(),
+                                      raw.transpose((0, *(a + 1 for a in transpose))))
+
+
 def ct_plan(spacing, transpose=(0, 1, 2), resampling=None):
     plans = {
         "transpose_forward": list(transpose),
