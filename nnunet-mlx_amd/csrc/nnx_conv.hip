@@ -2537,6 +2537,8 @@ void conv_x3_pack_weight(const float* d_w, int cout, const int* ksize, int c1, i
                      reinterpret_cast<uint4*>(d_packed), cout, taps, c1, c2, chunks1, chunks,
                      groups, nblk, scale, arith);
   launch_check("conv3d_x3_pack_weight");
+  if (arith == kBf16 && conv_bf16_direct_packed(ksize, c1, c2, cout))
+    conv_bf16_direct_pack(d_w, cout, c1, c2, scale, d_packed, st);
 }
 
 namespace {
@@ -2602,7 +2604,9 @@ bool conv_x3_supported(const int* ksize, const int* stride, int cout) {
   }
 }
 
-int conv_x3_stats_tiles(const ConvGeom& g, int cout) {
+int conv_x3_stats_tiles(const ConvGeom& g, int cout, int c1, int c2, int arith) {
+  if (arith == kBf16 && conv_bf16_direct_supported(g, c1, c2, cout))
+    return conv_bf16_direct_stats_tiles(g);
   const Box box = plan_x3(g, cout).box;
   return (int)(ceil_div(g.out[0], box.z) * ceil_div(g.out[1], box.y) * ceil_div(g.out[2], box.x));
 }
@@ -2615,6 +2619,14 @@ void conv3d_x3(const float* x1, int c1, const float* x2, int c2, const void* pac
   require(c1 >= 1 && (c2 == 0 || x2), "invalid convolution inputs");
   require(scale > 0.f && std::isfinite(scale), "weight scale must be positive");
   require(arith == kSplit3 || arith == kBf16, "unknown convolution arithmetic");
+  // (its 16-byte lines need aligned tensors, as every activation of a model is)
+  const uintptr_t ends = reinterpret_cast<uintptr_t>(x1) | reinterpret_cast<uintptr_t>(x2) |
+                         reinterpret_cast<uintptr_t>(y);
+  if (arith == kBf16 && ends % 16 == 0 && conv_bf16_direct_supported(g, c1, c2, cout)) {
+    conv3d_bf16_direct(x1, c1, x2, c2, packed, scale, bias, y, g, cout, st, stats, n1, n2);
+    return;
+  }
+  require(!stats || ends % 16 == 0, "activations must be 16-byte aligned");
   const X3Plan plan = plan_x3(g, cout);
   const Variant v = plan.v;
   IgemmArgs a = igemm_args(x1, c1, x2, c2, bias, y, g, cout, v, plan.box, stats, n1, n2);

@@ -148,7 +148,23 @@ void conv3d_x3(const float* x1, int c1, const float* x2, int c2, const void* pac
                float scale, const float* bias, float* y, const ConvGeom& g, int cout,
                hipStream_t st, float4* stats = nullptr, const PendingNorm& n1 = {},
                const PendingNorm& n2 = {}, int arith = kArithSplit3);
-int conv_x3_stats_tiles(const ConvGeom& g, int cout);
+int conv_x3_stats_tiles(const ConvGeom& g, int cout, int c1, int c2, int arith);
+
+// Compute units of the current device, a multiple of the 8 XCDs (the persistent kernels' grid).
+int compute_units();
+// Direct bf16 convolution of the stride-1 3x3x3 layers with 16-channel input blocks and C_out % 32
+// == 0 (nnx_bf16.hip), a route of conv3d_x3's bf16 arithmetic: its words take the low-half planes
+// that bf16 packing leaves unused, written by conv_x3_pack_weight where the layer's channels
+// allow it (the stride is not known there).
+bool conv_bf16_direct_packed(const int* ksize, int c1, int c2, int cout);
+bool conv_bf16_direct_supported(const ConvGeom& g, int c1, int c2, int cout);
+void conv_bf16_direct_pack(const float* d_w, int cout, int c1, int c2, float scale, void* d_packed,
+                           hipStream_t st);
+int conv_bf16_direct_stats_tiles(const ConvGeom& g);
+void conv3d_bf16_direct(const float* x1, int c1, const float* x2, int c2, const void* packed,
+                        float scale, const float* bias, float* y, const ConvGeom& g, int cout,
+                        hipStream_t st, float4* stats, const PendingNorm& n1,
+                        const PendingNorm& n2);
 
 // Winograd F(2x2, 3x3) in (y, x) with the three z taps direct, split-fp16 products
 // (nnx_wino.hip): stride-1 3x3x3 layers with C_out % 32 == 0 and input channel counts that are

@@ -531,7 +531,7 @@ struct Runner {
     // tensor for them.
     const ConvGeom g = make_conv_geom(n, in.d, c.k, c.s);
     const int tiles = c.wino    ? conv_wino_stats_tiles(g, c.cout)
-                      : c.split ? conv_x3_stats_tiles(g, c.cout)
+                      : c.split ? conv_x3_stats_tiles(g, c.cout, c.cin1, c.cin2, c.arith)
                                 : conv_stats_tiles(g, c.cout, c.cin1, c.cin2);
     if (plan->planning) {
       plan->stats = std::max(plan->stats, (size_t)n * tiles * c.cout * sizeof(float4));

@@ -656,22 +656,6 @@ __global__ void pack_wino_weight_kernel(const float* __restrict__ w, uint4* __re
   }
 }
 
-// Compute units of the current device, rounded down to a multiple of the 8 XCDs (the
-// persistent kernel's grid: one workgroup a CU).
-int device_cus() {
-  static int cached[64] = {0};
-  int dev = 0;
-  hip_check(hipGetDevice(&dev), "hipGetDevice");
-  if (dev < 0 || dev >= 64) dev = 0;
-  if (cached[dev] == 0) {
-    int n = 0;
-    hip_check(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev),
-              "hipDeviceGetAttribute");
-    cached[dev] = n >= 8 ? n / 8 * 8 : 8;
-  }
-  return cached[dev];
-}
-
 // The box of a layer: its z planes and tile grid, and the boxes per axis of an item.
 struct WinoPlan {
   int zb;
@@ -687,7 +671,7 @@ WinoPlan wino_plan(const ConvGeom& g, int cout) {
   p.nby = (int)ceil_div(g.out[1], p.tall ? 16 : 8);
   p.nbx = (int)ceil_div(g.out[2], p.tall ? 8 : 16);
   const int64_t columns = (int64_t)g.batch * p.nby * p.nbx * ceil_div(cout, 32);
-  const int64_t cus = device_cus();
+  const int64_t cus = compute_units();
   const int64_t rounds4 = ceil_div(columns * ceil_div(g.out[0], 4), cus);
   const int64_t rounds2 = ceil_div(columns * ceil_div(g.out[0], 2), cus);
   p.zb = 10 * rounds4 <= 6 * rounds2 ? 4 : 2;
@@ -696,6 +680,22 @@ WinoPlan wino_plan(const ConvGeom& g, int cout) {
 }
 
 }  // namespace
+
+// Compute units of the current device, rounded down to a multiple of the 8 XCDs (the
+// persistent kernel's grid: one workgroup a CU).
+int compute_units() {
+  static int cached[64] = {0};
+  int dev = 0;
+  hip_check(hipGetDevice(&dev), "hipGetDevice");
+  if (dev < 0 || dev >= 64) dev = 0;
+  if (cached[dev] == 0) {
+    int n = 0;
+    hip_check(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev),
+              "hipDeviceGetAttribute");
+    cached[dev] = n >= 8 ? n / 8 * 8 : 8;
+  }
+  return cached[dev];
+}
 
 // Layers outside this set take the direct split kernel (the route is chosen with it).
 bool conv_wino_supported(const ConvGeom& g, int c1, int c2, int cout) {
@@ -788,7 +788,7 @@ void conv3d_wino(const float* x1, int c1, const float* x2, int c2, const void* p
   const double bytes = 4.0 * ((double)g.batch * g.in[0] * g.in[1] * g.in[2] * (c1 + c2) +
                               out_vox * cout);
   ProfScope prof("conv3d_wino", flops, bytes, st);
-  const dim3 grid((unsigned)std::min<int64_t>(device_cus(), ceil_div(nwg, 8) * 8)), block(kWThreads);
+  const dim3 grid((unsigned)std::min<int64_t>(compute_units(), ceil_div(nwg, 8) * 8)), block(kWThreads);
   if (p.zb == 4 && !p.tall)
     hipLaunchKernelGGL((wino_yx_kernel<4, false>), grid, block, 0, st, a);
   else if (p.zb == 4)

@@ -561,7 +561,17 @@ def _bf16(a: np.ndarray) -> np.ndarray:
     return torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).to(torch.bfloat16).double().numpy()
 
 
-@pytest.mark.parametrize("case", CONV_CASES, ids=lambda c: f"b{c[0]}-{c[1]}-c{c[2]}+{c[3]}-o{c[4]}-k{c[5]}-s{c[6]}")
+# the direct bf16 kernel (3x3x3, stride 1, 16-channel blocks): boxes of 4 x 8 x 16
+BF16_DIRECT_CASES = [
+    (1, (5, 9, 17), 48, 0, 64, (3, 3, 3), (1, 1, 1)),    # one past a box on every axis
+    (2, (4, 8, 16), 32, 32, 96, (3, 3, 3), (1, 1, 1)),   # two inputs, half a column group
+    (3, (9, 13, 30), 64, 0, 32, (3, 3, 3), (1, 1, 1)),   # one column block, two planes a wave
+    (1, (1, 1, 1), 64, 16, 160, (3, 3, 3), (1, 1, 1)),
+    (16, (17, 20, 33), 16, 0, 64, (3, 3, 3), (1, 1, 1)),  # one chunk, boxes in turn across items
+]
+
+
+@pytest.mark.parametrize("case", CONV_CASES + BF16_DIRECT_CASES, ids=lambda c: f"b{c[0]}-{c[1]}-c{c[2]}+{c[3]}-o{c[4]}-k{c[5]}-s{c[6]}")
 def test_conv3d_bf16_matches_rounded_float64(lib, case):
     """bf16 arithmetic: the float64 convolution of the bf16-rounded input and weights (each
     product is exact in float32) to float32 accumulation error, and the bf16 bar
