@@ -229,7 +229,6 @@ __global__ __launch_bounds__(kBThreads, 1) void conv_bf16_kernel(Bf16Args a) {
     const int tid = threadIdx.x;
     const Bf16Box first = bf16_box(a, v);
     box_lines(tid, first, yx);
-    load_prm(tid, first.b);
     const Source src = source(first, 0);
     f4 hl[kLines];
 #pragma unroll
@@ -237,6 +236,7 @@ __global__ __launch_bounds__(kBThreads, 1) void conv_bf16_kernel(Bf16Args a) {
     const uint4* up = uaddr(tid & 63, first.ng, 0);
 #pragma unroll
     for (int s = 0; s < kRing; ++s) load_u(up, s);
+    load_prm(tid, first.b);
     lds_barrier();  // the parameters
     convert(hl, yx, src.z0, 0, 0);
     lds_barrier();

@@ -17,7 +17,8 @@
 // float32, each then split into fp16 halves.  V adds up to 4 inputs.
 //
 // Workgroup: 8 waves (two a SIMD), an output box of ZB z planes x 32 tiles (4 x 8 tiles =
-// 8 x 16 voxels, or 8 x 4 tiles where that wastes less) and 32 output channels.  Wave
+// 8 x 16 voxels; 8 x 4 tiles, or 4 x 4 in two slabs of planes, where that wastes less) and 32
+// output channels.  Wave
 // w = 2 xy + h owns the positions (xy, xx = 0, 1) for h = 0 and (xy, xx = 3, 2) for h = 1: its
 // accumulators are 2 x ZB blocks of 32 x 32 floats (128 registers a lane at ZB = 4), which
 // leaves room for a second wave on the SIMD to issue while one waits.  Per chunk of 16 input
@@ -76,23 +77,34 @@ constexpr int kTapWords = 128;    // packed words of one (position, z tap): hi, 
 constexpr int kPartSlots = 8 * 2 * 32 * 8;  // epilogue partials: wave, ox, tile, 4 columns
 constexpr int kRedSlots = 2 * 8 * 8;        // InstanceNorm partials: pass, wave, 4 columns
 
-// Box geometry.  A raw halo plane is stored as [y / 2][y % 2][x / 2][x % 2 ...] (tile rows and
+// Box shapes: tiles of a z plane side by side (wide, tall), or two slabs of ZB planes with 4 x 4
+// tiles each (cube), the MFMA rows 16-31 taking the upper slab.
+enum WinoShape { kWide, kTall, kCube };
+
+// Box geometry.  A raw halo plane is stored as [y / 2][y % 2][x % 2][x / 2] (tile rows and
 // columns are every second row and column) with q = channel quad fastest: slot = yi * py +
 // jump * (yi / 4) + yp * pyp + xp * pxp + xi * 4 + q.  For a fixed (row, column, quad) of the
 // patch the 32 tiles then fall on 32 different slots modulo 32 (ds_read_b128 serves 32 lanes
-// a pass from 32 16-byte groups).
-template <int ZB, bool TALL>
+// a pass from 32 16-byte groups); the cube's plane stride puts its two slabs 16 slots apart.
+template <int ZB, WinoShape S>
 struct WinoBoxGeom {
-  static constexpr int ty = TALL ? 8 : 4, tx = TALL ? 4 : 8;  // tiles
-  static constexpr int by = 2 * ty, bx = 2 * tx;              // output voxels
-  static constexpr int hz = ZB + 2, hy = by + 2, hx = bx + 2;  // halo
+  static constexpr int slabs = S == kCube ? 2 : 1;
+  static constexpr int ty = S == kTall ? 8 : 4, tx = S == kWide ? 8 : 4;  // tiles
+  static constexpr int by = 2 * ty, bx = 2 * tx, bz = ZB * slabs;  // output voxels
+  static constexpr int hz = bz + 2, hy = by + 2, hx = bx + 2;       // halo
   static constexpr int pxp = (tx + 1) * 4, pyp = 2 * pxp, py = 2 * pyp + 1;
-  static constexpr int jump = TALL ? 12 : 0;
-  static constexpr int slots = hz * kPlane;
+  static constexpr int jump = S == kTall ? 12 : 0;
+  static constexpr int plane = S == kCube ? 408 : kPlane;
+  static constexpr int rounds = (hz * plane + kWThreads - 1) / kWThreads;
+  // in-plane patterns of a thread's rounds: three for plane pairs of 1.5 rounds each, else one
+  // voxel a round
+  static constexpr int lines = S == kCube ? rounds : 3;
+  static constexpr int slots = rounds * kWThreads;
   // the epilogue's partials and reductions use one raw buffer
   static constexpr int buf = slots > kPartSlots + kRedSlots ? slots : kPartSlots + kRedSlots;
-  static_assert(py * ty + jump * (ty / 4) + 2 * pyp <= kPlane, "a halo plane fits its slots");
-  static_assert(hz % 2 == 0, "plane pairs are three rounds of the workgroup");
+  static_assert(py * ty + jump * (ty / 4) + 2 * pyp <= plane, "a halo plane fits its slots");
+  static_assert(S == kCube || hz % 2 == 0, "plane pairs are three rounds of the workgroup");
+  static_assert(S != kCube || ZB * plane % 32 == 16, "the slabs' tiles interleave");
   static_assert(2 * buf * 16 + 3 * kMaxChannels * 4 + 128 <= 160 * 1024, "LDS");
 };
 
@@ -142,12 +154,12 @@ __device__ __forceinline__ void split8(const float (&v)[8], h8& hi, h8& lo) {
   }
 }
 
-// Six patch points (two rows x columns P, Q, R; 8 channels each, two 16-byte reads) of halo
-// plane Z at LDS byte addresses ad[row * 3 + column], with the wait for them.  Written as
+// Six patch points (two rows x columns P, Q, R; 8 channels each, two 16-byte reads) at LDS byte
+// addresses ad[row * 3 + column] + OFFSET, with the wait for them.  Written as
 // one asm block so that the compiler's wait-count pass does not see LDS reads here: it
 // would otherwise order them behind the halo DMA in flight to the other buffer (it cannot
 // tell the two apart) and wait for that DMA first.
-template <int Z>
+template <int OFFSET>
 __device__ __forceinline__ void read_patch(const unsigned (&ad)[6], f4 (&v)[12]) {
   asm volatile(
       "ds_read_b128 %0, %12 offset:%18\n\tds_read_b128 %1, %12 offset:%19\n\t"
@@ -160,7 +172,7 @@ __device__ __forceinline__ void read_patch(const unsigned (&ad)[6], f4 (&v)[12])
       : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]),
         "=&v"(v[6]), "=&v"(v[7]), "=&v"(v[8]), "=&v"(v[9]), "=&v"(v[10]), "=&v"(v[11])
       : "v"(ad[0]), "v"(ad[1]), "v"(ad[2]), "v"(ad[3]), "v"(ad[4]), "v"(ad[5]),
-        "n"(Z * kPlane * 16), "n"(Z * kPlane * 16 + 16)
+        "n"(OFFSET), "n"(OFFSET + 16)
       : "memory");
 }
 
@@ -205,9 +217,9 @@ __device__ __forceinline__ WinoBox wino_box(const WinoArgs& a, int v) {
   return r;
 }
 
-template <int ZB, bool TALL>
+template <int ZB, WinoShape S>
 __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
-  using G = WinoBoxGeom<ZB, TALL>;
+  using G = WinoBoxGeom<ZB, S>;
   __shared__ __align__(16) f4 s_raw[2 * G::buf];             // two raw halo buffers
   __shared__ __align__(16) float s_prm[3 * kMaxChannels];    // mean, scale, beta by channel
   __shared__ __align__(16) float s_bias[32];                 // of the current column block
@@ -222,63 +234,72 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
   if (v >= vend) return;  // uniform over the workgroup, before any barrier
   __builtin_assume(a.chunks > 0);
   const int64_t plane_vox = (int64_t)a.H * a.W;
-  constexpr int kRounds = G::hz / 2 * 3;
+  constexpr int kRounds = G::rounds, kL = G::lines;
   uint64_t zero = (uint64_t)g_wino_zero;
   asm volatile("" : "+s"(zero));  // held, not loaded from the GOT at every use
 
-  // ---- raw halo lines.  Round 3 k + j of this thread is slot j * 512 + tid of the plane pair
-  // 2 k, 2 k + 1: three in-plane patterns j, the plane uniform over a wave.
+  // ---- raw halo lines.  Wide and tall: round 3 k + j of this thread is slot j * 512 + tid of the
+  // plane pair 2 k, 2 k + 1: three in-plane patterns j, the plane uniform over a wave; `at` is
+  // their in-plane voxel.  Cube: round r is slot r * 512 + tid of all planes, `at` its voxel in
+  // the item.  -1 outside the volume or on a padding slot; `quads`: two bits a pattern.
   auto round_plane = [&](int k, int j) { return 2 * k + ((j == 2 || (j == 1 && wave >= 4)) ? 1 : 0); };
-  // in-plane voxel offset (-1 outside the volume or on a padding slot) and channel quad of
-  // the three patterns for a box corner
-  auto box_lines = [&](int tid, const WinoBox& bx, int (&yx)[3], int& quads)
+  auto box_lines = [&](int tid, const WinoBox& bx, int (&at)[kL], int& quads)
       __attribute__((always_inline)) {
     quads = 0;
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const int s = j == 0 ? tid : j == 1 ? (tid < 256 ? 512 + tid : tid - 256) : 256 + tid;
+    for (int j = 0; j < kL; ++j) {
+      int s, hz = 0;
+      if constexpr (S == kCube) {
+        hz = (j * kWThreads + tid) / G::plane;
+        s = j * kWThreads + tid - hz * G::plane;
+      } else {
+        s = j == 0 ? tid : j == 1 ? (tid < 256 ? 512 + tid : tid - 256) : 256 + tid;
+      }
       int t = s;
-      if constexpr (TALL) t = s < G::py * 4 + G::jump ? s : s < G::py * 8 + 2 * G::jump ? s - G::jump
-                                                                                       : s - 2 * G::jump;
+      if constexpr (S == kTall) t = s < G::py * 4 + G::jump ? s : s < G::py * 8 + 2 * G::jump ? s - G::jump
+                                                                                             : s - 2 * G::jump;
       const int yi = t / G::py, rem = t - yi * G::py;
       const int yp = rem / G::pyp, rx = rem - yp * G::pyp;
       const int xp = rx / G::pxp, rq = rx - xp * G::pxp;
       const int hy = 2 * yi + yp, hx = 2 * (rq >> 2) + xp;
       const int yy = bx.byi * G::by - 1 + hy, xx = bx.bxi * G::bx - 1 + hx;
-      const bool line = s - t == G::jump * (yi >> 2) && rem < 2 * G::pyp && hy < G::hy &&
-                        (unsigned)yy < (unsigned)a.H && (unsigned)xx < (unsigned)a.W;
-      yx[j] = line ? yy * a.W + xx : -1;
-      quads |= (rq & 3) << (8 * j);
+      const int zz = bx.bzi * G::bz - 1 + hz;
+      bool line = s - t == G::jump * (yi >> 2) && rem < 2 * G::pyp && hy < G::hy && hx < G::hx &&
+                  (unsigned)yy < (unsigned)a.H && (unsigned)xx < (unsigned)a.W;
+      if constexpr (S == kCube) line = line && hz < G::hz && (unsigned)zz < (unsigned)a.D;
+      at[j] = line ? (S == kCube ? zz * a.H + yy : yy) * a.W + xx : -1;
+      quads |= (rq & 3) << (2 * j);
     }
   };
-  // Rounds [r0, r1) of a chunk of a box's halo into buffer `buf` (live = false: the zero line),
-  // spread over the previous chunk's products.
+  // Rounds [r0, r1) of a chunk of a box's halo into buffer `buf`, spread over the previous chunk's
+  // products.
   struct Source {
-    uint64_t base;         // channel chunk of the halo's first plane (may lie outside the volume)
+    uint64_t base;         // channel chunk of the halo's first plane (may lie outside the volume;
+                           // cube: of the item)
     int64_t plane_bytes;
     int C, z0;
   };
-  auto source = [&](const WinoBox& bx, int chunk, bool live) __attribute__((always_inline)) {
+  auto source = [&](const WinoBox& bx, int chunk) __attribute__((always_inline)) {
     const bool first = chunk < a.chunks0;
     Source r;
     r.C = first ? a.c0 : a.c1;
     r.plane_bytes = plane_vox * r.C * 4;
-    const int z = bx.bzi * ZB - 1;
-    r.base = (uint64_t)(first ? a.x0 : a.x1) + ((int64_t)bx.b * a.D + z) * r.plane_bytes +
+    r.z0 = S == kCube ? 0 : bx.bzi * G::bz - 1;
+    r.base = (uint64_t)(first ? a.x0 : a.x1) + ((int64_t)bx.b * a.D + r.z0) * r.plane_bytes +
              (first ? chunk : chunk - a.chunks0) * kWChunk * 4;
-    r.z0 = live ? z : INT32_MIN / 2;
     return r;
   };
-  auto fetch = [&](const Source& src, const int (&yx)[3], int quads, int buf, auto r0c, auto r1c)
+  auto fetch = [&](const Source& src, const int (&at)[kL], int quads, int buf, auto r0c, auto r1c)
       __attribute__((always_inline)) {
     f4* dst = s_raw + buf * G::buf + wave * 64;
 #pragma unroll
     for (int r = decltype(r0c)::value; r < decltype(r1c)::value; ++r) {
-      const int k = r / 3, j = r % 3, p = round_plane(k, j);
+      const int k = S == kCube ? 0 : r / 3, j = S == kCube ? r : r % 3;
+      const int p = S == kCube ? 0 : round_plane(k, j);
       // a per-lane plane index keeps the check a select of two addresses instead of a branch
-      const int z = yx[j] >= 0 ? src.z0 + p : -1;
+      const int z = at[j] >= 0 ? src.z0 + p : -1;
       const uint64_t in = src.base + p * src.plane_bytes +
-                          ((int64_t)yx[j] * src.C + ((quads >> (8 * j)) & 3) * 4) * 4;
+                          ((int64_t)at[j] * src.C + ((quads >> (2 * j)) & 3) * 4) * 4;
       const uint64_t g = (unsigned)z < (unsigned)a.D ? in : zero;
       __builtin_amdgcn_global_load_lds(
           (const void*)g, (__attribute__((address_space(3))) void*)(dst + r * kWThreads), 16, 0, 0);
@@ -302,32 +323,35 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
   // pass's operations: t = fma(x - mean, scale, beta), then max(s * t, t) with s = the
   // LeakyReLU slope under the activation and s = 1, the identity, without it).  Lines outside
   // the volume stay zero.
-  auto normalise = [&](const WinoBox& bx, const int (&yx)[3], int quads, int chunk, int buf)
+  auto normalise = [&](const WinoBox& bx, const int (&at)[kL], int quads, int chunk, int buf)
       __attribute__((always_inline)) {
     const bool first = chunk < a.chunks0;
     if ((first ? a.nrm0 : a.nrm1) == nullptr) return;
     const float s = (first ? a.act0 : a.act1) != 0 ? a.slope : 1.f;
     f4* lines = s_raw + buf * G::buf + threadIdx.x;
+    constexpr int kPer = S == kCube ? 1 : G::hz / 2;  // rounds of a pattern
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      if (yx[j] < 0) continue;
-      const float* prm = s_prm + chunk * kWChunk + ((quads >> (8 * j)) & 3) * 4;
+    for (int j = 0; j < kL; ++j) {
+      if (at[j] < 0) continue;
+      const float* prm = s_prm + chunk * kWChunk + ((quads >> (2 * j)) & 3) * 4;
       const f4 mean = *reinterpret_cast<const f4*>(prm);
       const f4 scale = *reinterpret_cast<const f4*>(prm + kMaxChannels);
       const f4 beta = *reinterpret_cast<const f4*>(prm + 2 * kMaxChannels);
-      f4 d[G::hz / 2];
+      f4 d[kPer];
 #pragma unroll
-      for (int k = 0; k < G::hz / 2; ++k) d[k] = lines[(3 * k + j) * kWThreads];
+      for (int k = 0; k < kPer; ++k) d[k] = lines[(kPer == 1 ? j : 3 * k + j) * kWThreads];
 #pragma unroll
-      for (int k = 0; k < G::hz / 2; ++k) {
-        const int z = bx.bzi * ZB - 1 + round_plane(k, j);
-        if ((unsigned)z >= (unsigned)a.D) continue;  // uniform over the wave
+      for (int k = 0; k < kPer; ++k) {
+        if constexpr (S != kCube) {
+          const int z = bx.bzi * G::bz - 1 + round_plane(k, j);
+          if ((unsigned)z >= (unsigned)a.D) continue;  // uniform over the wave
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float t = fmaf(d[k][e] - mean[e], scale[e], beta[e]);
           d[k][e] = fmaxf(s * t, t);
         }
-        lines[(3 * k + j) * kWThreads] = d[k];
+        lines[(kPer == 1 ? j : 3 * k + j) * kWThreads] = d[k];
       }
     }
   };
@@ -354,18 +378,18 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
   };
 
   // loop-carried: the lines of the box whose first chunk is in flight, its U, the raw buffer
-  int yx[3], quads, buf = 0;
+  int yx[kL], quads, buf = 0;
   {
     const int tid = threadIdx.x;
     const WinoBox first = wino_box(a, v);
     box_lines(tid, first, yx, quads);
-    load_prm(tid, first.b);
-    if (tid < 32) s_bias[tid] = a.bias ? a.bias[first.nt * 32 + tid] : 0.f;
-    fetch(source(first, 0, true), yx, quads, 0, std::integral_constant<int, 0>{},
+    fetch(source(first, 0), yx, quads, 0, std::integral_constant<int, 0>{},
           std::integral_constant<int, kRounds>{});
     const uint4* up = uaddr(tid & 63, first.nt, 0);
 #pragma unroll
     for (int kz = 0; kz < 3; ++kz) load_u(up, kz);
+    load_prm(tid, first.b);  // (behind the halo, whose latency theirs hides in)
+    if (tid < 32) s_bias[tid] = a.bias ? a.bias[first.nt * 32 + tid] : 0.f;
     lds_barrier();  // the parameters and the bias
   }
 
@@ -378,18 +402,19 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
     const WinoBox cur = wino_box(a, v);
     const int vnext = v + stride;
     const bool more = vnext < vend;
-    const int vn = more ? vnext : v;  // the next box (this one again after the last)
-    const WinoBox nxt = wino_box(a, vn);
+    const WinoBox nxt = more ? wino_box(a, vnext) : cur;
 
     // LDS byte addresses of this lane's six patch points in plane 0 of buffer 0
     unsigned ad[6];
     {
       const int t = lane & 31, g8 = lane >> 5;
-      const int tyl = TALL ? t >> 2 : t >> 3, txl = TALL ? t & 3 : t & 7;
+      const int tyl = S == kWide ? t >> 3 : S == kTall ? t >> 2 : (t >> 2) & 3;
+      const int txl = S == kWide ? t & 7 : t & 3;
+      const int slab = S == kCube ? (t >> 4) * ZB * G::plane : 0;
       const unsigned raw0 = (unsigned)(uintptr_t)((__attribute__((address_space(3))) f4*)s_raw);
       auto point = [&](int r, int c) {
         const int yi = tyl + (r >> 1);
-        return raw0 + 16u * (unsigned)(yi * G::py + G::jump * (yi >> 2) + (r & 1) * G::pyp +
+        return raw0 + 16u * (unsigned)(slab + yi * G::py + G::jump * (yi >> 2) + (r & 1) * G::pyp +
                                        (c & 1) * G::pxp + (txl + (c >> 1)) * 4 + 2 * g8);
       };
       ad[0] = point(ra, cp);
@@ -418,7 +443,7 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
     auto plane = [&](auto zc) __attribute__((always_inline)) {
       constexpr int Z = decltype(zc)::value;
       f4 d[12];
-      read_patch<Z>(ad, d);
+      read_patch<Z * G::plane * 16>(ad, d);
       float vp[8], vq8[8], vr8[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -455,18 +480,18 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
       normalise(cur, yx, quads, chunk, buf);
       lds_barrier();  // every thread's lines; the other buffer is free
       const bool last = chunk + 1 == a.chunks;
-      // the next chunk's halo; after the box's last chunk the next box's first (the zero line
-      // after the last box)
-      if (last) {
+      // the next chunk's halo; after the box's last chunk the next box's first, if there is one
+      if (last && more) {
         int tid_n = tid;
         asm volatile("" : "+v"(tid_n));  // computed here, not hoisted and held
         box_lines(tid_n, nxt, yx, quads);
       }
-      const Source src = source(last ? nxt : cur, last ? 0 : chunk + 1, !last || more);
+      const Source src = source(last ? nxt : cur, last ? 0 : chunk + 1);
       auto rounds = [&](auto ic) __attribute__((always_inline)) {
         constexpr int I = decltype(ic)::value;
-        fetch(src, yx, quads, buf ^ 1, std::integral_constant<int, I * kRounds / ZB>{},
-              std::integral_constant<int, (I + 1) * kRounds / ZB>{});
+        if (!last || more)
+          fetch(src, yx, quads, buf ^ 1, std::integral_constant<int, I * kRounds / ZB>{},
+                std::integral_constant<int, (I + 1) * kRounds / ZB>{});
       };
       const uint4* un = uaddr(lane, last ? nxt.nt : cur.nt, last ? 0 : chunk + 1);
       rounds(std::integral_constant<int, 0>{});
@@ -538,13 +563,13 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
       lds_barrier();
     }
     const int row = 8 * (rho >> 3) + 4 * (rho & 1) + ((rho >> 1) & 3);
-    const int yy = cur.byi * G::by + 2 * (TALL ? row >> 2 : row >> 3);
-    const int xx = cur.bxi * G::bx + 2 * (TALL ? row & 3 : row & 7) + ox;
-    const int z0 = cur.bzi * ZB;
+    const int yy = cur.byi * G::by + 2 * (S == kWide ? row >> 3 : S == kTall ? row >> 2 : (row >> 2) & 3);
+    const int xx = cur.bxi * G::bx + 2 * (S == kWide ? row & 7 : row & 3) + ox;
+    const int z0 = cur.bzi * G::bz + (S == kCube ? (row >> 4) * ZB : 0);
     const bool xin = xx < a.W;
     auto valid = [&](int z, int oy) { return xin && yy + oy < a.H && z0 + z < a.D; };
     if (a.stats) {
-      const int nz = min(ZB, a.D - z0), ny = min(G::by, a.H - cur.byi * G::by);
+      const int nz = min(G::bz, a.D - cur.bzi * G::bz), ny = min(G::by, a.H - cur.byi * G::by);
       const int nx = min(G::bx, a.W - cur.bxi * G::bx);
       const float cnt = (float)(nz * ny * nx);
       f4 sm = {0.f, 0.f, 0.f, 0.f};
@@ -595,8 +620,6 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
     if (!more) break;
     v = vnext;
   }
-  // the last (zero-line) DMA lands before the workgroup's LDS is released
-  __builtin_amdgcn_s_waitcnt(0);
 }
 
 // U[cout][cin][kz][xi] = sum_{b,e} G[xy][b] G[xx][e] w[cout][kz][b][e][cin] in float64, times
@@ -656,27 +679,36 @@ __global__ void pack_wino_weight_kernel(const float* __restrict__ w, uint4* __re
   }
 }
 
-// The box of a layer: its z planes and tile grid, and the boxes per axis of an item.
+// The box of a layer: its z planes and shape, and the boxes per axis of an item.
 struct WinoPlan {
   int zb;
-  bool tall;
+  WinoShape shape;
   int nbz, nby, nbx;
 };
 
+// The shape that needs the least time by rounds of boxes over the CUs: a box of four planes
+// takes 1 of it, one of two planes 0.6 (320 -> 320: 4.8 and 2.9 us a 16-channel chunk), so the
+// small boxes win where they fill CUs that would stand idle: 320 -> 320 on 8^3 x 8 95.6 us in
+// boxes of 4 x 8 x 16 (half of each outside the volume), 63.9 us in boxes of 4 x 8 x 8 (the three-axis
+// form: 67 to 69).
 WinoPlan wino_plan(const ConvGeom& g, int cout) {
-  WinoPlan p{};
-  const int64_t wide = ceil_div(g.out[1], 8) * ceil_div(g.out[2], 16);
-  const int64_t tall = ceil_div(g.out[1], 16) * ceil_div(g.out[2], 8);
-  p.tall = tall < wide;
-  p.nby = (int)ceil_div(g.out[1], p.tall ? 16 : 8);
-  p.nbx = (int)ceil_div(g.out[2], p.tall ? 8 : 16);
-  const int64_t columns = (int64_t)g.batch * p.nby * p.nbx * ceil_div(cout, 32);
   const int64_t cus = compute_units();
-  const int64_t rounds4 = ceil_div(columns * ceil_div(g.out[0], 4), cus);
-  const int64_t rounds2 = ceil_div(columns * ceil_div(g.out[0], 2), cus);
-  p.zb = 10 * rounds4 <= 6 * rounds2 ? 4 : 2;
-  p.nbz = (int)ceil_div(g.out[0], p.zb);
-  return p;
+  const int64_t columns = (int64_t)g.batch * ceil_div(cout, 32);
+  WinoPlan best{};
+  int64_t best_cost = -1;
+  auto consider = [&](int zb, WinoShape shape, int bz, int by, int bx, int64_t cost) {
+    const int64_t nbz = ceil_div(g.out[0], bz), nby = ceil_div(g.out[1], by), nbx = ceil_div(g.out[2], bx);
+    const int64_t total = ceil_div(columns * nbz * nby * nbx, cus) * cost;
+    if (best_cost >= 0 && total >= best_cost) return;
+    best_cost = total;
+    best = WinoPlan{zb, shape, (int)nbz, (int)nby, (int)nbx};
+  };
+  consider(4, kWide, 4, 8, 16, 10);
+  consider(4, kTall, 4, 16, 8, 10);
+  consider(2, kWide, 2, 8, 16, 6);
+  consider(2, kTall, 2, 16, 8, 6);
+  consider(2, kCube, 4, 8, 8, 6);
+  return best;
 }
 
 }  // namespace
@@ -789,14 +821,16 @@ void conv3d_wino(const float* x1, int c1, const float* x2, int c2, const void* p
                               out_vox * cout);
   ProfScope prof("conv3d_wino", flops, bytes, st);
   const dim3 grid((unsigned)std::min<int64_t>(compute_units(), ceil_div(nwg, 8) * 8)), block(kWThreads);
-  if (p.zb == 4 && !p.tall)
-    hipLaunchKernelGGL((wino_yx_kernel<4, false>), grid, block, 0, st, a);
+  if (p.zb == 4 && p.shape == kWide)
+    hipLaunchKernelGGL((wino_yx_kernel<4, kWide>), grid, block, 0, st, a);
   else if (p.zb == 4)
-    hipLaunchKernelGGL((wino_yx_kernel<4, true>), grid, block, 0, st, a);
-  else if (!p.tall)
-    hipLaunchKernelGGL((wino_yx_kernel<2, false>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((wino_yx_kernel<4, kTall>), grid, block, 0, st, a);
+  else if (p.shape == kWide)
+    hipLaunchKernelGGL((wino_yx_kernel<2, kWide>), grid, block, 0, st, a);
+  else if (p.shape == kTall)
+    hipLaunchKernelGGL((wino_yx_kernel<2, kTall>), grid, block, 0, st, a);
   else
-    hipLaunchKernelGGL((wino_yx_kernel<2, true>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((wino_yx_kernel<2, kCube>), grid, block, 0, st, a);
   launch_check("conv3d_winograd");
 }
 

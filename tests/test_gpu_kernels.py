@@ -192,6 +192,8 @@ def test_conv3d_winograd_random_shapes_match_float64(lib, case):
     (8, (18, 33, 24), 32, 0, 64),    # 4 x 16 x 8 boxes
     (1, (3, 8, 17), 32, 0, 32),      # 2 x 8 x 16 boxes
     (1, (3, 17, 7), 16, 32, 32),     # 2 x 16 x 8 boxes, an odd chunk count
+    (29, (7, 8, 8), 48, 0, 160),     # 4 x 8 x 8 boxes of two slabs, several a workgroup
+    (60, (9, 5, 7), 16, 0, 64),      # the same, one chunk, remainders on every axis
 ], ids=lambda c: f"b{c[0]}-{c[1]}-c{c[2]}+{c[3]}-o{c[4]}")
 def test_conv3d_winograd_box_shapes_match_float64(lib, case):
     """Each box shape of the Winograd kernel (the choice follows the volume and the number of
