@@ -139,6 +139,8 @@ struct IgemmArgs {
   const uint4* w16;   // split-fp16 packed weights (x3 kernel)
   int ntg;            // tap groups of 4 (x3 kernel)
   float out_scale;    // 1 / weight scale (x3 kernel)
+  int cper;           // chunks of a workgroup (igemm_x3): blockIdx.y takes [cper blockIdx.y, + cper)
+  int64_t split_stride;  // elements between the outputs of two blockIdx.y
   // pending InstanceNorm (+ LeakyReLU) of input 0 / 1: (mean, scale, beta, 0) per (b, c)
   const float4* nrm0;
   const float4* nrm1;
@@ -749,6 +751,8 @@ __global__ __launch_bounds__(64 * WM* WN, 3) void igemm_x3_kernel(IgemmArgs a) {
   extern __shared__ __align__(16) float lds[];
   constexpr int NT = 64 * WM * WN;
   static_assert(NT == kX3Threads, "split kernel variants use 256 threads");
+  a.y += blockIdx.y * a.split_stride;
+  const int cbeg = blockIdx.y * a.cper, cend = min(cbeg + a.cper, a.chunks);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -873,9 +877,9 @@ __global__ __launch_bounds__(64 * WM* WN, 3) void igemm_x3_kernel(IgemmArgs a) {
     }
   };
 
-  fetch(0);
+  fetch(cbeg);
   const int group_stride = a.nblk * 128;
-  for (int chunk = 0; chunk < a.chunks; ++chunk) {
+  for (int chunk = cbeg; chunk < cend; ++chunk) {
     // packed weights: [chunk][group][nblk] x {hi h8 of 64 lanes, lo h8 of 64 lanes}
     const uint4* wc = a.w16 + ((int64_t)chunk * NTG * a.nblk + nbk0) * 128 + lane;
     h8 A[2][MB][2], B[2][NB][2];
@@ -911,7 +915,7 @@ __global__ __launch_bounds__(64 * WM* WN, 3) void igemm_x3_kernel(IgemmArgs a) {
       }
       mma_products<AR>(acc, A[cur], B[cur]);
     }
-    if (chunk + 1 < a.chunks) fetch(chunk + 1);
+    if (chunk + 1 < cend) fetch(chunk + 1);
   }
   igemm_epilogue<MB, NB, WM, WN>(a, acc, lds, wm, wn, slot, row, nbk0, b, tzi, tyi, txi, oz0, oy0,
                                  ox0, a.out_scale);
@@ -1213,12 +1217,13 @@ void launch_igemm(const IgemmArgs& a, int nwg, bool async, hipStream_t st, doubl
 template <int MB, int NB, int WM, int WN, int NTG, bool VEC>
 void launch_x3_vec(const IgemmArgs& a, int arith, size_t lds_bytes, hipStream_t st) {
   constexpr int nt = 64 * WM * WN;
+  const dim3 grid((unsigned)a.nwg, (unsigned)ceil_div(a.chunks, a.cper));
   if (arith == kBf16)
-    hipLaunchKernelGGL((igemm_x3_kernel<MB, NB, WM, WN, NTG, VEC, kBf16>), dim3(a.nwg), dim3(nt),
+    hipLaunchKernelGGL((igemm_x3_kernel<MB, NB, WM, WN, NTG, VEC, kBf16>), grid, dim3(nt),
                        lds_bytes, st, a);
   else
-    hipLaunchKernelGGL((igemm_x3_kernel<MB, NB, WM, WN, NTG, VEC, kSplit3>), dim3(a.nwg),
-                       dim3(nt), lds_bytes, st, a);
+    hipLaunchKernelGGL((igemm_x3_kernel<MB, NB, WM, WN, NTG, VEC, kSplit3>), grid, dim3(nt),
+                       lds_bytes, st, a);
 }
 
 template <int MB, int NB, int WM, int WN, int NTG>
@@ -2611,10 +2616,26 @@ int conv_x3_stats_tiles(const ConvGeom& g, int cout, int c1, int c2, int arith) 
   return (int)(ceil_div(g.out[0], box.z) * ceil_div(g.out[1], box.y) * ceil_div(g.out[2], box.x));
 }
 
+// The register-staged (strided) kernel's layers with less than a workgroup a CU: chunks split over
+// the idle CUs (two workgroups a CU), at least four (8 channels each) a workgroup.
+int conv_x3_splits(const ConvGeom& g, int c1, int c2, int cout, int arith) {
+  if (arith == kBf16 && conv_bf16_direct_supported(g, c1, c2, cout)) return 1;
+  const X3Plan plan = plan_x3(g, cout);
+  if (plan.staged) return 1;
+  const int64_t nwg = (int64_t)g.batch * plan.box.tiles * ceil_div(cout, plan.v.n());
+  const int64_t chunks = ceil_div(c1, kChunk) + ceil_div(c2, kChunk);
+  const int64_t most = std::min<int64_t>(2 * compute_units() / nwg, chunks / 4);
+  const int64_t spatial = (int64_t)g.out[0] * g.out[1] * g.out[2];
+  if (most < 2 || !split_sum_supported(spatial, cout)) return 1;
+  if (split_sum_parts(spatial) > 1 && chunks < 16) return 1;
+  return (int)ceil_div(chunks, ceil_div(chunks, most));
+}
+
 void conv3d_x3(const float* x1, int c1, const float* x2, int c2, const void* packed,
                float scale, const float* bias, float* y, const ConvGeom& g, int cout,
                hipStream_t st, float4* stats, const PendingNorm& n1, const PendingNorm& n2,
-               int arith) {
+               int arith, int splits) {
+  require(splits == 1 || (!stats && !bias), "a split convolution is finished by its sum");
   require(x1 && y && packed, "convolution pointers must not be null");
   require(c1 >= 1 && (c2 == 0 || x2), "invalid convolution inputs");
   require(scale > 0.f && std::isfinite(scale), "weight scale must be positive");
@@ -2633,6 +2654,9 @@ void conv3d_x3(const float* x1, int c1, const float* x2, int c2, const void* pac
   a.w16 = reinterpret_cast<const uint4*>(packed);
   a.ntg = conv_x3_groups(g.k);
   a.out_scale = 1.0f / scale;
+  a.cper = (int)ceil_div(a.chunks, splits);
+  a.split_stride = (int64_t)g.batch * g.out[0] * g.out[1] * g.out[2] * cout;
+  require(!plan.staged || splits == 1, "the weight-staged kernel does not split");
   require(plan.staged || (int64_t)a.hz * a.hy * a.hx <= kX3MaxHalo,
           "split convolution halo exceeds the staging");
   double flops, bytes;
@@ -2682,7 +2706,9 @@ void conv3d_direct_cin1(const float* x, const float* w, const float* bias, float
   if (split) {
     // split products on MFMA: the output write bounds it (reported against HBM).  Each
     // block takes kDirX3TilesPerBlock consecutive tiles (weights split once per block).
-    const int tpb = kDirX3TilesPerBlock;
+    // fewer where that leaves CUs idle (a 32^3 tile has 128: 8 blocks of 16 took 68 us)
+    const int tpb = (int)std::min<int64_t>(
+        kDirX3TilesPerBlock, std::max<int64_t>(1, tiles * batch / (4 * compute_units())));
     const dim3 grid_x3((unsigned)ceil_div(tiles, tpb), (unsigned)batch);
     ProfScope prof("conv3d_direct_cin1_x3", 0.0, bytes, st);
     switch (cout / 4) {

@@ -147,7 +147,7 @@ void conv_x3_pack_weight(const float* d_w, int cout, const int* ksize, int c1, i
 void conv3d_x3(const float* x1, int c1, const float* x2, int c2, const void* packed,
                float scale, const float* bias, float* y, const ConvGeom& g, int cout,
                hipStream_t st, float4* stats = nullptr, const PendingNorm& n1 = {},
-               const PendingNorm& n2 = {}, int arith = kArithSplit3);
+               const PendingNorm& n2 = {}, int arith = kArithSplit3, int splits = 1);
 int conv_x3_stats_tiles(const ConvGeom& g, int cout, int c1, int c2, int arith);
 
 // Compute units of the current device, a multiple of the 8 XCDs (the persistent kernels' grid).
@@ -180,7 +180,18 @@ void conv_wino_pack_weight(const float* d_w, int cout, int c1, int c2, float sca
 void conv3d_wino(const float* x1, int c1, const float* x2, int c2, const void* packed,
                  float scale, const float* bias, float* y, const ConvGeom& g, int cout,
                  hipStream_t st, float4* stats = nullptr, const PendingNorm& n1 = {},
-                 const PendingNorm& n2 = {});
+                 const PendingNorm& n2 = {}, int splits = 1);
+// Splitting the input channels of a layer too small for the chip: with splits > 1 (a layer's
+// *_splits, given back to the convolution) y receives `splits` partial results without bias,
+// one after the other, which split_sum adds in order with the bias, storing the output and the
+// InstanceNorm parameters (as instnorm_merge_partials).
+int conv_wino_splits(const ConvGeom& g, int c1, int c2, int cout);
+int conv_x3_splits(const ConvGeom& g, int c1, int c2, int cout, int arith);
+bool split_sum_supported(int64_t spatial, int channels);
+int split_sum_parts(int64_t spatial);  // rows of `stats` an item (used where more than one)
+void split_sum(const float* partial, int splits, int batch, int64_t spatial, int channels,
+               const float* bias, const float* gamma, const float* beta, float eps, float* y,
+               float4* params, float4* stats, hipStream_t st);
 // Whether the split kernel handles this kernel size / stride (tap count and halo size).
 bool conv_x3_supported(const int* ksize, const int* stride, int cout);
 // With `stats`: per-block InstanceNorm partials, conv_direct_stats_tiles(size) per item.

@@ -11,6 +11,8 @@
 //      (+ residual before the activation), vectorised float4, in place allowed.
 #include <mutex>
 
+#include <type_traits>
+
 #include "nnx_internal.h"
 
 namespace nnx {
@@ -318,6 +320,134 @@ __global__ __launch_bounds__(256) void norm_merge_final_kernel(const float4* __r
   float scale = 1.0f / sqrtf(varf + eps);
   if (gamma) scale = gamma[c] * scale;
   params[(int64_t)b * C + c] = make_float4((float)m, scale, beta ? beta[c] : 0.f, 0.f);
+}
+
+// The end of a split convolution: y = sum over the splits in order (+ bias) of a (B, S, C)
+// tensor, and the InstanceNorm parameters of y.  A workgroup holds 8 channels of an item, at
+// most kSplitVox x 256 voxels, in registers (thread = channel quad and voxel modulo 256), so
+// the mean and the centred squares are two passes over registers; sums across threads in
+// float64.  Volumes of more voxels take a workgroup (blockIdx.z) per kSplitVox x 256 and leave
+// InstanceNorm partials (mean, M2, n) for instnorm_merge_partials; up to there it writes the
+// parameters and takes the place of the merge launch.  Latency: 5 us, of which a launch is 2
+// (21 to 28 us at 16^3 while a workgroup took a whole item).
+constexpr int kSplitVox = 4;
+
+__global__ __launch_bounds__(512) void split_sum_kernel(
+    const float* __restrict__ part, int splits, int64_t stride, int S, int C,
+    const float* __restrict__ bias, const float* __restrict__ gamma,
+    const float* __restrict__ beta, float eps, float* __restrict__ y, float4* __restrict__ params,
+    float4* __restrict__ stats) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  __shared__ double red[2][8][8];  // pass, wave, channel
+  const int q = threadIdx.x & 1, v0 = threadIdx.x >> 1, lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int c = blockIdx.x * 8 + q * 4;
+  const int first = blockIdx.z * kSplitVox * 256;
+  const int64_t item = ((int64_t)blockIdx.y * S + first) * C;
+  S = min(S - first, kSplitVox * 256);  // voxels of this workgroup
+  const int rounds = (S + 255) / 256;   // uniform
+  f4 b4 = {0.f, 0.f, 0.f, 0.f};
+  if (bias) b4 = *reinterpret_cast<const f4*>(bias + c);
+  // W voxels of the thread from round i0 on, W x P loads in flight (clamped at the last voxel)
+  f4 v[kSplitVox];
+#pragma unroll
+  for (int i = 0; i < kSplitVox; ++i) v[i] = f4{0.f, 0.f, 0.f, 0.f};
+  auto gather = [&](auto i0c, auto wc, auto pc) __attribute__((always_inline)) {
+    constexpr int I0 = decltype(i0c)::value, W = decltype(wc)::value, P = decltype(pc)::value;
+    const float* p[W];
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+      p[w] = part + item + (int64_t)min((I0 + w) * 256 + v0, S - 1) * C + c;
+    int s = 0;
+    for (; s + P <= splits; s += P) {
+      f4 t[P][W];
+#pragma unroll
+      for (int j = 0; j < P; ++j)
+#pragma unroll
+        for (int w = 0; w < W; ++w) t[j][w] = *reinterpret_cast<const f4*>(p[w] + (s + j) * stride);
+#pragma unroll
+      for (int j = 0; j < P; ++j)
+#pragma unroll
+        for (int w = 0; w < W; ++w) v[I0 + w] += t[j][w];
+    }
+    for (; s < splits; ++s)
+#pragma unroll
+      for (int w = 0; w < W; ++w) v[I0 + w] += *reinterpret_cast<const f4*>(p[w] + s * stride);
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      v[I0 + w] += b4;
+      const int vox = (I0 + w) * 256 + v0;
+      if (vox < S) *reinterpret_cast<f4*>(y + item + (int64_t)vox * C + c) = v[I0 + w];
+    }
+  };
+  if (rounds == 1) {
+    gather(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{},
+           std::integral_constant<int, 5>{});
+  } else {
+    using W4 = std::integral_constant<int, 4>;
+    using P2 = std::integral_constant<int, 2>;
+    gather(std::integral_constant<int, 0>{}, W4{}, P2{});
+  }
+  // over the workgroup's threads of this quad: rows of 16 by DPP and lane swaps in float32 (32
+  // values), the waves in float64
+  auto total = [&](f4 x, int pass, double (&out)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float d = x[e];
+      d += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(d), 0x122, 0xf, 0xf, false));
+      d += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(d), 0x124, 0xf, 0xf, false));
+      d += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(d), 0x128, 0xf, 0xf, false));
+      auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(d), __float_as_uint(d), false, false);
+      d = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      r = __builtin_amdgcn_permlane32_swap(__float_as_uint(d), __float_as_uint(d), false, false);
+      if (lane < 2)
+        red[pass][wave][q * 4 + e] = (double)__uint_as_float(r[0]) + (double)__uint_as_float(r[1]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      out[e] = red[pass][0][q * 4 + e];
+#pragma unroll
+      for (int w = 1; w < 8; ++w) out[e] += red[pass][w][q * 4 + e];
+    }
+  };
+  f4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < kSplitVox; ++i) {
+    if (i < rounds && i * 256 + v0 < S) sum += v[i];
+  }
+  double t[4];
+  total(sum, 0, t);
+  f4 mean;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) mean[e] = (float)(t[e] / (double)S);
+  f4 sq = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < kSplitVox; ++i) {
+    if (i < rounds && i * 256 + v0 < S) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float d = v[i][e] - mean[e];
+        sq[e] = fmaf(d, d, sq[e]);
+      }
+    }
+  }
+  total(sq, 1, t);
+  if (threadIdx.x < 2 && gridDim.z > 1) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      stats[((int64_t)blockIdx.y * gridDim.z + blockIdx.z) * C + c + e] =
+          make_float4(mean[e], (float)t[e], (float)S, 0.f);
+  } else if (threadIdx.x < 2) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float var = (float)(t[e] / (double)S);
+      float scale = 1.0f / sqrtf(var + eps);
+      if (gamma) scale = gamma[c + e] * scale;
+      params[(int64_t)blockIdx.y * C + c + e] =
+          make_float4(mean[e], scale, beta ? beta[c + e] : 0.f, 0.f);
+    }
+  }
 }
 
 // y = act(fma(x (+ bias) - mean, scale, beta) (+ residual)) over a (B, S, C) tensor, VW
@@ -643,15 +773,42 @@ void instnorm_merge_partials(float4* partials, int nparts, int batch, int64_t sp
     launch_check("instnorm merge partials");
     return;
   }
-  // ~2048 blocks in all; nslices <= nparts / 2 balanced slices of at least two rows each (a
-  // slice's result takes its first two rows)
-  const int nslices = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(2048, batch), nparts / 2));
+  // ~2048 blocks in all, at most 512 an item (a lane of the second pass merges one entry in 64
+  // after the other: 24 us over 2048 entries); nslices <= nparts / 2 balanced slices of at least two
+  // rows each (a slice's result takes its first two rows)
+  const int nslices = (int)std::max<int64_t>(
+      1, std::min<int64_t>(std::min<int64_t>(ceil_div(2048, batch), 512), nparts / 2));
   hipLaunchKernelGGL(norm_merge_slices_kernel, dim3(nslices, batch), dim3(256), 0, st, partials,
                      channels, nparts);
   launch_check("instnorm merge slices");
   hipLaunchKernelGGL(norm_merge_final_kernel, fgrid, dim3(256), 0, st, partials, params, beta,
                      gamma, spatial, channels, nparts, nslices, 0, eps);
   launch_check("instnorm merge partials");
+}
+
+int split_sum_parts(int64_t spatial) { return (int)ceil_div(spatial, 256 * kSplitVox); }
+
+bool split_sum_supported(int64_t spatial, int channels) {
+  return split_sum_parts(spatial) <= 64 && channels % 8 == 0 && channels <= 512;
+}
+
+void split_sum(const float* partial, int splits, int batch, int64_t spatial, int channels,
+               const float* bias, const float* gamma, const float* beta, float eps, float* y,
+               float4* params, float4* stats, hipStream_t st) {
+  require(partial && y && params && stats, "split sum pointers must not be null");
+  require(split_sum_supported(spatial, channels) && batch >= 1 && batch <= 65535 && splits >= 1,
+          "invalid split sum");
+  const int parts = split_sum_parts(spatial);
+  {
+  ProfScope prof("split_sum", 0.0, 4.0 * (double)batch * spatial * channels * (splits + 1), st);
+  hipLaunchKernelGGL(split_sum_kernel,
+                     dim3((unsigned)(channels / 8), (unsigned)batch, (unsigned)parts), dim3(512), 0, st,
+                     partial, splits, (int64_t)batch * spatial * channels, (int)spatial, channels,
+                     bias, gamma, beta, eps, y, params, stats);
+  launch_check("split sum");
+  }
+  if (parts > 1)
+    instnorm_merge_partials(stats, parts, batch, spatial, channels, gamma, beta, eps, params, st);
 }
 
 void instnorm_apply_params(const float* x, float* y, int batch, int64_t spatial, int channels,

@@ -187,6 +187,7 @@ struct Workspace {
   std::vector<std::unique_ptr<DevBuf>> bufs;
   DevBuf stats;   // per-tile InstanceNorm partials written by the conv epilogue
   size_t stats_bytes = 0;
+  DevBuf split;   // partial results of a split convolution
   float* get(size_t i) { return bufs[i]->as<float>(); }
 };
 
@@ -460,6 +461,7 @@ struct Planner {
   // During planning, records buffer sizes; during execution, hands out the same buffers.
   std::vector<size_t> sizes;
   size_t stats = 0;
+  size_t split = 0;
   size_t next = 0;
   bool planning = true;
   Workspace* ws = nullptr;
@@ -530,6 +532,33 @@ struct Runner {
     // Implicit GEMM: the epilogue writes per-tile statistics, so the norm never re-reads the
     // tensor for them.
     const ConvGeom g = make_conv_geom(n, in.d, c.k, c.s);
+    const int splits = c.wino    ? conv_wino_splits(g, c.cin1, c.cin2, c.cout)
+                       : c.split ? conv_x3_splits(g, c.cin1, c.cin2, c.cout, c.arith)
+                                 : 1;
+    if (splits > 1) {
+      // a layer too small for the chip: its input channels over several workgroups, then one
+      // kernel for the sum, the bias and the norm parameters
+      if (plan->planning) {
+        plan->split = std::max(plan->split, (size_t)splits * n * vox * c.cout * sizeof(float));
+        plan->stats = std::max(plan->stats, (size_t)n * split_sum_parts(vox) * c.cout * sizeof(float4));
+        return result;
+      }
+      float* partial = plan->ws->split.as<float>();
+      if (c.wino)
+        conv3d_wino(x1.data, c.cin1, x2.data, c.cin2, c.packed.ptr, c.scale, nullptr, partial, g,
+                    c.cout, st, nullptr, x1.norm, x2.norm, splits);
+      else
+        conv3d_x3(x1.data, c.cin1, x2.data, c.cin2, c.packed.ptr, c.scale, nullptr, partial, g,
+                  c.cout, st, nullptr, x1.norm, x2.norm, c.arith, splits);
+      split_sum(partial, splits, n, vox, c.cout, pdev(m, c.pb), pdev(m, c.pg), pdev(m, c.pbeta),
+                m->eps, out, params, plan->ws->stats.as<float4>(), st);
+      if (!defer)
+        instnorm_apply_params(out, out, n, vox, c.cout, params, nullptr, act, m->slope, residual,
+                              st);
+      if (layer_checks_enabled())
+        check_layer(m->params[c.pw].name, out, (int64_t)n * vox * c.cout, n, st);
+      return result;
+    }
     const int tiles = c.wino    ? conv_wino_stats_tiles(g, c.cout)
                       : c.split ? conv_x3_stats_tiles(g, c.cout, c.cin1, c.cin2, c.arith)
                                 : conv_stats_tiles(g, c.cout, c.cin1, c.cin2);
@@ -735,6 +764,7 @@ void ensure_workspace(nnx_model* m, int n, const Shape3& in) {
     ws.stats.ensure(plan.stats);
     ws.stats_bytes = plan.stats;
   }
+  ws.split.ensure(plan.split);
   ws.n = n;
   ws.in = in;
 }

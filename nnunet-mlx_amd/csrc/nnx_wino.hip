@@ -120,6 +120,8 @@ struct WinoArgs {
   int nbz, nby, nbx;
   int nbox;   // batch * nbz * nby * nbx (boxes of one column block)
   int nvirt;  // nbox * cout / 32: (column block, box) pairs, column block slowest
+  int cper;   // chunks of a workgroup: blockIdx.y takes chunks [cper blockIdx.y, + cper)
+  int64_t split_stride;  // elements between the outputs of two blockIdx.y
   float out_scale;
   float4* stats;
   const float4* nrm0;
@@ -232,7 +234,8 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
   const int vend = vbeg + vq + (xcd < vr ? 1 : 0);
   int v = vbeg + (int)(blockIdx.x >> 3);
   if (v >= vend) return;  // uniform over the workgroup, before any barrier
-  __builtin_assume(a.chunks > 0);
+  const int cbeg = blockIdx.y * a.cper, cend = min(cbeg + a.cper, a.chunks);
+  __builtin_assume(cend > cbeg);
   const int64_t plane_vox = (int64_t)a.H * a.W;
   constexpr int kRounds = G::rounds, kL = G::lines;
   uint64_t zero = (uint64_t)g_wino_zero;
@@ -383,9 +386,9 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
     const int tid = threadIdx.x;
     const WinoBox first = wino_box(a, v);
     box_lines(tid, first, yx, quads);
-    fetch(source(first, 0), yx, quads, 0, std::integral_constant<int, 0>{},
+    fetch(source(first, cbeg), yx, quads, 0, std::integral_constant<int, 0>{},
           std::integral_constant<int, kRounds>{});
-    const uint4* up = uaddr(tid & 63, first.nt, 0);
+    const uint4* up = uaddr(tid & 63, first.nt, cbeg);
 #pragma unroll
     for (int kz = 0; kz < 3; ++kz) load_u(up, kz);
     load_prm(tid, first.b);  // (behind the halo, whose latency theirs hides in)
@@ -475,25 +478,25 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
         }
     };
 
-    for (int chunk = 0; chunk < a.chunks; ++chunk) {
+    for (int chunk = cbeg; chunk < cend; ++chunk) {
       __builtin_amdgcn_s_waitcnt(0);  // this thread's halo lines and U have landed
       normalise(cur, yx, quads, chunk, buf);
       lds_barrier();  // every thread's lines; the other buffer is free
-      const bool last = chunk + 1 == a.chunks;
+      const bool last = chunk + 1 == cend;
       // the next chunk's halo; after the box's last chunk the next box's first, if there is one
       if (last && more) {
         int tid_n = tid;
         asm volatile("" : "+v"(tid_n));  // computed here, not hoisted and held
         box_lines(tid_n, nxt, yx, quads);
       }
-      const Source src = source(last ? nxt : cur, last ? 0 : chunk + 1);
+      const Source src = source(last ? nxt : cur, last ? cbeg : chunk + 1);
       auto rounds = [&](auto ic) __attribute__((always_inline)) {
         constexpr int I = decltype(ic)::value;
         if (!last || more)
           fetch(src, yx, quads, buf ^ 1, std::integral_constant<int, I * kRounds / ZB>{},
                 std::integral_constant<int, (I + 1) * kRounds / ZB>{});
       };
-      const uint4* un = uaddr(lane, last ? nxt.nt : cur.nt, last ? 0 : chunk + 1);
+      const uint4* un = uaddr(lane, last ? nxt.nt : cur.nt, last ? cbeg : chunk + 1);
       rounds(std::integral_constant<int, 0>{});
       plane(std::integral_constant<int, 0>{});
       rounds(std::integral_constant<int, 1>{});
@@ -609,7 +612,7 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
         for (int e = 0; e < 4; ++e) out[e] = make_float4(mean[e], t[e], cnt, 0.f);
       }
     }
-    float* out = a.y + (((int64_t)cur.b * a.D + z0) * plane_vox + (int64_t)yy * a.W + xx) * a.cout +
+    float* out = a.y + blockIdx.y * a.split_stride + (((int64_t)cur.b * a.D + z0) * plane_vox + (int64_t)yy * a.W + xx) * a.cout +
                  cur.nt * 32 + 4 * quad;
 #pragma unroll
     for (int z = 0; z < ZB; ++z)
@@ -737,6 +740,21 @@ bool conv_wino_supported(const ConvGeom& g, int c1, int c2, int cout) {
          c1 + c2 <= kMaxChannels;
 }
 
+// Layers with less than half a box a CU stand on a chain of chunks (2.9 us each) in a few
+// workgroups: their chunks are split over the idle CUs, at least two a workgroup, and summed
+// behind.
+int conv_wino_splits(const ConvGeom& g, int c1, int c2, int cout) {
+  const WinoPlan p = wino_plan(g, cout);
+  const int64_t boxes = (int64_t)g.batch * p.nbz * p.nby * p.nbx * (cout / 32);
+  const int chunks = (c1 + c2) / kWChunk;
+  const int64_t spatial = (int64_t)g.out[0] * g.out[1] * g.out[2];
+  const int64_t most = std::min<int64_t>(compute_units() / boxes, chunks / 2);
+  if (most < 2 || !split_sum_supported(spatial, cout)) return 1;
+  // where the sum is a launch more (6 us) it takes eight chunks to gain by it
+  if (split_sum_parts(spatial) > 1 && chunks < 8) return 1;
+  return (int)ceil_div(chunks, ceil_div(chunks, most));
+}
+
 int conv_wino_stats_tiles(const ConvGeom& g, int cout) {
   const WinoPlan p = wino_plan(g, cout);
   return p.nbz * p.nby * p.nbx;
@@ -774,9 +792,11 @@ void conv_wino_pack_weight(const float* d_w, int cout, int c1, int c2, float sca
 
 void conv3d_wino(const float* x1, int c1, const float* x2, int c2, const void* packed,
                  float scale, const float* bias, float* y, const ConvGeom& g, int cout,
-                 hipStream_t st, float4* stats, const PendingNorm& n1, const PendingNorm& n2) {
+                 hipStream_t st, float4* stats, const PendingNorm& n1, const PendingNorm& n2,
+                 int splits) {
   require(x1 && y && packed, "convolution pointers must not be null");
   require(c2 == 0 || x2, "invalid convolution inputs");
+  require(splits == 1 || (!stats && !bias), "a split convolution is finished by its sum");
   require(conv_wino_supported(g, c1, c2, cout),
           "the Winograd convolution takes stride-1 3x3x3 layers with C_out % 32 == 0 and input "
           "channel counts that are multiples of 16, at most 1024 input channels in all");
@@ -808,6 +828,8 @@ void conv3d_wino(const float* x1, int c1, const float* x2, int c2, const void* p
   require(nwg < (1LL << 31), "convolution grid too large");
   a.nvirt = (int)nwg;
   a.nbox = a.nvirt / (cout / 32);
+  a.cper = (int)ceil_div(a.chunks, splits);
+  a.split_stride = (int64_t)g.batch * g.out[0] * g.out[1] * g.out[2] * cout;
   a.out_scale = 1.0f / scale;
   a.stats = stats;
   a.nrm0 = n1.params;
@@ -820,7 +842,8 @@ void conv3d_wino(const float* x1, int c1, const float* x2, int c2, const void* p
   const double bytes = 4.0 * ((double)g.batch * g.in[0] * g.in[1] * g.in[2] * (c1 + c2) +
                               out_vox * cout);
   ProfScope prof("conv3d_wino", flops, bytes, st);
-  const dim3 grid((unsigned)std::min<int64_t>(compute_units(), ceil_div(nwg, 8) * 8)), block(kWThreads);
+  const dim3 grid((unsigned)std::min<int64_t>(compute_units(), ceil_div(nwg, 8) * 8),
+                  (unsigned)ceil_div(a.chunks, a.cper)), block(kWThreads);
   if (p.zb == 4 && p.shape == kWide)
     hipLaunchKernelGGL((wino_yx_kernel<4, kWide>), grid, block, 0, st, a);
   else if (p.zb == 4)

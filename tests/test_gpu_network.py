@@ -216,6 +216,27 @@ def test_conv_route_matches_oracle(device, monkeypatch, name, algo):
     assert rel_l2(got, ref) <= 1e-5, msg
 
 
+@pytest.mark.parametrize("patch", [(24, 40, 32), (64, 48, 32), (8, 8, 8)], ids=str)
+def test_split_layers_match_oracle(device, patch):
+    """One item of a network whose deep layers are too few boxes for the chip: their input
+    channels are split over workgroups and summed, with the norm parameters from the sum (up to
+    1024 voxels) or from its partials (1536 voxels in the second patch); one voxel in the last
+    stage of the third."""
+    spec = PlainConvUNetSpec(1, 3, (32, 64, 256, 320), K3 * 4, ((1, 1, 1),) + ((2, 2, 2),) * 3,
+                             (2,) * 4, (2,) * 3)
+    weights = random_weights(spec, seed=17, random_affine=True)
+    x = np.random.default_rng(3).standard_normal((1, *patch, 1)).astype(np.float32)
+    print(f"split layers, patch {patch}", flush=True)
+    net = build_network(spec)
+    net.load_weights(weights)
+    got = net(torch.from_numpy(x).to(device)).cpu().numpy()
+    net.close()
+    ref = OracleNetwork(spec, weights)(x)
+    msg = report(f"split layers {patch}", got, ref)
+    print(msg, flush=True)
+    assert np.abs(got - ref).max() <= 1e-3 and rel_l2(got, ref) <= 1e-5, msg
+
+
 def test_persistent_winograd_forward_is_bit_identical(device, monkeypatch):
     """The persistent Winograd kernel runs the layers with at least four boxes a CU (here
     the 64^3 and 32^3 stages at batch 4) with the one-box kernel's arithmetic, including
