@@ -366,13 +366,15 @@ def kernel_class_of(short: str) -> str | None:
     (igemm_kernel<MB, NB, WM, WN, ...> -> conv3d_igemm_m{16*MB*WM}n{16*NB*WN}, the
     split-fp16 kernels igemm_x3s_kernel / igemm_x3_kernel -> conv3d_x3s_* / conv3d_x3_*, and
     the Winograd kernels -> conv3d_wino, the
-    direct bf16 kernel -> conv3d_x3s_bf16_m512n64)."""
+    direct bf16 kernel -> conv3d_x3s_bf16_m512n64, the strided kernel -> conv3d_x3_m128n64)."""
     import re
 
     if short.startswith(("wino_yx_kernel", "wino_x3_kernel", "wino_x3p_kernel")):
         return "conv3d_wino"
     if short.startswith("conv_bf16_kernel"):
         return "conv3d_x3s_bf16_m512n64"
+    if short.startswith("conv_strided_kernel"):
+        return "conv3d_x3_bf16_m128n64" if "1>" in short else "conv3d_x3_m128n64"
     m = re.match(r"igemm(_x3s|_x3)?_kernel<(\d+), (\d+), (\d+), (\d+)([^>]*)>", short)
     if not m:
         return None

@@ -2612,6 +2612,7 @@ bool conv_x3_supported(const int* ksize, const int* stride, int cout) {
 int conv_x3_stats_tiles(const ConvGeom& g, int cout, int c1, int c2, int arith) {
   if (arith == kBf16 && conv_bf16_direct_supported(g, c1, c2, cout))
     return conv_bf16_direct_stats_tiles(g);
+  if (conv_strided_supported(g, c1, c2, cout)) return conv_strided_stats_tiles(g);
   const Box box = plan_x3(g, cout).box;
   return (int)(ceil_div(g.out[0], box.z) * ceil_div(g.out[1], box.y) * ceil_div(g.out[2], box.x));
 }
@@ -2620,6 +2621,7 @@ int conv_x3_stats_tiles(const ConvGeom& g, int cout, int c1, int c2, int arith) 
 // the idle CUs (two workgroups a CU), at least four (8 channels each) a workgroup.
 int conv_x3_splits(const ConvGeom& g, int c1, int c2, int cout, int arith) {
   if (arith == kBf16 && conv_bf16_direct_supported(g, c1, c2, cout)) return 1;
+  if (conv_strided_supported(g, c1, c2, cout)) return conv_strided_splits(g, c1, c2, cout);
   const X3Plan plan = plan_x3(g, cout);
   if (plan.staged) return 1;
   const int64_t nwg = (int64_t)g.batch * plan.box.tiles * ceil_div(cout, plan.v.n());
@@ -2645,6 +2647,11 @@ void conv3d_x3(const float* x1, int c1, const float* x2, int c2, const void* pac
                          reinterpret_cast<uintptr_t>(y);
   if (arith == kBf16 && ends % 16 == 0 && conv_bf16_direct_supported(g, c1, c2, cout)) {
     conv3d_bf16_direct(x1, c1, x2, c2, packed, scale, bias, y, g, cout, st, stats, n1, n2);
+    return;
+  }
+  if (ends % 16 == 0 && conv_strided_supported(g, c1, c2, cout)) {
+    conv3d_strided(x1, c1, x2, c2, packed, conv_packed_nblk(cout), scale, bias, y, g, cout, st, stats,
+                   n1, n2, arith, splits);
     return;
   }
   require(!stats || ends % 16 == 0, "activations must be 16-byte aligned");

@@ -166,6 +166,16 @@ void conv3d_bf16_direct(const float* x1, int c1, const float* x2, int c2, const 
                         hipStream_t st, float4* stats, const PendingNorm& n1,
                         const PendingNorm& n2);
 
+// Strided 3x3x3 convolutions with 16-channel input blocks and C_out % 32 == 0 (nnx_strided.hip), a
+// route of conv3d_x3 on its packed words (nblk16 = their 16-column blocks).
+bool conv_strided_supported(const ConvGeom& g, int c1, int c2, int cout);
+int conv_strided_stats_tiles(const ConvGeom& g);
+int conv_strided_splits(const ConvGeom& g, int c1, int c2, int cout);
+void conv3d_strided(const float* x1, int c1, const float* x2, int c2, const void* packed,
+                    int nblk16, float scale, const float* bias, float* y, const ConvGeom& g,
+                    int cout, hipStream_t st, float4* stats, const PendingNorm& n1,
+                    const PendingNorm& n2, int arith, int splits);
+
 // Winograd F(2x2, 3x3) in (y, x) with the three z taps direct, split-fp16 products
 // (nnx_wino.hip): stride-1 3x3x3 layers with C_out % 32 == 0 and input channel counts that are
 // multiples of 16.  Weights are transformed (U[kz] = G w[kz] G^T per input/output channel pair),

@@ -191,7 +191,7 @@ def test_conv3d_winograd_random_shapes_match_float64(lib, case):
     (8, (18, 23, 31), 16, 16, 32),   # 4 x 8 x 16 boxes, every axis with a remainder
     (8, (18, 33, 24), 32, 0, 64),    # 4 x 16 x 8 boxes
     (1, (3, 8, 17), 32, 0, 32),      # 2 x 8 x 16 boxes
-    (1, (3, 17, 7), 16, 32, 32),     # 2 x 16 x 8 boxes, an odd chunk count
+    (1, (3, 17, 7), 16, 32, 32),     # a single column of boxes, an odd chunk count
     (29, (7, 8, 8), 48, 0, 160),     # 4 x 8 x 8 boxes of two slabs, several a workgroup
     (60, (9, 5, 7), 16, 0, 64),      # the same, one chunk, remainders on every axis
 ], ids=lambda c: f"b{c[0]}-{c[1]}-c{c[2]}+{c[3]}-o{c[4]}")
@@ -561,6 +561,22 @@ def _check_split_tconv(lib, case):
 def _bf16(a: np.ndarray) -> np.ndarray:
     """Round to bf16 (nearest even), returned as float64."""
     return torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).to(torch.bfloat16).double().numpy()
+
+
+# the strided kernel (strides (1 or 2, 2, 2), 16-channel blocks): boxes of 4 x 4 x 8 outputs
+STRIDED_CASES = [
+    (1, (9, 9, 17), 16, 0, 64, (3, 3, 3), (2, 2, 2)),     # one past a box on every axis, one chunk
+    (3, (8, 8, 16), 32, 16, 96, (3, 3, 3), (2, 2, 2)),    # whole boxes, two inputs, half a group
+    (2, (5, 10, 15), 48, 0, 32, (3, 3, 3), (1, 2, 2)),    # z kept, one column block
+    (1, (1, 1, 1), 16, 16, 160, (3, 3, 3), (2, 2, 2)),
+    (12, (17, 30, 62), 16, 0, 64, (3, 3, 3), (1, 2, 2)),  # boxes in turn across items
+]
+
+
+@pytest.mark.parametrize("case", STRIDED_CASES, ids=lambda c: f"b{c[0]}-{c[1]}-c{c[2]}+{c[3]}-o{c[4]}-s{c[6]}")
+def test_conv3d_strided_boxes_match_float64(lib, case):
+    _check_split_conv(lib, case)
+    test_conv3d_bf16_matches_rounded_float64(lib, case)
 
 
 # the direct bf16 kernel (3x3x3, stride 1, 16-channel blocks): boxes of 4 x 8 x 16
