@@ -22,7 +22,7 @@
 // wave-private LDS tile.
 //
 // Bound by latency and issue (matrix cores about 40 % busy).  Against the weight-staged 16x16x32
-// kernel: 64 -> 64 on 64 x 80 x 80 x 4 0.752 -> 0.429 ms (845 TFLOP/s), 256 -> 256 on 16^3 x 8
+// kernel: 64 -> 64 on 64 x 80 x 80 x 4 0.753 -> 0.443 ms (818 TFLOP/s), 256 -> 256 on 16^3 x 8
 // 0.246 -> 0.109 ms (1065), 320 -> 320 on 8^3 0.140 -> 0.107 ms.
 #include <cmath>
 #include <type_traits>

@@ -21,7 +21,7 @@
 //
 // Bound by issue: the conversion's VALU work and the products take about as long, and each
 // SIMD's two waves overlap them in part.  Against the implicit GEMM: 32 -> 64 on 128^3 x 8, stride 2,
-// 1.40 -> 1.10 ms (211 TFLOP/s), 64 -> 128 on 37 x 61 x 43 x 2 66 -> 57 us, 256 -> 320 on 16^3 98 -> 50 us;
+// 1.42 -> 1.14 ms (203 TFLOP/s), 64 -> 128 on 37 x 61 x 43 x 2 66 -> 57 us, 256 -> 320 on 16^3 98 -> 50 us;
 // error against float64 2.5e-7 relative (3.3e-7).
 #include <cmath>
 #include <type_traits>

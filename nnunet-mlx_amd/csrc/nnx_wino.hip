@@ -49,9 +49,9 @@
 // busy at 1.9 GHz (2.4 GHz with the products left out, 2.0 GHz with the products alone), and
 // leaving out any one part (products 38 %, halo DMA 21 %, transform and split 18 %, epilogue
 // 11 %, patch reads 9 %, U loads 7 %) takes its share off the time.  Measured against the
-// three-axis form it replaces, ms: 32 + 32 -> 32 on 128^3 x 8 4.57 -> 3.94 (472 TFLOP/s of the
-// direct convolution's work), 128 -> 128 on 32^3 x 8 0.489 -> 0.438 (529), 64 -> 64 on
-// 37 x 61 x 43 x 4 0.256 -> 0.216 (398); error against float64 2.6e-7 to 3.6e-7 relative
+// three-axis form it replaces, ms: 32 + 32 -> 32 on 128^3 x 8 4.48 -> 3.79 (490 TFLOP/s of the
+// direct convolution's work), 128 -> 128 on 32^3 x 8 0.471 -> 0.406 (571), 64 -> 64 on
+// 37 x 61 x 43 x 4 0.249 -> 0.216 (398); error against float64 2.6e-7 to 3.6e-7 relative
 // (the three-axis form 2.5e-7 to 3.2e-7, the direct split kernel 3.4e-7).
 #include <cmath>
 #include <string>
