@@ -106,9 +106,10 @@ __global__ __launch_bounds__(256) void restore_argmax_kernel(const void* __restr
 // place where the axis-by-axis form reads it.  The resampler's clip to the plane's [min, max]
 // cannot change a finite result: it lies within a few float64 ulps of the bounds, which are
 // float32 (or float16) values, so the rounding to that type already returns them.  Only a NaN
-// (infinite or NaN logits) is replaced by the plane's minimum; a first pass that met one
-// raises a flag, and the two kernels behind it, which otherwise return at once, form the
-// minima and redo the voxels.
+// (infinite or NaN logits) is replaced, by what the clip makes of one: the plane's minimum, or
+// -inf where the plane holds NaN only (the bounds of an empty reduction).  A first pass that
+// met a NaN raises a flag, and the two kernels behind it, which otherwise return at once, form
+// these values and redo the voxels.
 //
 // Roofline: HBM — the logits of the source planes that the nearest indices pick, once, and 2 B a
 // voxel.  300 x 534 x 534 x 3 float16 -> 120 x 512 x 512: 4.90 ms as 30 launches
@@ -144,9 +145,9 @@ struct LinArgs {
   double ratio[3];
   uint16_t* labels;
   int* flag;
-  // redo pass: classes [c0, c1), minima[plane * (c1 - c0) + class - c0], running winners
+  // redo pass: classes [c0, c1), clipped NaN [plane * (c1 - c0) + class - c0], running winners
   int c0, c1;
-  const float* minima;
+  const float* clipped;
   float* best;
 };
 
@@ -210,7 +211,7 @@ __global__ __launch_bounds__(256) void restore_linear_kernel(LinArgs a) {
         if constexpr (REDO) {
           if (v != v) {
             const int plane = SEP == 0 ? taps[0].lo : SEP == 1 ? taps[1].lo : SEP == 2 ? taps[2].lo : 0;
-            v = (double)a.minima[(int64_t)plane * (a.c1 - a.c0) + c - a.c0];
+            v = (double)a.clipped[(int64_t)plane * (a.c1 - a.c0) + c - a.c0];
           }
         } else {
           nan |= v != v;
@@ -232,29 +233,41 @@ __global__ __launch_bounds__(256) void restore_linear_kernel(LinArgs a) {
 
 __global__ void restore_flag_clear_kernel(int* flag) { *flag = 0; }
 
-// minima[plane * (c1 - c0) + class - c0] over the source plane (SEP < 0: the volume) of each
-// class, NaN ignored; one workgroup a plane.  Returns at once unless the flag is raised.
+// clipped[plane * (c1 - c0) + class - c0] = min(max(NaN, lo), hi) with the bounds lo, hi of the
+// source plane (sep < 0: the volume) of each class, formed without its NaN; one workgroup a
+// plane.  Returns at once unless the flag is raised.
 template <bool HALF>
-__global__ __launch_bounds__(1024) void restore_minima_kernel(LinArgs a, int sep, float* minima) {
-  __shared__ float part[16];
+__global__ __launch_bounds__(1024) void restore_clipped_kernel(LinArgs a, int sep, float* clipped) {
+  __shared__ float low[16], high[16];
   if (*a.flag == 0) return;
   const int64_t m = sep < 0 ? (int64_t)a.n[0] * a.n[1] * a.n[2]
                             : (int64_t)a.n[0] * a.n[1] * a.n[2] / a.n[sep];
   const int64_t inner = sep == 0 || sep < 0 ? m : sep == 1 ? a.n[2] : 1;
   for (int c = a.c0; c < a.c1; ++c) {
-    float lo = INFINITY;
+    float lo = INFINITY, hi = -INFINITY;
     for (int64_t i = threadIdx.x; i < m; i += 1024) {
       const int64_t v = sep < 0 ? i : (i / inner * a.n[sep] + blockIdx.x) * inner + i % inner;
-      lo = fminf(lo, (float)load_logit<HALF>(a.logits, v * a.classes + c));
+      const float x = (float)load_logit<HALF>(a.logits, v * a.classes + c);
+      lo = fminf(lo, x);
+      hi = fmaxf(hi, x);
     }
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) lo = fminf(lo, __shfl_xor(lo, o));
+    for (int o = 32; o >= 1; o >>= 1) {
+      lo = fminf(lo, __shfl_xor(lo, o));
+      hi = fmaxf(hi, __shfl_xor(hi, o));
+    }
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = lo;
+    if ((threadIdx.x & 63) == 0) {
+      low[threadIdx.x >> 6] = lo;
+      high[threadIdx.x >> 6] = hi;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-      for (int w = 1; w < 16; ++w) lo = fminf(lo, part[w]);
-      minima[(int64_t)blockIdx.x * (a.c1 - a.c0) + c - a.c0] = lo;
+      for (int w = 1; w < 16; ++w) {
+        lo = fminf(lo, low[w]);
+        hi = fmaxf(hi, high[w]);
+      }
+      clipped[(int64_t)blockIdx.x * (a.c1 - a.c0) + c - a.c0] = fminf(lo, hi);
     }
   }
 }
@@ -296,19 +309,19 @@ int grid_for(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(cei
 int64_t align256(int64_t bytes) { return ceil_div(bytes, 256) * 256; }
 
 template <bool HALF, int SEP>
-void launch_linear(LinArgs a, int planes, float* minima, int64_t minima_room, hipStream_t st) {
+void launch_linear(LinArgs a, int planes, float* clipped, int64_t room, hipStream_t st) {
   const dim3 grid((unsigned)ceil_div(a.N[2], 64),
                   (unsigned)std::min<int64_t>(ceil_div(a.N[1], 4), 65535),
                   (unsigned)std::min(a.N[0], 65535));
   hipLaunchKernelGGL(restore_flag_clear_kernel, dim3(1), dim3(1), 0, st, a.flag);
   hipLaunchKernelGGL((restore_linear_kernel<HALF, SEP, false>), grid, dim3(256), 0, st, a);
-  // as many classes a round as the minima have room for (all of them, as a rule)
-  const int round = (int)std::min<int64_t>(a.classes, std::max<int64_t>(1, minima_room / planes));
+  // as many classes a round as the clipped values have room for (all of them, as a rule)
+  const int round = (int)std::min<int64_t>(a.classes, std::max<int64_t>(1, room / planes));
   for (a.c0 = 0; a.c0 < a.classes; a.c0 = a.c1) {
     a.c1 = std::min(a.classes, a.c0 + round);
-    a.minima = minima;
-    hipLaunchKernelGGL(restore_minima_kernel<HALF>, dim3((unsigned)planes), dim3(1024), 0, st, a,
-                       SEP, minima);
+    a.clipped = clipped;
+    hipLaunchKernelGGL(restore_clipped_kernel<HALF>, dim3((unsigned)planes), dim3(1024), 0, st, a,
+                       SEP, clipped);
     // a small grid (it loops): nearly always every workgroup returns at once, and the full
     // grid took 52 us to do so
     hipLaunchKernelGGL((restore_linear_kernel<HALF, SEP, true>),
@@ -333,16 +346,16 @@ void restore_linear(const void* logits, bool half, int classes, const int* src, 
   }
   a.labels = labels;
   a.flag = reinterpret_cast<int*>(work);
-  float* minima = reinterpret_cast<float*>(work + 256);
+  float* clipped = reinterpret_cast<float*>(work + 256);
   a.best = reinterpret_cast<float*>(work + 256 + align256(4 * n_src));
   const int planes = separate_axis < 0 ? 1 : src[separate_axis];
   ProfScope prof("restore_linear", 0.0, (half ? 2.0 : 4.0) * classes * n_src + 2.0 * n_dst, st);
   auto launch = [&](auto h) {
     constexpr bool H = decltype(h)::value;
-    if (separate_axis < 0) launch_linear<H, -1>(a, planes, minima, n_src, st);
-    else if (separate_axis == 0) launch_linear<H, 0>(a, planes, minima, n_src, st);
-    else if (separate_axis == 1) launch_linear<H, 1>(a, planes, minima, n_src, st);
-    else launch_linear<H, 2>(a, planes, minima, n_src, st);
+    if (separate_axis < 0) launch_linear<H, -1>(a, planes, clipped, n_src, st);
+    else if (separate_axis == 0) launch_linear<H, 0>(a, planes, clipped, n_src, st);
+    else if (separate_axis == 1) launch_linear<H, 1>(a, planes, clipped, n_src, st);
+    else launch_linear<H, 2>(a, planes, clipped, n_src, st);
   };
   if (half) launch(std::true_type{});
   else launch(std::false_type{});

@@ -159,12 +159,14 @@ def test_restore_class_labels_device_policy(device):
     ((9, 13, 70), (14, 9, 65), 0), ((9, 13, 70), (14, 9, 65), 1), ((9, 13, 70), (14, 9, 65), 2),
     ((9, 13, 70), (14, 9, 65), -1), ((1, 1, 1), (3, 2, 5), 0), ((7, 5, 64), (2, 5, 129), 1),
 ], ids=str)
-@pytest.mark.parametrize("special", [False, True], ids=["finite", "special"])
+@pytest.mark.parametrize("special", ["finite", "special", "empty plane", "empty volume"])
 def test_linear_restore_equals_the_resampler_by_class(device, source, target, axis, special):
     """The one-pass order-1 restoration gives the labels of the spline resampler run class by
     class and an argmax, bit for bit: every separate axis and none, up and down, rows around
     the 64-voxel blocks; with infinities and NaN (which the resampler's clip replaces by the
-    plane's minimum) planted in two classes."""
+    plane's minimum) planted in two classes; with a class NaN throughout one plane of the
+    separate axis or the whole volume, where the clip's bounds are those of an empty
+    reduction."""
     from nnunet_mlx import _native
     from nnunet_mlx.prediction.restore import resample_class_logits_argmax_spline_device
     from tests.test_gpu_preprocess import spline_device
@@ -172,7 +174,13 @@ def test_linear_restore_equals_the_resampler_by_class(device, source, target, ax
     print(f"linear restore {source} -> {target} axis {axis} special {special}", flush=True)
     rng = np.random.default_rng(5 + axis + sum(source))
     logits = (rng.standard_normal((*source, 4)) * 3).astype(np.float32)
-    if special:
+    if special == "empty plane":
+        at = [slice(None)] * 3
+        at[max(axis, 0)] = source[max(axis, 0)] // 2
+        logits[(*at, 1)] = np.nan
+    elif special == "empty volume":
+        logits[..., 2] = np.nan
+    elif special == "special":
         flat = logits.reshape(-1, 4)
         for value in (np.nan, np.inf, -np.inf):
             at = rng.integers(0, flat.shape[0], 3)
