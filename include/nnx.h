@@ -402,8 +402,10 @@ int nnx_restore_labels_spline(const void* d_logits, int half, int classes, const
  * channel to new_size (SciPy zoom in grid mode with edge extension, float64, clipped to the
  * input's [min, max]), order 1 or 3; with separate_axis in 0..2 the other two axes are
  * resized plane by plane (clipped per plane, float64) and separate_axis by half-pixel
- * nearest indices (order_z 0), rounded to float32 once.  The caller passes a device
- * workspace of nnx_resample_spline_workspace bytes.  Replaces resample_probabilities_or_data
+ * nearest indices (order_z 0), rounded to float32 once.  Bounds ignore NaN.  Order 3: an
+ * infinity or a NaN reaches every value of its channel (of its plane, with a separate axis),
+ * each of which becomes the lower bound, or -inf where all samples are NaN.  The caller passes
+ * a device workspace of nnx_resample_spline_workspace bytes.  Replaces resample_probabilities_or_data
  * for spline plans (src/nnunet_mlx/data/resampling.py:87-172, 268-306, 379-442, 476-501). */
 #define NNX_NORM_NONE 0
 #define NNX_NORM_CT 1

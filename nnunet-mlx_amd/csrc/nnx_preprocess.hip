@@ -596,12 +596,30 @@ __global__ __launch_bounds__(256) void interp_axis_kernel(const double* __restri
   }
 }
 
-// part[k * parts + j] = (min, max) over part j of plane k along `axis` of a (n0, n1, n2)
+// Bounds of a set of samples without its NaN (+inf, -inf of an empty one), and whether it holds
+// an infinity or a NaN.
+struct Extrema {
+  float lo, hi;
+  int nonfinite;
+};
+
+// The bounds that resampled values are clipped to.  Order 3 (`spread`): the recursions carry an
+// infinity or a NaN over its line, every line that crosses it and so on, so one of either makes
+// every value of the resized axes NaN, of which the clip makes the lower bound.  The
+// pieces that lines are cut into would end that at their ends: both bounds take its place.
+__device__ __forceinline__ float2 clip_bounds(const Extrema& e, bool spread) {
+  if (!spread || !e.nonfinite) return make_float2(e.lo, e.hi);
+  const float v = fminf(e.lo, e.hi);
+  return make_float2(v, v);
+}
+
+// part[k * parts + j] = bounds of part j of plane k along `axis` of a (n0, n1, n2)
 // float32 channel; grid (planes, parts).
 __global__ __launch_bounds__(256) void plane_minmax_kernel(const float* __restrict__ in,
                                                            int64_t n0, int64_t n1, int64_t n2,
-                                                           int axis, float2* __restrict__ part) {
+                                                           int axis, Extrema* __restrict__ part) {
   __shared__ float smin[4], smax[4];
+  __shared__ int sbad[4];
   const int64_t k = blockIdx.x;
   const int parts = gridDim.y, j = blockIdx.y;
   const int64_t dims[3] = {n0, n1, n2};
@@ -609,10 +627,12 @@ __global__ __launch_bounds__(256) void plane_minmax_kernel(const float* __restri
   const int64_t strides[3] = {n1 * n2, n2, 1};
   const int64_t m = dims[a1] * dims[a2];
   float lo = INFINITY, hi = -INFINITY;
+  bool bad = false;
   for (int64_t i = j * (int64_t)blockDim.x + threadIdx.x; i < m; i += (int64_t)parts * blockDim.x) {
     const float v = in[k * strides[axis] + (i / dims[a2]) * strides[a1] + (i % dims[a2]) * strides[a2]];
     lo = fminf(lo, v);
     hi = fmaxf(hi, v);
+    bad |= !isfinite(v);
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
@@ -620,9 +640,11 @@ __global__ __launch_bounds__(256) void plane_minmax_kernel(const float* __restri
     hi = fmaxf(hi, __shfl_xor(hi, o));
   }
   const int wave = threadIdx.x >> 6;
+  const bool any = __any(bad);
   if ((threadIdx.x & 63) == 0) {
     smin[wave] = lo;
     smax[wave] = hi;
+    sbad[wave] = any;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -630,37 +652,46 @@ __global__ __launch_bounds__(256) void plane_minmax_kernel(const float* __restri
       lo = fminf(lo, smin[w]);
       hi = fmaxf(hi, smax[w]);
     }
-    part[k * parts + j] = make_float2(lo, hi);
+    part[k * parts + j] = Extrema{lo, hi, sbad[0] | sbad[1] | sbad[2] | sbad[3]};
   }
 }
 
-// mm[k] = (min, max) over part[k * parts .. k * parts + parts), one thread per plane
-__global__ __launch_bounds__(256) void plane_parts_kernel(const float2* __restrict__ part,
-                                                          int64_t planes, int parts,
+// all[k] = bounds over part[k * parts .. k * parts + parts) and mm[k] = what plane k is clipped
+// to, one thread per plane
+__global__ __launch_bounds__(256) void plane_parts_kernel(const Extrema* __restrict__ part,
+                                                          int64_t planes, int parts, bool spread,
+                                                          Extrema* __restrict__ all,
                                                           float2* __restrict__ mm) {
   const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (k >= planes) return;
-  float lo = INFINITY, hi = -INFINITY;
+  Extrema e{INFINITY, -INFINITY, 0};
   for (int j = 0; j < parts; ++j) {
-    lo = fminf(lo, part[k * parts + j].x);
-    hi = fmaxf(hi, part[k * parts + j].y);
+    const Extrema& p = part[k * parts + j];
+    e.lo = fminf(e.lo, p.lo);
+    e.hi = fmaxf(e.hi, p.hi);
+    e.nonfinite |= p.nonfinite;
   }
-  mm[k] = make_float2(lo, hi);
+  all[k] = e;
+  mm[k] = clip_bounds(e, spread);
 }
 
-// mm[n] = (min, max) over mm[0 .. n)
-__global__ __launch_bounds__(64) void reduce_minmax_kernel(float2* mm, int64_t n) {
+// *mm = what the volume is clipped to, from the n planes' bounds
+__global__ __launch_bounds__(64) void reduce_minmax_kernel(const Extrema* __restrict__ all,
+                                                           int64_t n, bool spread, float2* mm) {
   float lo = INFINITY, hi = -INFINITY;
+  bool bad = false;
   for (int64_t i = threadIdx.x; i < n; i += 64) {
-    lo = fminf(lo, mm[i].x);
-    hi = fmaxf(hi, mm[i].y);
+    lo = fminf(lo, all[i].lo);
+    hi = fmaxf(hi, all[i].hi);
+    bad |= all[i].nonfinite != 0;
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
     lo = fminf(lo, __shfl_xor(lo, o));
     hi = fmaxf(hi, __shfl_xor(hi, o));
   }
-  if (threadIdx.x == 0) mm[n] = make_float2(lo, hi);
+  const bool any = __any(bad);
+  if (threadIdx.x == 0) *mm = clip_bounds(Extrema{lo, hi, any}, spread);
 }
 
 // One rounding of a float64 result: to float32, or to float16 (nearest even) when HALF,
@@ -854,6 +885,7 @@ struct SplinePlan {
   int pad[3];
   int axes[3], naxes;  // resized axes, in order
   int64_t a_elems, b_elems, mm_elems;
+  int64_t extrema;  // of the planes, then of their parts
 };
 
 SplinePlan spline_plan(const int64_t* size, const int64_t* new_size, int separate_axis) {
@@ -879,10 +911,16 @@ SplinePlan spline_plan(const int64_t* size, const int64_t* new_size, int separat
     int64_t& slot = (k % 2 == 0) ? p.a_elems : p.b_elems;
     slot = std::max(slot, sizes[k]);
   }
-  // per-plane (min, max) + the whole-volume entry, then the per-part partials
+  // per-plane bounds + the whole-volume entry
   const int64_t planes = separate_axis >= 0 ? p.n[separate_axis] : p.n[0];
-  p.mm_elems = planes + 1 + planes * kMinmaxParts;
+  p.mm_elems = planes + 1;
+  p.extrema = planes * (1 + kMinmaxParts);
   return p;
+}
+
+// Bytes of the bounds and the extrema behind them, up to the tables' alignment.
+int64_t bounds_bytes(const SplinePlan& p) {
+  return ceil_div(p.mm_elems * (int64_t)sizeof(float2) + p.extrema * (int64_t)sizeof(Extrema), 256) * 256;
 }
 
 // entries of the tap tables (order 3): the outputs of every resized axis
@@ -1141,7 +1179,7 @@ void crop_normalize_masked(const float* x, int channels, const int64_t* size,
 size_t resample_spline_workspace(const int64_t* size, const int64_t* new_size, int separate_axis) {
   const SplinePlan p = spline_plan(size, new_size, separate_axis);
   const int64_t planes = separate_axis >= 0 ? p.n[separate_axis] : 0;
-  return (size_t)(p.a_elems + p.b_elems) * sizeof(double) + (size_t)p.mm_elems * sizeof(float2) +
+  return (size_t)(p.a_elems + p.b_elems) * sizeof(double) + (size_t)bounds_bytes(p) +
          (size_t)tap_count(p) * sizeof(SplineTap) + (size_t)planes * sizeof(longlong2) + 1024;
 }
 
@@ -1164,8 +1202,8 @@ void resample_spline(const float* x, int channels, const int64_t* size, const in
   float2* mm = reinterpret_cast<float2*>(B + p.b_elems);
   const int64_t in_vox = size[0] * size[1] * size[2];
   const int64_t out_vox = new_size[0] * new_size[1] * new_size[2];
-  SplineTap* taps = reinterpret_cast<SplineTap*>(
-      reinterpret_cast<char*>(mm) + ceil_div(p.mm_elems * (int64_t)sizeof(float2), 256) * 256);
+  Extrema* extrema = reinterpret_cast<Extrema*>(mm + p.mm_elems);
+  SplineTap* taps = reinterpret_cast<SplineTap*>(reinterpret_cast<char*>(mm) + bounds_bytes(p));
   longlong2* sep_planes = reinterpret_cast<longlong2*>(
       reinterpret_cast<char*>(taps) + ceil_div(tap_count(p) * (int64_t)sizeof(SplineTap), 256) * 256);
   if (order == 3) {
@@ -1186,15 +1224,17 @@ void resample_spline(const float* x, int channels, const int64_t* size, const in
   for (int c = 0; c < channels; ++c) {
     const float* xc = x + (int64_t)c * in_vox;
     const int64_t planes = size[mm_axis];
-    float2* part = mm + planes + 1;
+    Extrema* part = extrema + planes;
+    const bool spread = order == 3;
     {
       ProfScope prof("spline_minmax", 0.0, 4.0 * (double)in_vox, st);
       hipLaunchKernelGGL(plane_minmax_kernel, dim3((unsigned)planes, kMinmaxParts), dim3(256), 0,
                          st, xc, size[0], size[1], size[2], mm_axis, part);
       hipLaunchKernelGGL(plane_parts_kernel, dim3((unsigned)ceil_div(planes, 256)), dim3(256), 0,
-                         st, part, planes, kMinmaxParts, mm);
+                         st, part, planes, kMinmaxParts, spread, extrema, mm);
       if (separate_axis < 0)
-        hipLaunchKernelGGL(reduce_minmax_kernel, dim3(1), dim3(64), 0, st, mm, size[0]);
+        hipLaunchKernelGGL(reduce_minmax_kernel, dim3(1), dim3(64), 0, st, extrema, planes, spread,
+                           mm + planes);
     }
     float* oc = out + (int64_t)c * out_vox;
     if (order == 3) {

@@ -169,6 +169,41 @@ def test_resample_spline_pieces(lib, shape, new_shape, axis):
     assert_one_rounding(got, want)
 
 
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf], ids=str)
+@pytest.mark.parametrize("shape,new_shape,axis", [
+    ((1, 130, 70, 9), (100, 90, 12), -1), ((1, 3, 70, 900), (5, 60, 1000), -1),
+    ((2, 5, 70, 900), (9, 90, 800), 0), ((1, 130, 4, 700), (150, 9, 650), 1),
+    ((1, 130, 70, 4), (150, 60, 7), 2), ((1, 1, 1, 1), (3, 1, 5), -1),
+], ids=str)
+def test_resample_spline_nonfinite_lines(lib, shape, new_shape, axis, bad):
+    """Order 3: one NaN or infinity makes every value of its volume (of its plane, along a
+    separate axis) NaN, as the recursions carry it over whole lines axis by axis, and the clip
+    makes the lower bound of each, which ignores NaN; planes without one are not touched.  Lines
+    of several pieces, the sample in the first, a middle and the last."""
+    rng = np.random.default_rng(shape[1])
+    data = (rng.standard_normal(shape) * 3).astype(np.float32)
+    clean = spline_device(lib, data, new_shape, 3, axis)
+    size = shape[1:]
+    for at in ((0, 0, 0), tuple(n // 2 for n in size), tuple(n - 1 for n in size)):
+        print(f"spline nonfinite {shape} -> {new_shape} axis {axis} {bad} at {at}", flush=True)
+        planted = data.copy()
+        planted[(0, *at)] = bad
+        got = spline_device(lib, planted, new_shape, 3, axis)
+        want = clean.copy()
+        if axis < 0:
+            where, source = slice(None), planted[0]
+        else:
+            o = np.arange(new_shape[axis])
+            nearest = np.floor(size[axis] / new_shape[axis] * (o + 0.5) - 0.5 + 0.5)
+            hit = np.clip(nearest.astype(int), 0, size[axis] - 1) == at[axis]
+            where = (slice(None),) * axis + (hit,)
+            source = np.take(planted[0], at[axis], axis)
+        # all NaN: the bounds of an empty reduction, of which the clip makes -inf
+        finite = source[~np.isnan(source)]
+        want[0][where] = finite.min() if finite.size else -np.inf
+        np.testing.assert_array_equal(got, want)
+
+
 def test_crop_normalize_long_rows(lib):
     """Rows past one round of eight loads a lane, in each order of the axes."""
     raw = (np.random.default_rng(2).standard_normal((1, 3, 2, 1030)) * 9).astype(np.float32)
