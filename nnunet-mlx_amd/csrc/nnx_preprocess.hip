@@ -306,51 +306,133 @@ __global__ __launch_bounds__(64) void zscore_final_kernel(const double2* __restr
   }
 }
 
+// A channel's normalisation.  `inside` (whether the filled mask is set at the value) is asked for by
+// the masked scheme only.
+struct ChannelNorm {
+  int scheme;
+  float mean, std, lower, upper;
+  __device__ ChannelNorm(const ChannelNorms& n, int c)
+      : scheme(n.scheme[c]), mean(n.mean[c]), std(n.std[c]), lower(n.lower[c]), upper(n.upper[c]) {}
+  template <class F>
+  __device__ __forceinline__ float operator()(float v, F&& inside) const {
+    if (scheme == NNX_NORM_CT) {
+      v = fminf(fmaxf(v, lower), upper);
+      v = __fdiv_rn(__fsub_rn(v, mean), std);
+    } else if (scheme == NNX_NORM_ZSCORE || (scheme == NNX_NORM_ZSCORE_MASKED && inside())) {
+      v = __fdiv_rn(__fsub_rn(v, mean), std);
+    }
+    return v;
+  }
+};
+
 // out[c][o0][o1][o2] = norm_c(x[c][r0][r1][r2]) with r[t_k] = s_k + o_k: out axis k is input
 // axis t_k, cropped to start s_k.  NNX_NORM_ZSCORE_MASKED normalises only where the filled
-// mask (raw-order box starting at (m0, m1, m2), extents (*, ME1, ME2)) is set.
-__global__ __launch_bounds__(256) void crop_normalize_kernel(
-    const float* __restrict__ x, int C, int64_t X, int64_t Y, int64_t Z, int t0, int t1, int t2,
-    int64_t s0, int64_t s1, int64_t s2, int64_t O0, int64_t O1, int64_t O2, ChannelNorms norms,
-    const uint8_t* __restrict__ mask, int64_t m0, int64_t m1, int64_t m2, int64_t ME1,
-    int64_t ME2, float* __restrict__ out) {
-  // a wave a row of out axis 2 at a time: the index arithmetic is per row
+// mask (a box of the raw axes) is set.  `in` and `mask` point at the window's first voxel of
+// channel 0; strides by out axis.
+struct CropArgs {
+  const float* in;
+  const uint8_t* mask;
+  float* out;
+  int channels;
+  int64_t in_channel;
+  int64_t n[3], in_stride[3], mask_stride[3];
+  ChannelNorms norms;
+};
+
+// A thread a voxel, for short rows: in 8 M voxels 34 us whatever their length (the index
+// arithmetic bounds it), where a wave a row takes 377 us at 8 voxels, 37 at 64, 35 at 72, 31 at
+// 80, 22 at 128 and 12 at 512 (5.2 TB/s).
+__global__ __launch_bounds__(256) void crop_normalize_kernel(CropArgs a) {
+  const int64_t per = a.n[0] * a.n[1] * a.n[2];
+  const int64_t total = per * a.channels;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
+       e += (int64_t)gridDim.x * blockDim.x) {
+    const int c = (int)(e / per);
+    const int64_t p = e - c * per;
+    const int64_t o2 = p % a.n[2], o1 = (p / a.n[2]) % a.n[1], o0 = p / (a.n[1] * a.n[2]);
+    const float v = a.in[c * a.in_channel + o0 * a.in_stride[0] + o1 * a.in_stride[1] + o2 * a.in_stride[2]];
+    a.out[e] = ChannelNorm(a.norms, c)(v, [&] {
+      return a.mask[o0 * a.mask_stride[0] + o1 * a.mask_stride[1] + o2 * a.mask_stride[2]] != 0;
+    });
+  }
+}
+
+// Rows of kRowForm voxels and more that are contiguous on both sides, a wave a row at a time: the
+// index arithmetic is per row, and eight loads of a lane are in flight.
+constexpr int64_t kRowForm = 80;
+
+__global__ __launch_bounds__(256) void crop_normalize_rows_kernel(CropArgs a) {
   const int lane = threadIdx.x & 63;
-  const int64_t rows = O0 * O1 * C;
-  const int64_t stride2 = t2 == 0 ? Y * Z : t2 == 1 ? Z : 1;
-  const int64_t mstride2 = t2 == 0 ? ME1 * ME2 : t2 == 1 ? ME2 : 1;
+  const int64_t n2 = a.n[2], rows = a.n[0] * a.n[1] * a.channels;
   for (int64_t r = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6); r < rows;
        r += (int64_t)gridDim.x * 4) {
-    const int64_t o1 = r % O1, rest = r / O1;
-    const int64_t o0 = rest % O0;
-    const int c = (int)(rest / O0);
-    const int64_t a0 = s0 + o0, a1 = s1 + o1, a2 = s2;
-    const int64_t r0 = t0 == 0 ? a0 : t1 == 0 ? a1 : a2;
-    const int64_t r1 = t0 == 1 ? a0 : t1 == 1 ? a1 : a2;
-    const int64_t r2 = t0 == 2 ? a0 : t1 == 2 ? a1 : a2;
-    const float* src = x + (int64_t)c * X * Y * Z + (r0 * Y + r1) * Z + r2;
-    const uint8_t* msrc = mask ? mask + ((r0 - m0) * ME1 + (r1 - m1)) * ME2 + (r2 - m2) : nullptr;
-    float* dst = out + r * O2;
-    const int scheme = norms.scheme[c];
-    const float lower = norms.lower[c], upper = norms.upper[c];
-    const float mean = norms.mean[c], std = norms.std[c];
-    for (int64_t o = lane; o < O2; o += 8 * 64) {
+    const int64_t o1 = r % a.n[1], rest = r / a.n[1];
+    const int64_t o0 = rest % a.n[0];
+    const int c = (int)(rest / a.n[0]);
+    const float* src = a.in + c * a.in_channel + o0 * a.in_stride[0] + o1 * a.in_stride[1];
+    const uint8_t* msrc = a.mask + o0 * a.mask_stride[0] + o1 * a.mask_stride[1];
+    float* dst = a.out + r * n2;
+    const ChannelNorm norm(a.norms, c);
+    for (int64_t o = lane; o < n2; o += 8 * 64) {
       float v[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = src[(o + j * 64 < O2 ? o + j * 64 : o) * stride2];
+      for (int j = 0; j < 8; ++j) v[j] = src[o + j * 64 < n2 ? o + j * 64 : o];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int64_t oj = o + j * 64;
-        if (oj >= O2) break;
-        if (scheme == NNX_NORM_CT) {
-          v[j] = fminf(fmaxf(v[j], lower), upper);
-          v[j] = __fdiv_rn(__fsub_rn(v[j], mean), std);
-        } else if (scheme == NNX_NORM_ZSCORE ||
-                   (scheme == NNX_NORM_ZSCORE_MASKED && msrc[oj * mstride2])) {
-          v[j] = __fdiv_rn(__fsub_rn(v[j], mean), std);
-        }
-        dst[oj] = v[j];
+        if (oj >= n2) break;
+        dst[oj] = norm(v[j], [&] { return msrc[oj] != 0; });
       }
+    }
+  }
+}
+
+// Transposed rows: the raw rows are out axis A (0 or 1).  A workgroup moves tiles of TA voxels of it
+// by 64 of out axis 2 through LDS, read along the one and written along the other (TA = 64, or
+// the next power of two from 16 on that holds a short axis).  Bound by HBM: 160 x 512 x 512 with
+// its axes in reverse 74 us (4.5 TB/s), where reads that stride over the raw rows took 212 us (a
+// thread a voxel) and 468 (a wave a row), both at the mercy of the caches; 40 x 512 x 512 likewise
+// 24, 54 and 163 us.  Out rows below kTileForm voxels fill too little of a tile's 64: 700 x 16 x
+// 700 to rows of 16, 40 us against 35 a thread a voxel, of 20, 40 against 43.
+constexpr int64_t kTileForm = 20;
+
+template <int A, int TA>
+__global__ __launch_bounds__(256) void crop_normalize_tiles_kernel(CropArgs a) {
+  constexpr int B = 1 - A, kPer = TA * 64 / 256;
+  __shared__ float tile[64][TA + 1];
+  const int64_t na = a.n[A], nb = a.n[B], n2 = a.n[2];
+  const int64_t ta = (na + TA - 1) / TA, t2 = (n2 + 63) / 64, total = ta * t2 * nb * a.channels;
+  const int64_t out_stride[2] = {a.n[1] * n2, n2};
+  for (int64_t t = blockIdx.x; t < total; t += gridDim.x) {
+    const int64_t a0 = t % ta * TA, rest = t / ta;
+    const int64_t j0 = rest % t2 * 64, plane = rest / t2;
+    const int64_t b = plane % nb;
+    const int c = (int)(plane / nb);
+    const float* src = a.in + c * a.in_channel + b * a.in_stride[B];
+    const uint8_t* msrc = a.mask + b * a.mask_stride[B];
+    const ChannelNorm norm(a.norms, c);
+    float v[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int l = i * 256 + (int)threadIdx.x;
+      v[i] = src[min(a0 + l % TA, na - 1) + min(j0 + l / TA, n2 - 1) * a.in_stride[2]];
+    }
+    __syncthreads();  // the last tile is read
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int l = i * 256 + (int)threadIdx.x;
+      tile[l / TA][l % TA] = norm(v[i], [&] {
+        return msrc[min(a0 + l % TA, na - 1) + min(j0 + l / TA, n2 - 1) * a.mask_stride[2]] != 0;
+      });
+    }
+    __syncthreads();
+    float* dst = a.out + c * (a.n[0] * a.n[1] * n2) + b * out_stride[B];
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int la = i * 4 + (int)(threadIdx.x >> 6);
+      if (a0 + la < na && j0 + lane < n2)
+        dst[(a0 + la) * out_stride[A] + j0 + lane] = tile[lane][la];
     }
   }
 }
@@ -1168,11 +1250,41 @@ void crop_normalize_masked(const float* x, int channels, const int64_t* size,
   }
   const int64_t total = out_size[0] * out_size[1] * out_size[2] * channels;
   ProfScope prof("preprocess_crop_normalize", 0.0, 8.0 * (double)total, st);
-  hipLaunchKernelGGL(crop_normalize_kernel, dim3(blocks_for(64 * ceil_div(total, out_size[2]))),
-                     dim3(256), 0, st, x,
-                     channels, size[0], size[1], size[2], transpose[0], transpose[1], transpose[2],
-                     start[0], start[1], start[2], out_size[0], out_size[1], out_size[2], cn,
-                     masked ? mask : nullptr, ms[0], ms[1], ms[2], me[1], me[2], out);
+  CropArgs a{};
+  a.out = out;
+  a.channels = channels;
+  a.in_channel = size[0] * size[1] * size[2];
+  a.norms = cn;
+  const int64_t in_strides[3] = {size[1] * size[2], size[2], 1};
+  const int64_t mask_strides[3] = {me[1] * me[2], me[2], 1};
+  int64_t first = 0, mask_first = 0;
+  for (int k = 0; k < 3; ++k) {
+    a.n[k] = out_size[k];
+    a.in_stride[k] = in_strides[transpose[k]];
+    a.mask_stride[k] = mask_strides[transpose[k]];
+    first += start[k] * a.in_stride[k];
+    mask_first += (start[k] - ms[transpose[k]]) * a.mask_stride[k];
+  }
+  a.in = x + first;
+  a.mask = masked ? mask + mask_first : nullptr;
+  if (transpose[2] != 2 && out_size[2] >= kTileForm) {
+    const int along = transpose[0] == 2 ? 0 : 1;
+    const int64_t n = a.n[along];
+    const int tile = n > 32 ? 64 : n > 16 ? 32 : 16;
+    const int64_t tiles = ceil_div(n, tile) * ceil_div(a.n[2], 64) * a.n[1 - along] * channels;
+    auto kernel = along == 0 ? (tile == 64 ? crop_normalize_tiles_kernel<0, 64>
+                                : tile == 32 ? crop_normalize_tiles_kernel<0, 32>
+                                             : crop_normalize_tiles_kernel<0, 16>)
+                             : (tile == 64 ? crop_normalize_tiles_kernel<1, 64>
+                                : tile == 32 ? crop_normalize_tiles_kernel<1, 32>
+                                             : crop_normalize_tiles_kernel<1, 16>);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)std::min<int64_t>(tiles, 1 << 20)), dim3(256), 0, st, a);
+  } else if (transpose[2] == 2 && out_size[2] >= kRowForm) {
+    hipLaunchKernelGGL(crop_normalize_rows_kernel, dim3(blocks_for(64 * (total / out_size[2]))),
+                       dim3(256), 0, st, a);
+  } else {
+    hipLaunchKernelGGL(crop_normalize_kernel, dim3(blocks_for(total)), dim3(256), 0, st, a);
+  }
   launch_check("crop_normalize");
 }
 

@@ -204,6 +204,45 @@ def test_resample_spline_nonfinite_lines(lib, shape, new_shape, axis, bad):
         np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("out_size", [
+    (3, 4, 79), (3, 4, 80), (2, 3, 513),                 # the least row with a wave of its own
+    (70, 5, 19), (70, 5, 20), (16, 3, 64), (17, 3, 65),  # tiles of 64, 32 and 16 of axis 0 or 1,
+    (5, 33, 64), (65, 64, 130), (64, 2, 63), (9, 130, 21)], ids=str)
+@pytest.mark.parametrize("transpose", list(itertools.permutations(range(3))))
+def test_crop_normalize_forms(lib, transpose, out_size):
+    """The row, tile and voxel forms at the edges of their ranges and of their tiles, bit for bit:
+    a window off every corner of the volume, CT, masked z-score and no normalisation, the mask
+    over a box that is larger than the window."""
+    print(f"crop/normalise {transpose} -> {out_size}", flush=True)
+    rng = np.random.default_rng(out_size[2])
+    start = (1, 2, 3)
+    tshape = tuple(s + n + 1 for s, n in zip(start, out_size))
+    shape = tuple(tshape[transpose.index(a)] for a in range(3))
+    raw = (rng.standard_normal((3, *shape)) * 900).astype(np.float32)
+    mask = rng.integers(0, 2, tuple(n - 1 for n in shape)).astype(np.uint8)
+    norm = np.array([[41.5, 60.25, -1000.0, 1500.0], [3.25, 7.5, 0, 0], [0] * 4], dtype=np.float32)
+    schemes = [_native.NNX_NORM_CT, _native.NNX_NORM_ZSCORE_MASKED, _native.NNX_NORM_NONE]
+    out = torch.full((3, *out_size), float("nan"), device="cuda")
+    dmask = torch.from_numpy(mask).cuda()
+    _native.check(lib.nnx_crop_normalize_masked(
+        dev(raw).data_ptr(), 3, _native.i64s(shape), _native.ints(transpose),
+        _native.i64s(start), _native.i64s(out_size), _native.ints(schemes),
+        norm.ctypes.data_as(ctypes.POINTER(ctypes.c_float)), dmask.data_ptr(),
+        _native.i64s((1, 1, 1)), _native.i64s(mask.shape), out.data_ptr(), stream()))
+    got = out.cpu().numpy()
+
+    def window(a, first):
+        return a.transpose(transpose)[tuple(slice(s - f, s - f + n)
+                                            for s, f, n in zip(start, first, out_size))]
+
+    crop = [window(c, (0, 0, 0)) for c in raw]
+    inside = window(mask, (1, 1, 1)) != 0
+    zscore = (crop[1] - np.float32(3.25)) / np.float32(7.5)
+    np.testing.assert_array_equal(got[0], op.ct_normalize(crop[0], 41.5, 60.25, -1000.0, 1500.0))
+    np.testing.assert_array_equal(got[1], np.where(inside, zscore, crop[1]))
+    np.testing.assert_array_equal(got[2], crop[2])
+
+
 def test_crop_normalize_long_rows(lib):
     """Rows past one round of eight loads a lane, in each order of the axes."""
     raw = (np.random.default_rng(2).standard_normal((1, 3, 2, 1030)) * 9).astype(np.float32)
