@@ -43,6 +43,9 @@ def sparse_volume(rng, shape, boxes):
     ((1, 9, 10, 11), [(0, ((2, 3, 4), (5, 9, 6)))]),
     ((2, 17, 5, 33), [(0, ((0, 1, 30), (3, 2, 33))), (1, ((10, 0, 2), (17, 4, 3)))]),
     ((3, 64, 48, 40), [(2, ((1, 1, 1), (63, 47, 39)))]),
+    ((2, 300, 303, 3), [(1, ((7, 5, 1), (299, 294, 2)))]),  # more short rows than loads in flight
+    ((1, 5, 7, 64), [(0, ((1, 2, 0), (4, 6, 1))), (0, ((2, 3, 63), (3, 5, 64)))]),
+    ((1, 5, 7, 65), [(0, ((4, 6, 64), (5, 7, 65)))]),
 ])
 def test_nonzero_bbox(lib, shape, boxes):
     print(f"bbox case {shape}", flush=True)
