@@ -2617,6 +2617,16 @@ int conv_x3_stats_tiles(const ConvGeom& g, int cout, int c1, int c2, int arith) 
   return (int)(ceil_div(g.out[0], box.z) * ceil_div(g.out[1], box.y) * ceil_div(g.out[2], box.x));
 }
 
+int conv_x3_stats_room(const ConvGeom& g, int cout, int c1, int c2, int arith) {
+  const Box box = plan_x3(g, cout).box;
+  int64_t room = ceil_div(g.out[0], box.z) * ceil_div(g.out[1], box.y) * ceil_div(g.out[2], box.x);
+  if (arith == kBf16 && conv_bf16_direct_packed(g.k, c1, c2, cout))
+    room = std::max<int64_t>(room, conv_bf16_direct_stats_tiles(g));
+  if (conv_strided_layer(g, c1, c2, cout))
+    room = std::max<int64_t>(room, conv_strided_stats_tiles(g));
+  return (int)room;
+}
+
 // The register-staged (strided) kernel's layers with less than a workgroup a CU: chunks split over
 // the idle CUs (two workgroups a CU), at least four (8 channels each) a workgroup.
 int conv_x3_splits(const ConvGeom& g, int c1, int c2, int cout, int arith) {

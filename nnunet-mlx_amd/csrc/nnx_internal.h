@@ -149,6 +149,9 @@ void conv3d_x3(const float* x1, int c1, const float* x2, int c2, const void* pac
                hipStream_t st, float4* stats = nullptr, const PendingNorm& n1 = {},
                const PendingNorm& n2 = {}, int arith = kArithSplit3, int splits = 1);
 int conv_x3_stats_tiles(const ConvGeom& g, int cout, int c1, int c2, int arith);
+// *_stats_room: partials per item that suffice for g and for every smaller batch or volume, whose
+// kernels and boxes may differ.
+int conv_x3_stats_room(const ConvGeom& g, int cout, int c1, int c2, int arith);
 
 // Compute units of the current device, a multiple of the 8 XCDs (the persistent kernels' grid).
 int compute_units();
@@ -170,6 +173,7 @@ void conv3d_bf16_direct(const float* x1, int c1, const float* x2, int c2, const 
 // route of conv3d_x3 on its packed words (nblk16 = their 16-column blocks).
 bool conv_strided_supported(const ConvGeom& g, int c1, int c2, int cout);
 int conv_strided_stats_tiles(const ConvGeom& g);
+bool conv_strided_layer(const ConvGeom& g, int c1, int c2, int cout);  // supported at some size
 int conv_strided_splits(const ConvGeom& g, int c1, int c2, int cout);
 void conv3d_strided(const float* x1, int c1, const float* x2, int c2, const void* packed,
                     int nblk16, float scale, const float* bias, float* y, const ConvGeom& g,
@@ -183,6 +187,7 @@ void conv3d_strided(const float* x1, int c1, const float* x2, int c2, const void
 // tiles = conv_wino_stats_tiles (the output boxes of an item).
 bool conv_wino_supported(const ConvGeom& g, int c1, int c2, int cout);
 int conv_wino_stats_tiles(const ConvGeom& g, int cout);
+int conv_wino_stats_room(const ConvGeom& g);
 float wino_weight_scale(float max_abs);
 int64_t conv_wino_packed_bytes(int cout, int c1, int c2);
 void conv_wino_pack_weight(const float* d_w, int cout, int c1, int c2, float scale,
@@ -198,6 +203,9 @@ void conv3d_wino(const float* x1, int c1, const float* x2, int c2, const void* p
 int conv_wino_splits(const ConvGeom& g, int c1, int c2, int cout);
 int conv_x3_splits(const ConvGeom& g, int c1, int c2, int cout, int arith);
 bool split_sum_supported(int64_t spatial, int channels);
+// Bytes of the partial results of any split layer: a split fills at most the CUs once with
+// 32-column Winograd boxes of 512 voxels, or twice with 64 x 64 or 64 x 128 tiles.
+inline size_t split_sum_room() { return (size_t)compute_units() * 32 * 512 * sizeof(float); }
 int split_sum_parts(int64_t spatial);  // rows of `stats` an item (used where more than one)
 void split_sum(const float* partial, int splits, int batch, int64_t spatial, int channels,
                const float* bias, const float* gamma, const float* beta, float eps, float* y,

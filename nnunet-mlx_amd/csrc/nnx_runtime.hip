@@ -532,17 +532,23 @@ struct Runner {
     // Implicit GEMM: the epilogue writes per-tile statistics, so the norm never re-reads the
     // tensor for them.
     const ConvGeom g = make_conv_geom(n, in.d, c.k, c.s);
+    if (plan->planning) {
+      // room for the smaller batches and volumes that may follow too: they never allocate
+      const int room = c.wino    ? conv_wino_stats_room(g)
+                       : c.split ? conv_x3_stats_room(g, c.cout, c.cin1, c.cin2, c.arith)
+                                 : conv_stats_tiles(g, c.cout, c.cin1, c.cin2);
+      plan->stats = std::max(plan->stats, (size_t)n * room * c.cout * sizeof(float4));
+      if (c.wino || c.split) plan->split = split_sum_room();
+      return result;
+    }
     const int splits = c.wino    ? conv_wino_splits(g, c.cin1, c.cin2, c.cout)
                        : c.split ? conv_x3_splits(g, c.cin1, c.cin2, c.cout, c.arith)
                                  : 1;
     if (splits > 1) {
       // a layer too small for the chip: its input channels over several workgroups, then one
       // kernel for the sum, the bias and the norm parameters
-      if (plan->planning) {
-        plan->split = std::max(plan->split, (size_t)splits * n * vox * c.cout * sizeof(float));
-        plan->stats = std::max(plan->stats, (size_t)n * split_sum_parts(vox) * c.cout * sizeof(float4));
-        return result;
-      }
+      require((size_t)splits * n * vox * c.cout * sizeof(float) <= plan->ws->split.bytes,
+              "split convolution workspace too small");
       float* partial = plan->ws->split.as<float>();
       if (c.wino)
         conv3d_wino(x1.data, c.cin1, x2.data, c.cin2, c.packed.ptr, c.scale, nullptr, partial, g,
@@ -562,10 +568,8 @@ struct Runner {
     const int tiles = c.wino    ? conv_wino_stats_tiles(g, c.cout)
                       : c.split ? conv_x3_stats_tiles(g, c.cout, c.cin1, c.cin2, c.arith)
                                 : conv_stats_tiles(g, c.cout, c.cin1, c.cin2);
-    if (plan->planning) {
-      plan->stats = std::max(plan->stats, (size_t)n * tiles * c.cout * sizeof(float4));
-      return result;
-    }
+    require((size_t)n * tiles * c.cout * sizeof(float4) <= plan->ws->stats_bytes,
+            "convolution statistics workspace too small");
     float4* stats = plan->ws->stats.as<float4>();
     if (c.wino)
       conv3d_wino(x1.data, c.cin1, x2.data, c.cin2, c.packed.ptr, c.scale, pdev(m, c.pb), out, g,

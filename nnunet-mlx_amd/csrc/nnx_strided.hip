@@ -443,6 +443,10 @@ bool conv_strided_supported(const ConvGeom& g, int c1, int c2, int cout) {
   if (cout > 64 && (int64_t)g.batch * conv_strided_stats_tiles(g) * ceil_div(cout, 64) >=
                        6 * (int64_t)compute_units())
     return false;
+  return conv_strided_layer(g, c1, c2, cout);
+}
+
+bool conv_strided_layer(const ConvGeom& g, int c1, int c2, int cout) {
   for (int i = 0; i < 3; ++i)
     if (g.k[i] != 3) return false;
   return (g.s[0] == 1 || g.s[0] == 2) && g.s[1] == 2 && g.s[2] == 2 && c1 > 0 && c1 % kSChunk == 0 &&

@@ -689,6 +689,16 @@ struct WinoPlan {
   int nbz, nby, nbx;
 };
 
+// Every box: planes of a slab, shape, voxels a side and cost.
+template <class F>
+void wino_boxes(F&& f) {
+  f(4, kWide, 4, 8, 16, 10);
+  f(4, kTall, 4, 16, 8, 10);
+  f(2, kWide, 2, 8, 16, 6);
+  f(2, kTall, 2, 16, 8, 6);
+  f(2, kCube, 4, 8, 8, 6);
+}
+
 // The shape that needs the least time by rounds of boxes over the CUs: a box of four planes
 // takes 1 of it, one of two planes 0.6 (320 -> 320: 4.8 and 2.9 us a 16-channel chunk), so the
 // small boxes win where they fill CUs that would stand idle: 320 -> 320 on 8^3 x 8 95.6 us in
@@ -706,11 +716,7 @@ WinoPlan wino_plan(const ConvGeom& g, int cout) {
     best_cost = total;
     best = WinoPlan{zb, shape, (int)nbz, (int)nby, (int)nbx};
   };
-  consider(4, kWide, 4, 8, 16, 10);
-  consider(4, kTall, 4, 16, 8, 10);
-  consider(2, kWide, 2, 8, 16, 6);
-  consider(2, kTall, 2, 16, 8, 6);
-  consider(2, kCube, 4, 8, 8, 6);
+  wino_boxes(consider);
   return best;
 }
 
@@ -758,6 +764,14 @@ int conv_wino_splits(const ConvGeom& g, int c1, int c2, int cout) {
 int conv_wino_stats_tiles(const ConvGeom& g, int cout) {
   const WinoPlan p = wino_plan(g, cout);
   return p.nbz * p.nby * p.nbx;
+}
+
+int conv_wino_stats_room(const ConvGeom& g) {
+  int64_t room = 0;
+  wino_boxes([&](int, WinoShape, int bz, int by, int bx, int64_t) {
+    room = std::max(room, ceil_div(g.out[0], bz) * ceil_div(g.out[1], by) * ceil_div(g.out[2], bx));
+  });
+  return (int)room;
 }
 
 float wino_weight_scale(float max_abs) {

@@ -237,6 +237,32 @@ def test_split_layers_match_oracle(device, patch):
     assert np.abs(got - ref).max() <= 1e-3 and rel_l2(got, ref) <= 1e-5, msg
 
 
+@pytest.mark.parametrize("precision", ["fp32-split", "bf16"])
+def test_smaller_forwards_allocate_nothing(device, precision):
+    """Whatever kernels, boxes and splits the smaller batches and volumes take, the buffers of the
+    largest forward hold them (a forward that is recorded into a graph cannot allocate)."""
+    spec = PlainConvUNetSpec(1, 3, (32, 64, 256, 320), K3 * 4, ((1, 1, 1),) + ((2, 2, 2),) * 3,
+                             (2,) * 4, (2,) * 3)
+    net = build_network(spec, precision=precision)
+    net.load_weights(random_weights(spec, seed=17, random_affine=True))
+
+    def forward(n, *size):
+        x = torch.zeros((n, *size, 1), device=device)
+        out = torch.empty((n, *size, 3), device=device)
+        net.forward_into(x, out)
+        torch.cuda.synchronize()
+        del x, out
+        torch.cuda.empty_cache()
+        return torch.cuda.mem_get_info()[0]
+
+    free = forward(16, 64, 64, 64)
+    for shape in ((8, 64, 64, 64), (3, 64, 64, 64), (1, 64, 64, 64), (16, 32, 40, 24), (2, 32, 32, 32),
+                  (1, 56, 64, 16), (1, 8, 8, 8)):
+        print(f"smaller forward {precision} {shape}", flush=True)
+        assert forward(*shape) == free, shape
+    net.close()
+
+
 def test_persistent_winograd_forward_is_bit_identical(device, monkeypatch):
     """The persistent Winograd kernel runs the layers with at least four boxes a CU (here
     the 64^3 and 32^3 stages at batch 4) with the one-box kernel's arithmetic, including
