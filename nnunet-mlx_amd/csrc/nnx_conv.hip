@@ -2652,6 +2652,8 @@ void conv3d_x3(const float* x1, int c1, const float* x2, int c2, const void* pac
   require(c1 >= 1 && (c2 == 0 || x2), "invalid convolution inputs");
   require(scale > 0.f && std::isfinite(scale), "weight scale must be positive");
   require(arith == kSplit3 || arith == kBf16, "unknown convolution arithmetic");
+  require(!(n1.params && n2.params) || n1.slope == n2.slope,
+          "pending normalisations of one convolution must share the LeakyReLU slope");
   // (its 16-byte lines need aligned tensors, as every activation of a model is)
   const uintptr_t ends = reinterpret_cast<uintptr_t>(x1) | reinterpret_cast<uintptr_t>(x2) |
                          reinterpret_cast<uintptr_t>(y);

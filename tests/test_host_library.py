@@ -296,3 +296,54 @@ def test_finalize_failed_part_way_leaves_the_model_refusing_retries():
         assert b"failed part-way" in lib.nnx_last_error()
     finally:
         lib.nnx_model_destroy(handle)
+
+
+_SLOPES_PROGRAM = r"""
+#include "nnx_internal.h"
+int main() {
+  alignas(16) static char buffer[64];
+  float* p = reinterpret_cast<float*>(buffer);
+  nnx::PendingNorm a{reinterpret_cast<float4*>(p), true, 0.01f}, b = a;
+  b.slope = 0.2f;
+  const int size[3] = {8, 8, 8}, k[3] = {3, 3, 3}, flat[3] = {1, 3, 3};
+  const int one[3] = {1, 1, 1}, two[3] = {2, 2, 2};
+  int refused = 0;
+  auto run = [&](const int* kernel, const int* stride, int arith) {
+    try {
+      nnx::conv3d_x3(p, 32, p, 32, p, 1.f, nullptr, p, nnx::make_conv_geom(1, size, kernel, stride),
+                     64, nullptr, nullptr, a, b, arith);
+    } catch (const nnx::Error& e) {
+      std::printf("%s\n", e.what());
+      refused += std::string(e.what()).find("slope") != std::string::npos;
+    }
+  };
+  run(k, one, nnx::kArithBf16);      // the direct bf16 kernel
+  run(k, two, nnx::kArithBf16);      // the strided kernel
+  run(k, two, nnx::kArithSplit3);
+  run(flat, one, nnx::kArithSplit3);  // the implicit GEMM
+  return refused == 4 ? 0 : 1;
+}
+"""
+
+
+def test_every_split_route_refuses_two_slopes(tmp_path):
+    """Two pending normalisations of one convolution share the LeakyReLU slope on every route
+    behind conv3d_x3: refused before any device call, so on a host without a GPU the message
+    is this one and not that of the first device query."""
+    import subprocess
+
+    import torch
+
+    from nnunet_mlx import _native
+
+    if torch.cuda.is_available():
+        pytest.skip("a route without the check would launch on the program's host pointers")
+    source, program = tmp_path / "slopes.cpp", tmp_path / "slopes"
+    source.write_text(_SLOPES_PROGRAM)
+    lib = _native.library_path()
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    f"-I{ROOT / 'nnunet-mlx_amd' / 'csrc'}", str(source), str(lib),
+                    "-L/opt/rocm/lib", "-lamdhip64", f"-Wl,-rpath,{lib.parent}:/opt/rocm/lib",
+                    "-o", str(program)], check=True, timeout=120)
+    run = subprocess.run([str(program)], capture_output=True, text=True, timeout=120)
+    assert run.returncode == 0, run.stdout + run.stderr
