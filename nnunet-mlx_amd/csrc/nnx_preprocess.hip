@@ -1029,6 +1029,11 @@ SplinePlan spline_plan(const int64_t* size, const int64_t* new_size, int separat
   return p;
 }
 
+// Bytes of the two volumes, up to the alignment of what follows.
+int64_t volume_bytes(const SplinePlan& p) {
+  return ceil_div((p.a_elems + p.b_elems) * (int64_t)sizeof(double), 256) * 256;
+}
+
 // Bytes of the bounds and the extrema behind them, up to the tables' alignment.
 int64_t bounds_bytes(const SplinePlan& p) {
   return ceil_div(p.mm_elems * (int64_t)sizeof(float2) + p.extrema * (int64_t)sizeof(Extrema), 256) * 256;
@@ -1320,7 +1325,7 @@ void crop_normalize_masked(const float* x, int channels, const int64_t* size,
 size_t resample_spline_workspace(const int64_t* size, const int64_t* new_size, int separate_axis) {
   const SplinePlan p = spline_plan(size, new_size, separate_axis);
   const int64_t planes = separate_axis >= 0 ? p.n[separate_axis] : 0;
-  return (size_t)(p.a_elems + p.b_elems) * sizeof(double) + (size_t)bounds_bytes(p) +
+  return (size_t)volume_bytes(p) + (size_t)bounds_bytes(p) +
          (size_t)tap_count(p) * sizeof(SplineTap) + (size_t)planes * sizeof(longlong2) + 1024;
 }
 
@@ -1340,7 +1345,8 @@ void resample_spline(const float* x, int channels, const int64_t* size, const in
           "resampling workspace too small");
   double* A = static_cast<double*>(work);
   double* B = A + p.a_elems;
-  float2* mm = reinterpret_cast<float2*>(B + p.b_elems);
+  // (the tables behind hold 16-byte values, and the volumes may be an odd number of doubles)
+  float2* mm = reinterpret_cast<float2*>(static_cast<char*>(work) + volume_bytes(p));
   const int64_t in_vox = size[0] * size[1] * size[2];
   const int64_t out_vox = new_size[0] * new_size[1] * new_size[2];
   Extrema* extrema = reinterpret_cast<Extrema*>(mm + p.mm_elems);

@@ -162,6 +162,7 @@ def test_resample_spline_separate_axis(lib, axis):
     ((1, 3, 5, 1240), (7, 4, 300), 0),       # three row tiles, downsampled
     ((1, 1, 1, 1), (3, 1, 5), -1),           # one sample a line
     ((1, 130, 5, 4), (31, 9, 3), 1),         # separate middle axis
+    ((1, 3, 5, 7), (4, 7, 9), 1),            # an odd number of doubles before the tables
 ], ids=str)
 def test_resample_spline_pieces(lib, shape, new_shape, axis):
     """Order 3 at the edges of the pieces that a line is cut into."""
