@@ -373,13 +373,17 @@ int nnx_torch_resize_argmax(const void* d_logits, int half, int classes, const i
  * nnx_resample_spline does (order 1 or 3, separate_axis -1 or 0..2), rounded once to
  * float32 — or to float16 when half != 0 (float16 logits) — and folded into a
  * first-maximum argmax (strict ">", ties keep the earliest class) written as uint16 labels.
- * One class at a time through a device workspace of
- * nnx_restore_labels_spline_workspace bytes (0 = invalid shapes).  Replaces the host
+ * Order 1 forms every class of a voxel in one pass, order 3 takes one class at a time.  The
+ * device workspace is nnx_restore_labels_spline_order_workspace bytes for its order, or
+ * nnx_restore_labels_spline_workspace for either (0 = invalid arguments); for 300 x 534 x 534
+ * to 120 x 512 x 512 the first asks 0.47 GB at order 1, the second 2.0 GB.  Replaces the host
  * restoration resample_class_logits_argmax_parallel / separate_plane_argmax
  * (src/nnunet_mlx/prediction/restore.py:28-158) over resample_probabilities_or_data
  * (src/nnunet_mlx/data/resampling.py:87-172). */
 size_t nnx_restore_labels_spline_workspace(const int* src_shape, const int* dst_shape,
                                            int separate_axis);
+size_t nnx_restore_labels_spline_order_workspace(const int* src_shape, const int* dst_shape,
+                                                 int order, int separate_axis);
 int nnx_restore_labels_spline(const void* d_logits, int half, int classes, const int* src_shape,
                               const int* dst_shape, int order, int separate_axis, void* d_work,
                               size_t work_bytes, uint16_t* d_labels, void* stream);

@@ -280,7 +280,7 @@ void torch_resize(const void* in, bool half, int channels, const int* in_size,
 void torch_resize_argmax(const void* in, bool half, int classes, const int* in_size,
                          const int64_t* in_strides, const int* out_size, int mode,
                          uint16_t* labels, hipStream_t st);
-size_t restore_labels_spline_workspace(const int* src, const int* dst, int separate_axis);
+size_t restore_labels_spline_workspace(const int* src, const int* dst, int order, int separate_axis);
 void restore_labels_spline(const void* logits, bool half, int classes, const int* src,
                            const int* dst, int order, int separate_axis, void* work,
                            size_t work_bytes, uint16_t* labels, hipStream_t st);

@@ -329,8 +329,8 @@ void launch_linear(LinArgs a, int planes, float* clipped, int64_t room, hipStrea
   }
 }
 
-// `work`: the spline entry's workspace (its first 256 bytes hold the flag, then a float per
-// source voxel, then one per output voxel)
+// `work`: its first 256 bytes hold the flag, then a float per source voxel, then one per output
+// voxel
 void restore_linear(const void* logits, bool half, int classes, const int* src, const int* dst,
                     int separate_axis, char* work, uint16_t* labels, hipStream_t st) {
   LinArgs a{};
@@ -364,9 +364,12 @@ void restore_linear(const void* logits, bool half, int classes, const int* src, 
 
 }  // namespace
 
-size_t restore_labels_spline_workspace(const int* src, const int* dst, int separate_axis) {
+// Order 1: the flag, the clipped values and the running winners of the redo pass; order 3: a class's
+// logits and values, the winners and the resampler's workspace.
+size_t restore_labels_spline_workspace(const int* src, const int* dst, int order, int separate_axis) {
   const int64_t s[3] = {src[0], src[1], src[2]}, d[3] = {dst[0], dst[1], dst[2]};
   const int64_t n_src = s[0] * s[1] * s[2], n_dst = d[0] * d[1] * d[2];
+  if (order == 1) return (size_t)(256 + align256(4 * n_src) + align256(4 * n_dst));
   return (size_t)(align256(4 * n_src) + 2 * align256(4 * n_dst)) +
          resample_spline_workspace(s, d, separate_axis);
 }
@@ -379,7 +382,7 @@ void restore_labels_spline(const void* logits, bool half, int classes, const int
   for (int i = 0; i < 3; ++i)
     require(src[i] >= 1 && dst[i] >= 1, "restoration shapes must be positive");
   require(separate_axis >= -1 && separate_axis < 3, "separate axis must be -1, 0, 1 or 2");
-  require(work_bytes >= restore_labels_spline_workspace(src, dst, separate_axis),
+  require(work_bytes >= restore_labels_spline_workspace(src, dst, order, separate_axis),
           "restoration workspace too small");
   const int64_t s[3] = {src[0], src[1], src[2]}, d[3] = {dst[0], dst[1], dst[2]};
   const int64_t n_src = s[0] * s[1] * s[2], n_dst = d[0] * d[1] * d[2];

@@ -1383,10 +1383,16 @@ int nnx_restore_labels(const void* d_logits, int half, int classes, const int* s
 
 size_t nnx_restore_labels_spline_workspace(const int* src_shape, const int* dst_shape,
                                            int separate_axis) {
+  return nnx_restore_labels_spline_order_workspace(src_shape, dst_shape, 3, separate_axis);
+}
+
+size_t nnx_restore_labels_spline_order_workspace(const int* src_shape, const int* dst_shape,
+                                                 int order, int separate_axis) {
   if (!src_shape || !dst_shape || separate_axis < -1 || separate_axis > 2) return 0;
+  if (order != 1 && order != 3) return 0;
   for (int a = 0; a < 3; ++a)
     if (src_shape[a] < 1 || dst_shape[a] < 1) return 0;
-  return restore_labels_spline_workspace(src_shape, dst_shape, separate_axis);
+  return restore_labels_spline_workspace(src_shape, dst_shape, order, separate_axis);
 }
 
 int nnx_restore_labels_spline(const void* d_logits, int half, int classes, const int* src_shape,

@@ -206,6 +206,8 @@ _SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
         ctypes.c_int, [c_void_p, ctypes.c_int, ctypes.c_int, c_int_p, c_int_p, c_void_p, c_void_p]
     ),
     "nnx_restore_labels_spline_workspace": (ctypes.c_size_t, [c_int_p, c_int_p, ctypes.c_int]),
+    "nnx_restore_labels_spline_order_workspace": (
+        ctypes.c_size_t, [c_int_p, c_int_p, ctypes.c_int, ctypes.c_int]),
     "nnx_restore_labels_spline": (
         ctypes.c_int,
         [c_void_p, ctypes.c_int, ctypes.c_int, c_int_p, c_int_p, ctypes.c_int, ctypes.c_int,

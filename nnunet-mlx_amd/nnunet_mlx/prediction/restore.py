@@ -171,7 +171,7 @@ def resample_class_logits_argmax_spline_device(logits: torch.Tensor, new_shape: 
     lib = _native.load()
     src = _native.ints(logits.shape[:3])
     dst = _native.ints(target)
-    size = lib.nnx_restore_labels_spline_workspace(src, dst, axis)
+    size = lib.nnx_restore_labels_spline_order_workspace(src, dst, order, axis)
     if size == 0:
         raise ContractError("invalid restoration shapes")
     work = torch.empty(size, dtype=torch.uint8, device=logits.device)

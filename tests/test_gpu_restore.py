@@ -197,3 +197,30 @@ def test_linear_restore_equals_the_resampler_by_class(device, source, target, ax
         higher = values[c] > best
         best, want = np.where(higher, values[c], best), np.where(higher, c, want).astype(np.uint16)
     np.testing.assert_array_equal(got.cpu().numpy().view(np.uint16), want)
+
+
+@pytest.mark.parametrize("order", [1, 3])
+def test_spline_restore_refuses_a_byte_less(device, order):
+    """The workspace of an order suffices, one byte less is refused and writes nothing."""
+    from nnunet_mlx import _native
+    from tests.helpers import stream
+
+    lib = _native.load()
+    source, target = (9, 13, 70), (14, 9, 65)
+    src, dst = _native.ints(source), _native.ints(target)
+    logits = torch.randn((*source, 3), device=device)
+    size = lib.nnx_restore_labels_spline_order_workspace(src, dst, order, 0)
+    work = torch.empty(size, dtype=torch.uint8, device=device)
+    labels = torch.full(target, 77, dtype=torch.int16, device=device)
+
+    def call(nbytes):
+        return lib.nnx_restore_labels_spline(logits.data_ptr(), 0, 3, src, dst, order, 0,
+                                             work.data_ptr(), nbytes, labels.data_ptr(), stream())
+
+    print(f"restoration workspace, order {order}", flush=True)
+    assert call(size - 1) == _native.NNX_ERR_INVALID and "workspace" in _native.last_error()
+    torch.cuda.synchronize()
+    assert bool((labels == 77).all())
+    _native.check(call(size))
+    torch.cuda.synchronize()
+    assert int(labels.max()) <= 2

@@ -298,6 +298,25 @@ def test_finalize_failed_part_way_leaves_the_model_refusing_retries():
         lib.nnx_model_destroy(handle)
 
 
+@pytest.mark.parametrize("axis", [-1, 0, 1, 2])
+def test_restoration_workspace_follows_the_order(axis):
+    """Order 1 needs its flag and a float a source and an output voxel; the query without an
+    order answers for either, and an order that restoration does not take for none."""
+    from nnunet_mlx import _native
+
+    lib = _native.load()
+    src, dst = _native.ints((30, 53, 54)), _native.ints((12, 51, 52))
+    up = lambda n: -(-4 * n // 256) * 256  # noqa: E731
+    linear = lib.nnx_restore_labels_spline_order_workspace(src, dst, 1, axis)
+    assert linear == 256 + up(30 * 53 * 54) + up(12 * 51 * 52)
+    cubic = lib.nnx_restore_labels_spline_order_workspace(src, dst, 3, axis)
+    assert cubic == lib.nnx_restore_labels_spline_workspace(src, dst, axis) > 3 * linear
+    for order in (-1, 0, 2, 4):
+        assert lib.nnx_restore_labels_spline_order_workspace(src, dst, order, axis) == 0
+    assert lib.nnx_restore_labels_spline_order_workspace(None, dst, 1, axis) == 0
+    assert lib.nnx_restore_labels_spline_order_workspace(src, dst, 1, 3) == 0
+
+
 _SLOPES_PROGRAM = r"""
 #include "nnx_internal.h"
 int main() {
