@@ -34,6 +34,13 @@
 //      every z tap that reaches an output plane of the box (up to 18 MFMAs).  U (2 positions x
 //      3 taps, 48 registers) is reloaded from L2 tap by tap as the chunk's last product with it
 //      is issued, so its latency is covered by the planes that follow.
+//
+// Sums: an accumulator rounds once a product, and that is most of the error: squared and
+// relative it measures 1.5e-15 a rounding, in accumulators that hold three z taps and three
+// products a chunk.  From four chunks on two of the taps are therefore summed from zero, their
+// small products first, and added as one (4 roundings a chunk instead of 9) in half the output
+// planes, from six chunks in all; it takes the last plane's V in registers and 16 additions for
+// six products.
 // Epilogue, a z plane at a time: each wave applies its share of the x-output transform and
 // writes its two partials to LDS, and a thread sums the eight waves' partials of one tile
 // column for four output channels (y-output transform), scales back, adds the bias and stores
@@ -45,14 +52,22 @@
 // issues the next box's first halo DMA and U loads; the epilogue exchanges through the raw
 // buffer that this DMA does not target.
 //
-// Bound by power and issue together: a 128 -> 128 layer on 32^3 x 8 keeps the matrix cores 38 %
-// busy at 1.9 GHz (2.4 GHz with the products left out, 2.0 GHz with the products alone), and
-// leaving out any one part (products 38 %, halo DMA 21 %, transform and split 18 %, epilogue
-// 11 %, patch reads 9 %, U loads 7 %) takes its share off the time.  Measured against the
-// three-axis form it replaces, ms: 32 + 32 -> 32 on 128^3 x 8 4.48 -> 3.79 (490 TFLOP/s of the
-// direct convolution's work), 128 -> 128 on 32^3 x 8 0.471 -> 0.406 (571), 64 -> 64 on
-// 37 x 61 x 43 x 4 0.249 -> 0.216 (398); error against float64 2.6e-7 to 3.6e-7 relative
-// (the three-axis form 2.5e-7 to 3.2e-7, the direct split kernel 3.4e-7).
+// Bound by power and issue together: a 128 -> 128 layer on 32^3 x 8 kept the matrix cores 38 %
+// busy at 1.9 GHz (2.4 GHz with the products left out, 2.0 GHz with the products alone) with
+// plain sums, and leaving out any one part (products 38 %, halo DMA 21 %, transform and split
+// 18 %, epilogue 11 %, patch reads 9 %, U loads 7 %) took its share off the time.  The kernels of
+// 4-plane boxes are at the register limit of 256: three of the six spill 8 or 12 bytes a lane, and all
+// of them 66 to 69 scalar registers to vector lanes.
+// Measured, three-axis form / plain sums / now, us and relative error against float64:
+//   32 + 32 -> 32 on 128^3 x 8       4400 / 3650 / 3840   2.62 / 2.79 / 2.52e-7  (484 TFLOP/s of
+//                                                          the direct convolution's work)
+//   128 -> 128 on 32^3 x 8            492 /  407 /  433   3.06 / 3.54 / 2.61e-7  (536)
+//   64 -> 64 on 37 x 61 x 43 x 4      257 /  222 /  233   2.61 / 2.78 / 2.52e-7  (369)
+//   256 + 256 -> 256 on 16^3 x 8      427 /  360 /  380   5.18 / 6.65 / 4.44e-7
+//   320 -> 320 on 5 x 6 x 7          65.3 / 60.1 / 64.5   4.19 / 5.20 / 3.56e-7 (on 12 x 13 x 11)
+//   32 -> 192 on 6 x 9 x 8 x 8       12.8 / 13.4 / 13.2   2.40 / 2.24 / 2.24e-7
+// The last, like 32 -> 32 on 8^3 (11.2 / 11.9 / 11.7), is one box of two chunks a CU: the fixed
+// part of a launch, which the three-axis form had smaller.
 #include <cmath>
 #include <string>
 #include <type_traits>
@@ -178,6 +193,33 @@ __device__ __forceinline__ void read_patch(const unsigned (&ad)[6], f4 (&v)[12])
       : "memory");
 }
 
+// The same by columns, two (P and Q) and one (R).
+template <int OFFSET>
+__device__ __forceinline__ void read_column(unsigned a0, unsigned a1, f4 (&v)[4]) {
+  asm volatile(
+      "ds_read_b128 %0, %4 offset:%6\n\tds_read_b128 %1, %4 offset:%7\n\t"
+      "ds_read_b128 %2, %5 offset:%6\n\tds_read_b128 %3, %5 offset:%7\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+      : "v"(a0), "v"(a1), "n"(OFFSET), "n"(OFFSET + 16)
+      : "memory");
+}
+
+template <int OFFSET>
+__device__ __forceinline__ void read_columns(unsigned a0, unsigned a1, unsigned b0, unsigned b1,
+                                             f4 (&v)[4], f4 (&w)[4]) {
+  asm volatile(
+      "ds_read_b128 %0, %8 offset:%12\n\tds_read_b128 %1, %8 offset:%13\n\t"
+      "ds_read_b128 %2, %9 offset:%12\n\tds_read_b128 %3, %9 offset:%13\n\t"
+      "ds_read_b128 %4, %10 offset:%12\n\tds_read_b128 %5, %10 offset:%13\n\t"
+      "ds_read_b128 %6, %11 offset:%12\n\tds_read_b128 %7, %11 offset:%13\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(w[0]), "=&v"(w[1]),
+        "=&v"(w[2]), "=&v"(w[3])
+      : "v"(a0), "v"(a1), "v"(b0), "v"(b1), "n"(OFFSET), "n"(OFFSET + 16)
+      : "memory");
+}
+
 // x summed over the eight lanes of a wave that share lane % 8, in every lane: a rotation by
 // 8 within rows of 16, then v_permlane16_swap and v_permlane32_swap (each leaves a pair's two
 // values in every lane of the pair).
@@ -219,7 +261,8 @@ __device__ __forceinline__ WinoBox wino_box(const WinoArgs& a, int v) {
   return r;
 }
 
-template <int ZB, WinoShape S>
+// CH: output planes of a slab whose first two z taps are summed apart.
+template <int ZB, WinoShape S, int CH>
 __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
   using G = WinoBoxGeom<ZB, S>;
   __shared__ __align__(16) f4 s_raw[2 * G::buf];             // two raw halo buffers
@@ -274,8 +317,9 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
       quads |= (rq & 3) << (2 * j);
     }
   };
-  // Rounds [r0, r1) of a chunk of a box's halo into buffer `buf`, spread over the previous chunk's
-  // products.
+  // A chunk of a box's halo into buffer `buf`, during the previous chunk's products.  The address of
+  // a pattern is formed once for its planes (formed for each round and spread over the planes,
+  // 128 -> 128 on 32^3 x 8 took 449 us instead of 436).
   struct Source {
     uint64_t base;         // channel chunk of the halo's first plane (may lie outside the volume;
                            // cube: of the item)
@@ -292,20 +336,22 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
              (first ? chunk : chunk - a.chunks0) * kWChunk * 4;
     return r;
   };
-  auto fetch = [&](const Source& src, const int (&at)[kL], int quads, int buf, auto r0c, auto r1c)
-      __attribute__((always_inline)) {
+  auto fetch = [&](const Source& src, const int (&at)[kL], int quads, int buf) __attribute__((always_inline)) {
     f4* dst = s_raw + buf * G::buf + wave * 64;
 #pragma unroll
-    for (int r = decltype(r0c)::value; r < decltype(r1c)::value; ++r) {
-      const int k = S == kCube ? 0 : r / 3, j = S == kCube ? r : r % 3;
-      const int p = S == kCube ? 0 : round_plane(k, j);
-      // a per-lane plane index keeps the check a select of two addresses instead of a branch
-      const int z = at[j] >= 0 ? src.z0 + p : -1;
-      const uint64_t in = src.base + p * src.plane_bytes +
-                          ((int64_t)at[j] * src.C + ((quads >> (2 * j)) & 3) * 4) * 4;
-      const uint64_t g = (unsigned)z < (unsigned)a.D ? in : zero;
-      __builtin_amdgcn_global_load_lds(
-          (const void*)g, (__attribute__((address_space(3))) void*)(dst + r * kWThreads), 16, 0, 0);
+    for (int j = 0; j < kL; ++j) {
+      // this thread's line of the pattern in plane 0 (cube: the line)
+      const uint64_t line = src.base + ((int64_t)at[j] * src.C + ((quads >> (2 * j)) & 3) * 4) * 4;
+      constexpr int kPer = S == kCube ? 1 : G::hz / 2;
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) {
+        const int r = S == kCube ? j : 3 * k + j;
+        const int p = S == kCube ? 0 : round_plane(k, j);
+        const bool in = at[j] >= 0 && (unsigned)(src.z0 + p) < (unsigned)a.D;
+        const uint64_t g = in ? line + p * src.plane_bytes : zero;
+        __builtin_amdgcn_global_load_lds(
+            (const void*)g, (__attribute__((address_space(3))) void*)(dst + r * kWThreads), 16, 0, 0);
+      }
     }
   };
   // pending-norm parameters of every input channel (both inputs, in chunk order) of item b
@@ -386,8 +432,7 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
     const int tid = threadIdx.x;
     const WinoBox first = wino_box(a, v);
     box_lines(tid, first, yx, quads);
-    fetch(source(first, cbeg), yx, quads, 0, std::integral_constant<int, 0>{},
-          std::integral_constant<int, kRounds>{});
+    fetch(source(first, cbeg), yx, quads, 0);
     const uint4* up = uaddr(tid & 63, first.nt, cbeg);
 #pragma unroll
     for (int kz = 0; kz < 3; ++kz) load_u(up, kz);
@@ -441,41 +486,104 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[p][z][r] = 0.f;
 
-    // input plane Z of the halo: V of both positions, then its products with every z tap kz
-    // whose output plane Z - kz lies in the box
+    // Input plane Z of the halo: V of both positions, then its products.  z tap 2 of an output plane
+    // is added to its accumulator, tap 0 and 1 too from plane CH on; below it they are summed
+    // from zero, the small products first, once both planes' V are there, and then added.
+    h8 vh[2][2], vl[2][2];  // V of this plane and the last, split: [plane & 1][position]
     auto plane = [&](auto zc) __attribute__((always_inline)) {
-      constexpr int Z = decltype(zc)::value;
-      f4 d[12];
-      read_patch<Z * G::plane * 16>(ad, d);
-      float vp[8], vq8[8], vr8[8];
+      constexpr int Z = decltype(zc)::value, kAt = Z * G::plane * 16, now = Z & 1;
+      if constexpr (CH > 0 && ZB == 4) {
+        // (two columns, then one: the last plane's V is held too, and the registers are full)
+        float vq[8];
+        {
+          f4 dp[4], dq[4];
+          read_columns<kAt>(ad[0], ad[3], ad[1], ad[4], dp, dq);
+          float va[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        vp[e] = fmaf(sy, d[6 + (e >> 2)][e & 3], d[e >> 2][e & 3]);
-        vq8[e] = fmaf(sy, d[8 + (e >> 2)][e & 3], d[2 + (e >> 2)][e & 3]);
-        vr8[e] = fmaf(sy, d[10 + (e >> 2)][e & 3], d[4 + (e >> 2)][e & 3]);
+          for (int e = 0; e < 8; ++e) {
+            vq[e] = fmaf(sy, dq[2 + (e >> 2)][e & 3], dq[e >> 2][e & 3]);
+            va[e] = fmaf(sy, dp[2 + (e >> 2)][e & 3], dp[e >> 2][e & 3]) - vq[e];
+          }
+          split8(va, vh[now][0], vl[now][0]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        f4 dr[4];
+        read_column<kAt>(ad[2], ad[5], dr);
+        float vb[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          vb[e] = fmaf(sx, vq[e], fmaf(sy, dr[2 + (e >> 2)][e & 3], dr[e >> 2][e & 3]));
+        split8(vb, vh[now][1], vl[now][1]);
+        __builtin_amdgcn_sched_barrier(0);
+      } else {
+        f4 d[12];
+        read_patch<kAt>(ad, d);
+        float va[8], vb[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float vp = fmaf(sy, d[6 + (e >> 2)][e & 3], d[e >> 2][e & 3]);
+          const float vq = fmaf(sy, d[8 + (e >> 2)][e & 3], d[2 + (e >> 2)][e & 3]);
+          const float vr = fmaf(sy, d[10 + (e >> 2)][e & 3], d[4 + (e >> 2)][e & 3]);
+          va[e] = vp - vq;
+          vb[e] = fmaf(sx, vq, vr);
+        }
+        split8(va, vh[now][0], vl[now][0]);
+        split8(vb, vh[now][1], vl[now][1]);
       }
-      float va[8], vb[8];
+      // product 0: lo * hi, 1: hi * lo, 2: hi * hi
+      auto product = [&](int which, int v, int p, int kz, f16v c) __attribute__((always_inline)) {
+        return mfma32(which == 0 ? vl[v][p] : vh[v][p],
+                      *reinterpret_cast<const h8*>(&ub[p][kz][which == 1 ? 1 : 0]), c);
+      };
+      constexpr bool chain = Z >= 1 && Z - 1 < CH;
+      if constexpr (chain) {
+        if constexpr (ZB == 2) {
+          f16v t[2]{};
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        va[e] = vp[e] - vq8[e];
-        vb[e] = fmaf(sx, vq8[e], vr8[e]);
+          for (int i = 0; i < 6; ++i)
+#pragma unroll
+            for (int p = 0; p < 2; ++p) t[p] = product(i >> 1, (Z - 1 + (i & 1)) & 1, p, i & 1, t[p]);
+          if constexpr (Z >= 2) {
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+              acc[i & 1][Z - 2] = product(2 - (i >> 1), now, i & 1, 2, acc[i & 1][Z - 2]);
+          }
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            acc[p][Z - 1] += t[p];
+            asm volatile("" : "+v"(acc[p][Z - 1]));  // added here, not where it is used next
+          }
+        } else {
+          // (one position after the other: the registers hold one sum.  The third tap's products
+          // of both positions cover the wait for the first)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            f16v t{};
+#pragma unroll
+            for (int i = 0; i < 6; ++i) t = product(i >> 1, (Z - 1 + (i & 1)) & 1, p, i & 1, t);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (Z >= 2) {
+#pragma unroll
+              for (int i = 0; i < 6; ++i)
+                if (p == 0) acc[i & 1][Z - 2] = product(2 - (i >> 1), now, i & 1, 2, acc[i & 1][Z - 2]);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+            acc[p][Z - 1] += t;
+            asm volatile("" : "+v"(acc[p][Z - 1]));  // added here: left to its next use, t is held till then
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
       }
-      h8 hi[2], lo[2];
-      split8(va, hi[0], lo[0]);
-      split8(vb, hi[1], lo[1]);
 #pragma unroll
-      for (int product = 0; product < 3; ++product)
+      for (int which = 2; which >= 0; --which)
 #pragma unroll
         for (int kz = 0; kz < 3; ++kz) {
-          constexpr int none = -1;
-          const int o = Z - kz >= 0 && Z - kz < ZB ? Z - kz : none;
-          if (o == none) continue;
+          const int o = Z - kz;
+          if (o < 0 || o >= ZB || (kz < 2 && o < CH) || (kz == 2 && chain)) continue;
 #pragma unroll
-          for (int p = 0; p < 2; ++p)
-            acc[p][o] = mfma32(product == 2 ? lo[p] : hi[p],
-                               *reinterpret_cast<const h8*>(&ub[p][kz][product == 1 ? 1 : 0]),
-                               acc[p][o]);
+          for (int p = 0; p < 2; ++p) acc[p][o] = product(which, now, p, kz, acc[p][o]);
         }
+      if constexpr (CH > 0) __builtin_amdgcn_sched_barrier(0);
     };
 
     for (int chunk = cbeg; chunk < cend; ++chunk) {
@@ -490,25 +598,17 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
         box_lines(tid_n, nxt, yx, quads);
       }
       const Source src = source(last ? nxt : cur, last ? cbeg : chunk + 1);
-      auto rounds = [&](auto ic) __attribute__((always_inline)) {
-        constexpr int I = decltype(ic)::value;
-        if (!last || more)
-          fetch(src, yx, quads, buf ^ 1, std::integral_constant<int, I * kRounds / ZB>{},
-                std::integral_constant<int, (I + 1) * kRounds / ZB>{});
-      };
+      if (!last || more) fetch(src, yx, quads, buf ^ 1);
       const uint4* un = uaddr(lane, last ? nxt.nt : cur.nt, last ? cbeg : chunk + 1);
-      rounds(std::integral_constant<int, 0>{});
       plane(std::integral_constant<int, 0>{});
-      rounds(std::integral_constant<int, 1>{});
       plane(std::integral_constant<int, 1>{});
       if constexpr (ZB == 4) {
-        rounds(std::integral_constant<int, 2>{});
         plane(std::integral_constant<int, 2>{});
-        rounds(std::integral_constant<int, 3>{});
         plane(std::integral_constant<int, 3>{});
       }
-      load_u(un, 0);
+      if constexpr (CH < ZB) load_u(un, 0);
       plane(std::integral_constant<int, ZB>{});
+      if constexpr (CH == ZB) load_u(un, 0);
       load_u(un, 1);
       plane(std::integral_constant<int, ZB + 1>{});
       load_u(un, 2);
@@ -520,7 +620,6 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
 
     // ---- epilogue, in the raw buffer of the box's last chunk
     lds_barrier();  // every wave is past its last read of it
-    float* part = reinterpret_cast<float*>(s_raw + (buf ^ 1) * G::buf);
     f4* red = s_raw + (buf ^ 1) * G::buf + kPartSlots;
     if (nxt.b != cur.b) load_prm(tid, nxt.b);  // visible after the barriers below
     const int quad = tid & 7, rho = (tid >> 3) & 31, ox = tid >> 8;
@@ -530,6 +629,7 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
     for (int z = 0; z < ZB; ++z) {
       // partials [wave][ox][tile][column]; tile row r sits at rho(r) = (r / 8) * 8 + (r % 4) * 2 +
       // (r / 4) % 2, so that a wave's two row groups (r and r + 4) write different banks
+      float* part = reinterpret_cast<float*>(s_raw + (more || (z & 1) == 0 ? buf ^ 1 : buf) * G::buf);
       float* pw = part + wave * 2048 + (lane >> 5) * 32 + (lane & 31);
       auto write_parts = [&](auto hc) __attribute__((always_inline)) {
 #pragma unroll
@@ -563,7 +663,7 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
                *reinterpret_cast<const f4*>(pr + (2 * i + 1) * 2048);
       yo[z][0] = ((m[0] + m[1]) + m[2]) * a.out_scale + bias;
       yo[z][1] = ((m[1] - m[2]) - m[3]) * a.out_scale + bias;
-      lds_barrier();
+      if (more) lds_barrier();  // (the last box's planes take the two buffers in turn)
     }
     const int row = 8 * (rho >> 3) + 4 * (rho & 1) + ((rho >> 1) & 3);
     const int yy = cur.byi * G::by + 2 * (S == kWide ? row >> 3 : S == kTall ? row >> 2 : (row >> 2) & 3);
@@ -858,16 +958,22 @@ void conv3d_wino(const float* x1, int c1, const float* x2, int c2, const void* p
   ProfScope prof("conv3d_wino", flops, bytes, st);
   const dim3 grid((unsigned)std::min<int64_t>(compute_units(), ceil_div(nwg, 8) * 8),
                   (unsigned)ceil_div(a.chunks, a.cper)), block(kWThreads);
-  if (p.zb == 4 && p.shape == kWide)
-    hipLaunchKernelGGL((wino_yx_kernel<4, kWide>), grid, block, 0, st, a);
-  else if (p.zb == 4)
-    hipLaunchKernelGGL((wino_yx_kernel<4, kTall>), grid, block, 0, st, a);
-  else if (p.shape == kWide)
-    hipLaunchKernelGGL((wino_yx_kernel<2, kWide>), grid, block, 0, st, a);
-  else if (p.shape == kTall)
-    hipLaunchKernelGGL((wino_yx_kernel<2, kTall>), grid, block, 0, st, a);
+  auto launch = [&](auto chained) {
+    constexpr int C = decltype(chained)::value;
+    auto kernel = p.zb == 4 ? (p.shape == kWide ? wino_yx_kernel<4, kWide, C> : wino_yx_kernel<4, kTall, C>)
+                  : p.shape == kWide ? wino_yx_kernel<2, kWide, C / 2>
+                  : p.shape == kTall ? wino_yx_kernel<2, kTall, C / 2>
+                                     : wino_yx_kernel<2, kCube, C / 2>;
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, a);
+  };
+  // The error must not exceed the three-axis form's: up to three chunks a workgroup it does not
+  // with plain sums, up to five with half the planes' apart (see the head of the file).
+  if (a.cper <= 3)
+    launch(std::integral_constant<int, 0>{});
+  else if (a.cper <= 5)
+    launch(std::integral_constant<int, 2>{});
   else
-    hipLaunchKernelGGL((wino_yx_kernel<2, kCube>), grid, block, 0, st, a);
+    launch(std::integral_constant<int, 4>{});
   launch_check("conv3d_winograd");
 }
 
