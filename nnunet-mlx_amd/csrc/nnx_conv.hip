@@ -139,13 +139,13 @@ struct IgemmArgs {
   const uint4* w16;   // split-fp16 packed weights (x3 kernel)
   int ntg;            // tap groups of 4 (x3 kernel)
   float out_scale;    // 1 / weight scale (x3 kernel)
-  int cper;           // chunks of a workgroup (igemm_x3): blockIdx.y takes [cper blockIdx.y, + cper)
-  int64_t split_stride;  // elements between the outputs of two blockIdx.y
   // pending InstanceNorm (+ LeakyReLU) of input 0 / 1: (mean, scale, beta, 0) per (b, c)
   const float4* nrm0;
   const float4* nrm1;
   int act0, act1;
   float slope;
+  int cper;           // chunks of a workgroup (igemm_x3): blockIdx.y takes [cper blockIdx.y, + cper)
+  int64_t split_stride;  // elements between the outputs of two blockIdx.y
 };
 
 // The pending normalisation of one halo line (4 channels c..c+3 of the chunk's source):
