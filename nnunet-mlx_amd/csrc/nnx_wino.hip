@@ -56,8 +56,8 @@
 // busy at 1.9 GHz (2.4 GHz with the products left out, 2.0 GHz with the products alone) with
 // plain sums, and leaving out any one part (products 38 %, halo DMA 21 %, transform and split
 // 18 %, epilogue 11 %, patch reads 9 %, U loads 7 %) took its share off the time.  The kernels of
-// 4-plane boxes are at the register limit of 256: three of the six spill 8 or 12 bytes a lane, and all
-// of them 66 to 69 scalar registers to vector lanes.
+// 4-plane boxes are at the register limit of 256: those with half the sums apart spill one (8 bytes a
+// lane), and all of them 56 to 61 scalar registers to vector lanes.
 // Measured, three-axis form / plain sums / now, us and relative error against float64:
 //   32 + 32 -> 32 on 128^3 x 8       4400 / 3650 / 3840   2.62 / 2.79 / 2.52e-7  (484 TFLOP/s of
 //                                                          the direct convolution's work)
@@ -65,9 +65,7 @@
 //   64 -> 64 on 37 x 61 x 43 x 4      257 /  222 /  233   2.61 / 2.78 / 2.52e-7  (369)
 //   256 + 256 -> 256 on 16^3 x 8      427 /  360 /  380   5.18 / 6.65 / 4.44e-7
 //   320 -> 320 on 5 x 6 x 7          65.3 / 60.1 / 64.5   4.19 / 5.20 / 3.56e-7 (on 12 x 13 x 11)
-//   32 -> 192 on 6 x 9 x 8 x 8       12.8 / 13.4 / 13.2   2.40 / 2.24 / 2.24e-7
-// The last, like 32 -> 32 on 8^3 (11.2 / 11.9 / 11.7), is one box of two chunks a CU: the fixed
-// part of a launch, which the three-axis form had smaller.
+//   32 -> 192 on 6 x 9 x 8 x 8       12.9 / 13.5 / 12.9   2.40 / 2.24 / 2.24e-7
 #include <cmath>
 #include <string>
 #include <type_traits>
@@ -143,7 +141,17 @@ struct WinoArgs {
   const float4* nrm1;
   int act0, act1;
   float slope;
+  unsigned rbox, rz, ry, rx;  // reciprocals of nbox, nbz, nby, nbx
 };
+
+// n / d by d's reciprocal floor((2^32 - 1) / d): the product is the quotient or one less, as n is
+// below 2^32.  (A box takes twelve of them before its first load: as divisions they were 0.4 us of
+// every launch.)
+inline unsigned reciprocal(int d) { return 0xffffffffu / (unsigned)d; }
+__device__ __forceinline__ int divide(int n, int d, unsigned r) {
+  const int q = (int)__umulhi((unsigned)n, r);
+  return n - q * d >= d ? q + 1 : q;
+}
 
 // 16 zero bytes: halo lines outside the volume are fetched from here.
 __device__ __align__(16) float g_wino_zero[4];
@@ -250,14 +258,15 @@ struct WinoBox {
 
 __device__ __forceinline__ WinoBox wino_box(const WinoArgs& a, int v) {
   WinoBox r;
-  r.nt = v / a.nbox;
+  r.nt = divide(v, a.nbox, a.rbox);
   int box = v - r.nt * a.nbox;
-  r.bxi = box % a.nbx;
-  box /= a.nbx;
-  r.byi = box % a.nby;
-  box /= a.nby;
-  r.bzi = box % a.nbz;
-  r.b = box / a.nbz;
+  int q = divide(box, a.nbx, a.rx);
+  r.bxi = box - q * a.nbx;
+  box = q;
+  q = divide(box, a.nby, a.ry);
+  r.byi = box - q * a.nby;
+  r.b = divide(q, a.nbz, a.rz);
+  r.bzi = q - r.b * a.nbz;
   return r;
 }
 
@@ -942,6 +951,10 @@ void conv3d_wino(const float* x1, int c1, const float* x2, int c2, const void* p
   require(nwg < (1LL << 31), "convolution grid too large");
   a.nvirt = (int)nwg;
   a.nbox = a.nvirt / (cout / 32);
+  a.rbox = reciprocal(a.nbox);
+  a.rz = reciprocal(a.nbz);
+  a.ry = reciprocal(a.nby);
+  a.rx = reciprocal(a.nbx);
   a.cper = (int)ceil_div(a.chunks, splits);
   a.split_stride = (int64_t)g.batch * g.out[0] * g.out[1] * g.out[2] * cout;
   a.out_scale = 1.0f / scale;
