@@ -27,7 +27,8 @@
 //      LDS buffers during the previous chunk, its slots laid out so that the 32 tiles of a
 //      half-wave read 32 different 16-byte bank groups;
 //   2. each thread applies the input's pending InstanceNorm (+ LeakyReLU) in place to the
-//      lines that it fetched itself (so it waits for its own loads only); one barrier;
+//      lines that it fetched itself (so it waits for its own loads only); one barrier, behind
+//      which it waits for U too;
 //   3. the next chunk's halo DMA is issued, into the other buffer;
 //   4. per input plane each wave reads the two rows and three columns of its positions'
 //      patches, forms V, splits it in registers and issues the products with the packed U of
@@ -59,13 +60,13 @@
 // 4-plane boxes are at the register limit of 256: those with half the sums apart spill one (8 bytes a
 // lane), and all of them 56 to 61 scalar registers to vector lanes.
 // Measured, three-axis form / plain sums / now, us and relative error against float64:
-//   32 + 32 -> 32 on 128^3 x 8       4400 / 3650 / 3840   2.62 / 2.79 / 2.52e-7  (484 TFLOP/s of
+//   32 + 32 -> 32 on 128^3 x 8       4400 / 3650 / 3830   2.62 / 2.79 / 2.52e-7  (485 TFLOP/s of
 //                                                          the direct convolution's work)
-//   128 -> 128 on 32^3 x 8            492 /  407 /  433   3.06 / 3.54 / 2.61e-7  (536)
-//   64 -> 64 on 37 x 61 x 43 x 4      257 /  222 /  233   2.61 / 2.78 / 2.52e-7  (369)
-//   256 + 256 -> 256 on 16^3 x 8      427 /  360 /  380   5.18 / 6.65 / 4.44e-7
-//   320 -> 320 on 5 x 6 x 7          65.3 / 60.1 / 64.5   4.19 / 5.20 / 3.56e-7 (on 12 x 13 x 11)
-//   32 -> 192 on 6 x 9 x 8 x 8       12.9 / 13.5 / 12.9   2.40 / 2.24 / 2.24e-7
+//   128 -> 128 on 32^3 x 8            492 /  407 /  424   3.06 / 3.54 / 2.61e-7  (547)
+//   64 -> 64 on 37 x 61 x 43 x 4      257 /  222 /  229   2.61 / 2.78 / 2.52e-7  (375)
+//   256 + 256 -> 256 on 16^3 x 8      427 /  365 /  385   5.18 / 6.65 / 4.44e-7
+//   320 -> 320 on 5 x 6 x 7          65.3 / 60.0 / 61.3   4.19 / 5.20 / 3.56e-7 (on 12 x 13 x 11)
+//   32 -> 192 on 6 x 9 x 8 x 8       12.8 / 13.3 / 12.5   2.40 / 2.24 / 2.24e-7
 #include <cmath>
 #include <string>
 #include <type_traits>
@@ -447,6 +448,7 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
     for (int kz = 0; kz < 3; ++kz) load_u(up, kz);
     load_prm(tid, first.b);  // (behind the halo, whose latency theirs hides in)
     if (tid < 32) s_bias[tid] = a.bias ? a.bias[first.nt * 32 + tid] : 0.f;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();  // the parameters and the bias
   }
 
@@ -596,9 +598,14 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
     };
 
     for (int chunk = cbeg; chunk < cend; ++chunk) {
-      __builtin_amdgcn_s_waitcnt(0);  // this thread's halo lines and U have landed
+      // This thread's halo lines have landed: vector-memory operations complete in order, and the
+      // twelve loads of U follow the halo's, as may stores of the last box.  U is waited for behind
+      // the barrier (320 -> 320 on 5 x 6 x 7 64.2 to 61.3 us, 128 -> 128 on 32^3 x 8 430 to 424), but
+      // before the next halo's loads, which the compiler would wait for with it.
+      asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
       normalise(cur, yx, quads, chunk, buf);
       lds_barrier();  // every thread's lines; the other buffer is free
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       const bool last = chunk + 1 == cend;
       // the next chunk's halo; after the box's last chunk the next box's first, if there is one
       if (last && more) {
