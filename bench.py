@@ -364,17 +364,17 @@ def _short_kernel(name: str) -> str:
 def kernel_class_of(short: str) -> str | None:
     """Map a rocprof kernel name to the profiling class bench.py reports
     (igemm_kernel<MB, NB, WM, WN, ...> -> conv3d_igemm_m{16*MB*WM}n{16*NB*WN}, the
-    split-fp16 kernels igemm_x3s_kernel / igemm_x3_kernel -> conv3d_x3s_* / conv3d_x3_*, and
-    the Winograd kernels -> conv3d_wino, the
-    direct bf16 kernel -> conv3d_x3s_bf16_m512n64, the strided kernel -> conv3d_x3_m128n64)."""
+    split-fp16 kernels igemm_x3s_kernel / igemm_x3_kernel -> conv3d_x3s_* / conv3d_x3_*, the
+    Winograd kernel -> conv3d_wino, the direct bf16 kernel -> conv3d_x3s_bf16_m512n64, the
+    strided kernel -> conv3d_x3_strided or conv3d_x3_bf16_strided)."""
     import re
 
-    if short.startswith(("wino_yx_kernel", "wino_x3_kernel", "wino_x3p_kernel")):
+    if short.startswith("wino_yx_kernel"):
         return "conv3d_wino"
     if short.startswith("conv_bf16_kernel"):
         return "conv3d_x3s_bf16_m512n64"
     if short.startswith("conv_strided_kernel"):
-        return "conv3d_x3_bf16_m128n64" if "1>" in short else "conv3d_x3_m128n64"
+        return "conv3d_x3_bf16_strided" if short.endswith(", 1>") else "conv3d_x3_strided"
     m = re.match(r"igemm(_x3s|_x3)?_kernel<(\d+), (\d+), (\d+), (\d+)([^>]*)>", short)
     if not m:
         return None
@@ -649,23 +649,23 @@ def measured_traffic(kernel_class: str) -> float | None:
 WINO_ISSUED = 16 / 36
 
 
-def kernel_table(classes: dict, steps: int, traffic: bool = True,
-                 wino_issued: float = 64 / 216) -> tuple[dict, dict]:
+def kernel_table(classes: dict, steps: int, traffic: bool = True) -> tuple[dict, dict]:
     """Per-kernel-class rates of a KernelProfile (launches and ms per step) and the roofline
     object of the dominant class (largest share of the timed region): algorithmic FLOPs or
     bytes over its launch time, against the published peak of the unit that bounds it.
     `traffic`: take the HBM bytes per launch from the liver-case counter summary (only the
-    liver workload's launches are the ones it measured).  `wino_issued`: issued products per
-    direct product of the Winograd class (the default is F(2x2x2)'s)."""
+    liver workload's launches are the ones it measured)."""
     kernels = {}
     for name, c in sorted(classes.items(), key=lambda kv: -kv[1]["ms"]):
         entry = {"launches": c["launches"] // steps, "ms": round(c["ms"] / steps, 3)}
         if c["flops"]:
             entry["tflops"] = round(c["flops"] / (c["ms"] * 1e-3) / 1e12, 2)
             if name.startswith("conv3d_x3") and "_bf16" in name:
-                # issued bf16 MFMA work: 1 product per term, 4-tap groups (27 -> 28 taps)
+                # issued bf16 MFMA work: 1 product per term, 27 taps in the direct kernel and
+                # groups of 4 or 2 in the others (27 -> 28 taps)
+                taps = 27 if name.endswith("m512n64") else 28
                 entry["frac_bf16_mfma_issued"] = round(
-                    entry["tflops"] * 28 / 27 / PEAK_FP16_MFMA_TFLOPS, 4)
+                    entry["tflops"] * taps / 27 / PEAK_FP16_MFMA_TFLOPS, 4)
             elif name.startswith("conv3d_x3"):
                 # issued fp16 MFMA work: 3 products per term, 4-tap groups (27 -> 28 taps)
                 entry["frac_fp16_mfma_issued"] = round(
@@ -673,7 +673,7 @@ def kernel_table(classes: dict, steps: int, traffic: bool = True,
             elif name == "conv3d_wino":
                 # issued fp16 MFMA work: 3 products per term of the transformed convolution
                 entry["frac_fp16_mfma_issued"] = round(
-                    entry["tflops"] * SPLIT_PRODUCTS * wino_issued / PEAK_FP16_MFMA_TFLOPS, 4)
+                    entry["tflops"] * SPLIT_PRODUCTS * WINO_ISSUED / PEAK_FP16_MFMA_TFLOPS, 4)
             elif name.startswith("tconv3d_x3"):
                 # issued MFMA work of the pointwise GEMM: 3 fp16 products per term (1 bf16
                 # product in the bf16 variant; bf16 and fp16 share the dense peak); the
@@ -870,8 +870,7 @@ def ensemble_workload(args) -> int:
         torch.cuda.synchronize()
         step_s = (time.perf_counter() - t0) / args.steps
     device_peak_gb = peak.gb()
-    kernels, roofline = kernel_table(prof.classes, steps=args.steps, traffic=False,
-                                     wino_issued=WINO_ISSUED)
+    kernels, roofline = kernel_table(prof.classes, steps=args.steps, traffic=False)
     steps = [len(s) for s in sw.compute_steps([max(a, b) for a, b in zip(volume.shape[1:], patch)],
                                               patch, step_fraction=0.5)]
     tiles = int(np.prod(steps))
@@ -1090,7 +1089,7 @@ def main() -> int:
 
     device_peak_gb = peak.gb()
     classes = prof.classes
-    kernels, roofline = kernel_table(classes, steps=args.steps, wino_issued=WINO_ISSUED)
+    kernels, roofline = kernel_table(classes, steps=args.steps)
     # 3x3x3 convolution rate against the float32-class MFMA peak of the arithmetic used
     conv_frac = conv_mfma_frac(classes, args.precision)
 

@@ -505,7 +505,7 @@ void conv3d_strided(const float* x1, int c1, const float* x2, int c2, const void
   a.act1 = n2.act ? 1 : 0;
   a.slope = n1.params ? n1.slope : n2.slope;
   const double out_vox = (double)g.batch * g.out[0] * g.out[1] * g.out[2];
-  ProfScope prof(arith == kArithBf16 ? "conv3d_x3_bf16_m128n64" : "conv3d_x3_m128n64",
+  ProfScope prof(arith == kArithBf16 ? "conv3d_x3_bf16_strided" : "conv3d_x3_strided",
                  2.0 * (c1 + c2) * cout * 27.0 * out_vox,
                  4.0 * ((double)g.batch * g.in[0] * g.in[1] * g.in[2] * (c1 + c2) + out_vox * cout),
                  st);

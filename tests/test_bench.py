@@ -15,8 +15,10 @@ def test_kernel_names_map_to_the_profiled_classes():
     import bench
 
     cases = {
-        "wino_x3_kernel": "conv3d_wino",
-        "wino_x3p_kernel": "conv3d_wino",
+        "wino_yx_kernel<4, (nnx::": "conv3d_wino",
+        "conv_bf16_kernel<2>": "conv3d_x3s_bf16_m512n64",
+        "conv_strided_kernel<2, 0>": "conv3d_x3_strided",
+        "conv_strided_kernel<1, 1>": "conv3d_x3_bf16_strided",
         "igemm_x3_kernel<2, 2, 2, 2, 7, true, 0>": "conv3d_x3_m64n64",
         "igemm_x3_kernel<2, 4, 2, 2, 7, true, 0>": "conv3d_x3_m64n128",
         "igemm_x3s_kernel<4, 2, 4, 1, 7, true, 1>": "conv3d_x3s_bf16_m256n32",
@@ -25,15 +27,16 @@ def test_kernel_names_map_to_the_profiled_classes():
     }
     for name, cls in cases.items():
         assert bench.kernel_class_of(name) == cls, name
-    short = bench._short_kernel("void nnx::(anonymous namespace)::wino_x3p_kernel("
+    short = bench._short_kernel("void nnx::(anonymous namespace)::wino_yx_kernel<4, "
+                                "(nnx::(anonymous namespace)::WinoShape)0, 2>("
                                 "nnx::(anonymous namespace)::WinoArgs)")
-    assert short == "wino_x3p_kernel"
+    assert bench.kernel_class_of(short) == "conv3d_wino", short
 
 
 def test_kernel_table_prices_each_class_on_its_own_unit():
     """Split-fp16 classes report their issued fraction of the dense fp16 MFMA peak (three
-    products per float32 product; the Winograd class 64 transform positions per 8 x 27
-    taps), the HBM-bound head its fraction of HBM, and the roofline object follows the
+    products per float32 product; the Winograd class 16 transform positions per 4 x 9
+    taps of a plane), the HBM-bound head its fraction of HBM, and the roofline object follows the
     class with the largest share of the time."""
     sys.path.insert(0, str(ROOT))
     import bench
@@ -49,7 +52,7 @@ def test_kernel_table_prices_each_class_on_its_own_unit():
     k, roof = bench.kernel_table(classes, 1, traffic=False)
     p16 = bench.PEAK_FP16_MFMA_TFLOPS
     assert k["conv3d_wino"]["tflops"] == 400.0
-    assert abs(k["conv3d_wino"]["frac_fp16_mfma_issued"] - 400.0 * 3 * 64 / 216 / p16) < 1e-4
+    assert abs(k["conv3d_wino"]["frac_fp16_mfma_issued"] - 400.0 * 3 * 16 / 36 / p16) < 1e-4
     assert abs(k["conv3d_x3_m64n64"]["frac_fp16_mfma_issued"] - 150.0 * 3 * 28 / 27 / p16) < 1e-4
     assert abs(k["tconv3d_x3"]["frac_fp16_mfma_issued"] - 140.0 * 3 / p16) < 1e-4
     assert abs(k["tconv3d_x3_bf16"]["frac_bf16_mfma_issued"] - 140.0 / p16) < 1e-4
