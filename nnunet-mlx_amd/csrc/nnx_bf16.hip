@@ -3,7 +3,8 @@
 // float32 accumulation.
 //
 // Workgroup: 8 waves (two a SIMD), an output box of 4 x 8 x 16 voxels and 32 NC output
-// channels (NC = 2, or 1 where C_out is an odd multiple of 32).  A wave owns one of the four
+// channels (NC = 2, or 1 where C_out is 32; of 96 or 160 channels the last group computes 32 for
+// nothing, a quarter and a sixth of the products).  A wave owns one of the four
 // 4 x 8 patches of the (y, x) plane as its MFMA rows, 32 channels as its columns, and all four
 // z planes (NC = 2) or two of them (NC = 1) as separate accumulators, so the A operand of an
 // input plane and a (ky, kx) tap, read from LDS once, serves every kz that reaches an output

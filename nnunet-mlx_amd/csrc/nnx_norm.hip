@@ -325,8 +325,9 @@ __global__ __launch_bounds__(256) void norm_merge_final_kernel(const float4* __r
 // The end of a split convolution: y = sum over the splits in order (+ bias) of a (B, S, C)
 // tensor, and the InstanceNorm parameters of y.  A workgroup holds 8 channels of an item, at
 // most kSplitVox x 256 voxels, in registers (thread = channel quad and voxel modulo 256), so
-// the mean and the centred squares are two passes over registers; sums across threads in
-// float64.  Volumes of more voxels take a workgroup (blockIdx.z) per kSplitVox x 256 and leave
+// the mean and the centred squares are two passes over registers; up to 128 values (a thread's
+// four, a wave's 32 threads of a quad) are summed in float32 and the eight waves in float64.
+// Volumes of more voxels take a workgroup (blockIdx.z) per kSplitVox x 256 and leave
 // InstanceNorm partials (mean, M2, n) for instnorm_merge_partials; up to there it writes the
 // parameters and takes the place of the merge launch.  Latency: 5 us, of which a launch is 2
 // (21 to 28 us at 16^3 while a workgroup took a whole item).
