@@ -27,7 +27,7 @@
 // copy); the crop/normalise pass reads and writes 4 B per kept voxel.  A CT of 120 x 512 x 512 to
 // 300 x 534 x 534 by order 3 with a separate axis: 2.68 -> 0.86 ms per case; prefilter and
 // interpolation 1.54 -> 0.42 ms with the plane copies included (strided pass 0.27 ms, contiguous
-// pass 0.15 ms at 4 TB/s), bounds 0.20 -> 0.05, crop 0.13 -> 0.04.
+// pass 0.15 ms at 4 TB/s), bounds 0.20 -> 0.04, crop 0.13 -> 0.04.
 
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>

@@ -53,20 +53,22 @@
 // issues the next box's first halo DMA and U loads; the epilogue exchanges through the raw
 // buffer that this DMA does not target.
 //
-// Bound by power and issue together: a 128 -> 128 layer on 32^3 x 8 kept the matrix cores 38 %
-// busy at 1.9 GHz (2.4 GHz with the products left out, 2.0 GHz with the products alone) with
-// plain sums, and leaving out any one part (products 38 %, halo DMA 21 %, transform and split
-// 18 %, epilogue 11 %, patch reads 9 %, U loads 7 %) took its share off the time.  The kernels of
-// 4-plane boxes are at the register limit of 256: those with half the sums apart spill one (8 bytes a
-// lane), and all of them 56 to 61 scalar registers to vector lanes.
+// Bound by power and issue together: the matrix cores are 32 % busy in 32 + 32 -> 32 on 128^3 x 8
+// and 35 % in 128 -> 128 on 32^3 x 8 (23 % in the 32-channel layers of a network, two chunks a
+// box), a wave issues VALU work in 24 to 27 % of its cycles and waits in 27 to 30 %.  With plain
+// sums, leaving out any one part of 128 -> 128 (products 38 %, halo DMA 21 %, transform and split
+// 18 %, epilogue 11 %, patch reads 9 %, U loads 7 %) took its share off the time, and the clock
+// rose from 1.9 to 2.4 GHz without the products.  The kernels of 4-plane boxes are at the register
+// limit of 256: those with half the sums apart spill one (8 bytes a lane), and all of them 56 to 61
+// scalar registers to vector lanes.
 // Measured, three-axis form / plain sums / now, us and relative error against float64:
-//   32 + 32 -> 32 on 128^3 x 8       4400 / 3650 / 3830   2.62 / 2.79 / 2.52e-7  (485 TFLOP/s of
+//   32 + 32 -> 32 on 128^3 x 8       4300 / 3615 / 3730   2.62 / 2.79 / 2.52e-7  (498 TFLOP/s of
 //                                                          the direct convolution's work)
-//   128 -> 128 on 32^3 x 8            492 /  407 /  424   3.06 / 3.54 / 2.61e-7  (547)
-//   64 -> 64 on 37 x 61 x 43 x 4      257 /  222 /  229   2.61 / 2.78 / 2.52e-7  (375)
-//   256 + 256 -> 256 on 16^3 x 8      427 /  365 /  385   5.18 / 6.65 / 4.44e-7
-//   320 -> 320 on 5 x 6 x 7          65.3 / 60.0 / 61.3   4.19 / 5.20 / 3.56e-7 (on 12 x 13 x 11)
-//   32 -> 192 on 6 x 9 x 8 x 8       12.8 / 13.3 / 12.5   2.40 / 2.24 / 2.24e-7
+//   128 -> 128 on 32^3 x 8            464 /  402 /  411   3.06 / 3.54 / 2.61e-7  (564)
+//   64 -> 64 on 37 x 61 x 43 x 4      245 /  219 /  219   2.61 / 2.78 / 2.52e-7  (392)
+//   256 + 256 -> 256 on 16^3 x 8      415 /  366 /  382   5.18 / 6.65 / 4.44e-7
+//   320 -> 320 on 5 x 6 x 7          65.4 / 60.2 / 61.6   4.19 / 5.20 / 3.56e-7 (on 12 x 13 x 11)
+//   32 -> 192 on 6 x 9 x 8 x 8       12.7 / 13.4 / 12.6   2.40 / 2.24 / 2.24e-7
 #include <cmath>
 #include <string>
 #include <type_traits>
@@ -503,7 +505,8 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
     h8 vh[2][2], vl[2][2];  // V of this plane and the last, split: [plane & 1][position]
     auto plane = [&](auto zc) __attribute__((always_inline)) {
       constexpr int Z = decltype(zc)::value, kAt = Z * G::plane * 16, now = Z & 1;
-      if constexpr (CH > 0 && ZB == 4) {
+      constexpr bool chain = Z >= 1 && Z - 1 < CH;
+      if constexpr (chain && ZB == 4) {
         // (two columns, then one: the last plane's V is held too, and the registers are full)
         float vq[8];
         {
@@ -546,7 +549,6 @@ __global__ __launch_bounds__(kWThreads, 1) void wino_yx_kernel(WinoArgs a) {
         return mfma32(which == 0 ? vl[v][p] : vh[v][p],
                       *reinterpret_cast<const h8*>(&ub[p][kz][which == 1 ? 1 : 0]), c);
       };
-      constexpr bool chain = Z >= 1 && Z - 1 < CH;
       if constexpr (chain) {
         if constexpr (ZB == 2) {
           f16v t[2]{};
