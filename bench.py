@@ -358,6 +358,7 @@ def _short_kernel(name: str) -> str:
     import re
 
     name = name.replace("void ", "").replace("nnx::(anonymous namespace)::", "")
+    name = re.sub(r"\(WinoShape\)(\d)", lambda m: ("wide", "tall", "cube")[int(m.group(1))], name)
     return re.split(r"\((?!anon)", name)[0].strip()
 
 
@@ -443,9 +444,9 @@ def summarize_profiles(directory: str) -> None:
     gib_kib = 1024.0 * 1024.0
     fetch_factor = gib_kib / neg["FETCH_SIZE"]
     write_factor = gib_kib / neg["WRITE_SIZE"]
-    agg = defaultdict(lambda: [0, 0.0, 0.0])
+    agg = defaultdict(lambda: [0, 0.0, 0.0])  # by class, as the bench reports it
     for (_, short), v in per.items():
-        a = agg[short]
+        a = agg[kernel_class_of(short) or short]
         a[0] += 1
         a[1] += v.get("FETCH_SIZE", 0.0) * fetch_factor * 1024
         a[2] += v.get("WRITE_SIZE", 0.0) * write_factor * 1024
@@ -469,10 +470,9 @@ def summarize_profiles(directory: str) -> None:
         "| kernel | launches | fetch bytes/launch | write bytes/launch | traffic bytes/launch |",
         "|---|---:|---:|---:|---:|",
     ]
-    for short, (n, f, w) in sorted(agg.items(), key=lambda kv: -(kv[1][1] + kv[1][2])):
+    for cls, (n, f, w) in sorted(agg.items(), key=lambda kv: -(kv[1][1] + kv[1][2])):
         if n == 0 or (f + w) / n < 1e6:
             continue
-        cls = kernel_class_of(short) or short
         lines.append(f"| `{cls}` | {n} | {f/n:.4g} | {w/n:.4g} | {(f+w)/n:.4g} |")
     TRAFFIC_FILE.write_text("\n".join(lines) + "\n")
     print(f"wrote {out / 'kernel_stats_liver.md'} and {TRAFFIC_FILE}")
@@ -532,7 +532,7 @@ def summarize_sq_counters(base: Path, target: Path) -> None:
         "| VALU active / wave cycles |",
         "|---|---:|---:|---:|---:|---:|---:|---:|---:|---:|---:|",
     ]
-    for k, n, a in rows[:8]:
+    for k, n, a in rows[:14]:
         waves = a["SQ_WAVES"]
         cyc = a["GRBM_GUI_ACTIVE"] / 8.0
         lines.append(
