@@ -53,9 +53,9 @@
 // issues the next box's first halo DMA and U loads; the epilogue exchanges through the raw
 // buffer that this DMA does not target.
 //
-// Bound by power and issue together: the matrix cores are 32 % busy in 32 + 32 -> 32 on 128^3 x 8
-// and 35 % in 128 -> 128 on 32^3 x 8 (23 % in the 32-channel layers of a network, two chunks a
-// box), a wave issues VALU work in 24 to 27 % of its cycles and waits in 27 to 30 %.  With plain
+// Bound by power and issue together: the matrix cores are 33 % busy in 32 + 32 -> 32 on 128^3 x 8
+// and 36 % in 128 -> 128 on 32^3 x 8 (23 % in the 32-channel layers of a network, two chunks a
+// box), a wave issues VALU work in 25 to 27 % of its cycles and waits in 27 to 30 %.  With plain
 // sums, leaving out any one part of 128 -> 128 (products 38 %, halo DMA 21 %, transform and split
 // 18 %, epilogue 11 %, patch reads 9 %, U loads 7 %) took its share off the time, and the clock
 // rose from 1.9 to 2.4 GHz without the products.  The kernels of 4-plane boxes are at the register

@@ -18,7 +18,7 @@ MODEL = {
     # Measured MI355X device peak (library workspace + torch allocations) for a 2x284x400x400
     # case, five folds, 8 mirror views, 32 views a forward (bench.py --workload autopet-sw);
     # larger inputs need more.
-    "peak_memory_gb": 51.4,
+    "peak_memory_gb": 51.2,
     "summary": "Tumor lesion segmentation of co-registered CT and SUV PET volumes.",
     "labels": {"1": "tumor"},
 }
