@@ -208,12 +208,12 @@ def test_conv3d_winograd_random_shapes_match_float64(lib, case):
     (29, (7, 8, 8), 48, 0, 160),     # 4 x 8 x 8 boxes of two slabs, several a workgroup
     (60, (9, 5, 7), 16, 0, 64),      # the same, one chunk, remainders on every axis
     (26, (2, 16, 8), 16, 0, 320),    # 2 x 16 x 8 boxes, several a workgroup
-    (5, (6, 9, 8), 32, 0, 192),      # the same with remainders
+    (8, (6, 9, 8), 32, 0, 192),      # the same with remainders
     # two z taps summed apart in half the output planes (four and five chunks) and in all (from six)
     (8, (18, 23, 31), 64, 0, 32), (8, (18, 23, 31), 96, 16, 32),
     (8, (18, 33, 24), 48, 32, 64), (8, (18, 33, 24), 96, 0, 64),
     (1, (3, 8, 17), 64, 0, 32), (1, (3, 8, 17), 16, 96, 32),
-    (5, (6, 9, 8), 64, 16, 192), (5, (6, 9, 8), 112, 0, 192),
+    (8, (6, 9, 8), 64, 16, 192), (8, (6, 9, 8), 112, 0, 192),
     (29, (7, 8, 8), 64, 0, 160), (29, (7, 8, 8), 96, 0, 160),
 ], ids=lambda c: f"b{c[0]}-{c[1]}-c{c[2]}+{c[3]}-o{c[4]}")
 def test_conv3d_winograd_box_shapes_match_float64(lib, case):
