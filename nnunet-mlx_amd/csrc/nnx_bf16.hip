@@ -414,13 +414,20 @@ int conv_bf16_direct_stats_tiles(const ConvGeom& g) {
 // With one or two chunks and less than a box a CU, the first halo's latency is most of a box, and
 // the weight-staged kernel's smaller tiles are ahead (32 -> 192 on 6 x 9 x 8 x 8: 16.6 against
 // 18.1 us); from there on this kernel is (20.1 us both on 32 -> 96, 12 x 30 x 40 x 2; 67 against
-// 52 us on 128 -> 128, 32^3).
+// 52 us on 128 -> 128, 32^3).  A full round of it, a box of 4 x 8 x 16 voxels and 64 channels a CU,
+// takes about 2/3 of that kernel's, three a CU of 256 voxels, fitted, and 32 channels; narrow
+// volumes, whose boxes here are mostly padding, need more rounds than that wins (us, here against
+// there: 128 -> 128 on 70 x 2 x 70 x 4, three rounds against one, 136 and 75; 76 x 32 x 8 x 2, two
+// against one, 97 and 71; 256 -> 320 on 16 x 32 x 20 x 2, two and two, 186 and 239; 128 -> 128 on
+// 70 x 9 x 70 x 2, three and three, 151 and 201).
 bool conv_bf16_direct_supported(const ConvGeom& g, int c1, int c2, int cout) {
   if (!conv_bf16_direct_packed(g.k, c1, c2, cout) || g.s[0] != 1 || g.s[1] != 1 || g.s[2] != 1)
     return false;
   const int64_t boxes = (int64_t)g.batch * conv_bf16_direct_stats_tiles(g) *
                         ceil_div(cout / 32, cout == 32 ? 1 : 2);
-  return c1 + c2 > 2 * kBChunk || boxes >= compute_units();
+  if (c1 + c2 <= 2 * kBChunk && boxes < compute_units()) return false;
+  const int64_t cus = compute_units();
+  return 2 * ceil_div(boxes, cus) <= 3 * ceil_div(conv_x3_boxes(g) * (cout / 32), 3 * cus);
 }
 
 void conv_bf16_direct_pack(const float* d_w, int cout, int c1, int c2, float scale, void* d_packed,

@@ -2598,6 +2598,15 @@ X3Plan plan_x3(const ConvGeom& g, int cout) {
 
 }  // namespace
 
+int64_t conv_x3_boxes(const ConvGeom& g) {
+  const bool unit = g.s[0] == 1 && g.s[1] == 1 && g.s[2] == 1;
+  const int64_t wbytes =
+      (int64_t)x3s_lds_bytes(0, conv_x3_groups(g.k), kX3S.NB * kX3S.WN);
+  const Box box = unit ? choose_box(kX3S, g, false, (kX3sLdsBytes - wbytes) / 32)
+                       : choose_box(kX3F, g, false, kX3MaxHalo);
+  return (int64_t)g.batch * box.tiles;
+}
+
 bool conv_x3_supported(const int* ksize, const int* stride, int cout) {
   // the halo box depends on kernel and stride only; probe with a large volume
   const int big[3] = {256, 256, 256};
@@ -2612,7 +2621,7 @@ bool conv_x3_supported(const int* ksize, const int* stride, int cout) {
 int conv_x3_stats_tiles(const ConvGeom& g, int cout, int c1, int c2, int arith) {
   if (arith == kBf16 && conv_bf16_direct_supported(g, c1, c2, cout))
     return conv_bf16_direct_stats_tiles(g);
-  if (conv_strided_supported(g, c1, c2, cout)) return conv_strided_stats_tiles(g);
+  if (conv_strided_supported(g, c1, c2, cout, arith)) return conv_strided_stats_tiles(g);
   const Box box = plan_x3(g, cout).box;
   return (int)(ceil_div(g.out[0], box.z) * ceil_div(g.out[1], box.y) * ceil_div(g.out[2], box.x));
 }
@@ -2631,7 +2640,7 @@ int conv_x3_stats_room(const ConvGeom& g, int cout, int c1, int c2, int arith) {
 // the idle CUs (two workgroups a CU), at least four (8 channels each) a workgroup.
 int conv_x3_splits(const ConvGeom& g, int c1, int c2, int cout, int arith) {
   if (arith == kBf16 && conv_bf16_direct_supported(g, c1, c2, cout)) return 1;
-  if (conv_strided_supported(g, c1, c2, cout)) return conv_strided_splits(g, c1, c2, cout);
+  if (conv_strided_supported(g, c1, c2, cout, arith)) return conv_strided_splits(g, c1, c2, cout);
   const X3Plan plan = plan_x3(g, cout);
   if (plan.staged) return 1;
   const int64_t nwg = (int64_t)g.batch * plan.box.tiles * ceil_div(cout, plan.v.n());
@@ -2661,7 +2670,7 @@ void conv3d_x3(const float* x1, int c1, const float* x2, int c2, const void* pac
     conv3d_bf16_direct(x1, c1, x2, c2, packed, scale, bias, y, g, cout, st, stats, n1, n2);
     return;
   }
-  if (ends % 16 == 0 && conv_strided_supported(g, c1, c2, cout)) {
+  if (ends % 16 == 0 && conv_strided_supported(g, c1, c2, cout, arith)) {
     conv3d_strided(x1, c1, x2, c2, packed, conv_packed_nblk(cout), scale, bias, y, g, cout, st, stats,
                    n1, n2, arith, splits);
     return;

@@ -149,6 +149,9 @@ void conv3d_x3(const float* x1, int c1, const float* x2, int c2, const void* pac
                hipStream_t st, float4* stats = nullptr, const PendingNorm& n1 = {},
                const PendingNorm& n2 = {}, int arith = kArithSplit3, int splits = 1);
 int conv_x3_stats_tiles(const ConvGeom& g, int cout, int c1, int c2, int arith);
+// Boxes of the batch that its implicit GEMM takes, shaped to the volume: 256 voxels where the stride
+// is 1, 64 elsewhere (what the fixed boxes of its other routes are weighed against).
+int64_t conv_x3_boxes(const ConvGeom& g);
 // *_stats_room: partials per item that suffice for g and for every smaller batch or volume, whose
 // kernels and boxes may differ.
 int conv_x3_stats_room(const ConvGeom& g, int cout, int c1, int c2, int arith);
@@ -171,7 +174,7 @@ void conv3d_bf16_direct(const float* x1, int c1, const float* x2, int c2, const 
 
 // Strided 3x3x3 convolutions with 16-channel input blocks and C_out % 32 == 0 (nnx_strided.hip), a
 // route of conv3d_x3 on its packed words (nblk16 = their 16-column blocks).
-bool conv_strided_supported(const ConvGeom& g, int c1, int c2, int cout);
+bool conv_strided_supported(const ConvGeom& g, int c1, int c2, int cout, int arith);
 int conv_strided_stats_tiles(const ConvGeom& g);
 bool conv_strided_layer(const ConvGeom& g, int c1, int c2, int cout);  // supported at some size
 int conv_strided_splits(const ConvGeom& g, int c1, int c2, int cout);

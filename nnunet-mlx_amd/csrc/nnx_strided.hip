@@ -439,11 +439,23 @@ int conv_strided_stats_tiles(const ConvGeom& g) {
 // 64 -> 128 on 64^3 x 8, 8192, 491 against 486; with stride 1 in z 64 -> 128 on
 // 37 x 61 x 43 x 2, 1824, 103 against 100; below: 64 -> 128 on 64^3, 1024, 64 against 73;
 // 256 -> 320 on 16^3 x 8, 320, 88 against 106; 320 -> 320 on 8^3 58 against 88).
-bool conv_strided_supported(const ConvGeom& g, int c1, int c2, int cout) {
-  if (cout > 64 && (int64_t)g.batch * conv_strided_stats_tiles(g) * ceil_div(cout, 64) >=
-                       6 * (int64_t)compute_units())
-    return false;
-  return conv_strided_layer(g, c1, c2, cout);
+// So do outputs that leave boxes of 2 x 4 x 8 voxels half empty, where the GEMM's fitted ones come
+// to three a CU for four here, or in bf16, where this kernel's boxes are the cheaper, to three for
+// five (64 -> 128 to 82 x 32 x 4 x 2, 1312 boxes for 672, 79 against 48, in bf16 48 against 36;
+// 128 -> 320 to 30 x 16 x 4 x 2, 600 for 320, 65 against 53, but in bf16 it is 38 against 34 there
+// and 28 against 32 on 64 -> 64 to 36 x 32 x 10 x 2, 576 for 432).  While the resident workgroups
+// take all boxes in one round this kernel is ahead at any fill (128 -> 128 to 20 x 32 x 4 x 2, 320
+// for 160, 45 against 54; in bf16 64 -> 320 to 20 x 16 x 4 x 2, 400 for 200, 17 against 19), but
+// for split layers of one to four chunks only up to a box a CU (that layer, 27 against 23).
+bool conv_strided_supported(const ConvGeom& g, int c1, int c2, int cout, int arith) {
+  if (!conv_strided_layer(g, c1, c2, cout)) return false;
+  const int64_t cus = compute_units(), groups = ceil_div(cout, 64);
+  const int64_t boxes = (int64_t)g.batch * conv_strided_stats_tiles(g) * groups;
+  if (cout > 64 && boxes >= 6 * cus) return false;
+  const int64_t resident = arith == kArithSplit3 && c1 + c2 <= 64 ? cus : 2 * cus;
+  return boxes <= resident ||
+         3 * ceil_div(boxes, cus) <
+             (arith == kArithSplit3 ? 4 : 5) * ceil_div(conv_x3_boxes(g) * groups, cus);
 }
 
 bool conv_strided_layer(const ConvGeom& g, int c1, int c2, int cout) {

@@ -600,6 +600,11 @@ STRIDED_CASES = [
     (2, (5, 10, 15), 48, 0, 32, (3, 3, 3), (1, 2, 2)),    # z kept, one column block
     (1, (1, 1, 1), 16, 16, 160, (3, 3, 3), (2, 2, 2)),
     (12, (17, 30, 62), 16, 0, 64, (3, 3, 3), (1, 2, 2)),  # boxes in turn across items
+    # narrow outputs: boxes half empty, at most one a CU and more (the implicit GEMM's fitted boxes)
+    (4, (15, 64, 7), 16, 0, 64, (3, 3, 3), (1, 2, 2)),
+    (5, (15, 64, 7), 16, 0, 64, (3, 3, 3), (1, 2, 2)),
+    (5, (31, 64, 7), 64, 16, 96, (3, 3, 3), (2, 2, 2)),   # three a CU for two
+    (9, (31, 64, 7), 16, 0, 64, (3, 3, 3), (1, 2, 2)),    # five a CU for three
 ]
 
 
@@ -616,6 +621,10 @@ BF16_DIRECT_CASES = [
     (3, (9, 13, 30), 64, 0, 32, (3, 3, 3), (1, 1, 1)),   # one column block, two planes a wave
     (1, (1, 1, 1), 64, 16, 160, (3, 3, 3), (1, 1, 1)),
     (16, (17, 20, 33), 16, 0, 64, (3, 3, 3), (1, 1, 1)),  # one chunk, boxes in turn across items
+    # narrow volumes: one round of boxes, and two for one of the weight-staged kernel's
+    (8, (16, 62, 4), 48, 0, 64, (3, 3, 3), (1, 1, 1)),
+    (9, (16, 62, 4), 48, 0, 64, (3, 3, 3), (1, 1, 1)),
+    (9, (62, 2, 33), 32, 16, 64, (3, 3, 3), (1, 1, 1)),
 ]
 
 
